@@ -9,7 +9,9 @@
 //     A  = X X^T              NT, P = X,  Q = X   (symmetric: upper tiles only)
 //     B' = c A A + b A + a I  NT, P = A,  Q = A   (A symmetric, so A A = A A^T)
 //     X' = B' X               NN, P = B', Q = X   (= B X + a X)
-// Workspace matrices are zero-padded to multiples of 256.  The padding of X
+// Workspace matrices are zero-padded to multiples of the tile (256 here; calls
+// whose products would not fill the chip with 256 x 256 tiles take 64- or
+// 128-wide ones, tile_gemm.hip, by ns_tile_choice).  The padding of X
 // and A stays zero through every product (B' carries a on its padded
 // diagonal, which meets only zero rows of X), so only the final store is
 // bounds-checked.
@@ -37,28 +39,14 @@
 
 #include "common.hpp"
 #include "vecio.hpp"
+#include "gemm.hpp"
+#include "tile_gemm.hpp"
 #include "../../include/muon_sr_amd.h"
 
 namespace msr {
 
-typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
-typedef float f32x16_t __attribute__((ext_vector_type(16)));
-typedef short s16x4_t __attribute__((ext_vector_type(4)));
-typedef __attribute__((address_space(3))) s16x4_t lds_s16x4_t;
-
 constexpr int BM = 256, BN = 256, BK = 64;
 constexpr int GEMM_THREADS = 512;
-
-// Muon apply fused into the store of the last Newton-Schulz product
-// (msr_muon_ns_apply): matrix b of a launch updates params p[b] with seed[b].
-constexpr int APPLY_MAX = 128;   // matrices per launch (kernel-argument table)
-struct ApplyTab {
-    uint16_t *p[APPLY_MAX];
-    uint32_t seed[APPLY_MAX];
-    const uint16_t *inject;      // uint16 [count][numel] of this launch (NOISE_INJECT), or null
-    int64_t numel;
-    float lr, decay, scale;      // decay = 1 - lr * wd
-};
 
 struct GemmArgs {
     const uint16_t *P; int64_t ldp, sP;
@@ -91,51 +79,6 @@ struct GemmArgs {
     int *tile_ctr;          // dynamic tile order (see the kernel), or null: [0, 8) per XCD, [8] work-groups done
 };
 
-// p[off + j] <- SR(p*(1 - lr*wd) - lr*(f32(u_j)*scale)) for the j < valid bf16 values u
-// (packed in u[4]) of one 8-element chunk: the arithmetic and noise of
-// muon_apply_kernel (muon_sr/triton_muon_sr.py:53-80); off is the element index in p.
-// vec: the chunk is 16-byte aligned and off a multiple of 8.
-// The parameter chunk of apply_chunk (loaded ahead so that the loads of a thread's
-// chunks overlap).
-__device__ __forceinline__ u32x4_t apply_load(const uint16_t *P, int64_t off, int valid, bool vec) {
-    if (vec && valid == 8) return ld_nt4(P + off);
-    uint32_t wp[4] = {0u, 0u, 0u, 0u};
-#pragma unroll
-    for (int j = 0; j < 8; ++j)
-        if (j < valid) wp[j >> 1] |= (uint32_t)P[off + j] << (16 * (j & 1));
-    return u32x4_t{wp[0], wp[1], wp[2], wp[3]};
-}
-
-template <int MODE>
-__device__ __forceinline__ void apply_chunk(const ApplyTab &ap, uint16_t *P, const Noise &ns, int64_t off, int valid,
-                                            bool vec, const uint32_t u[4], u32x4_t pw) {
-    const uint32_t wp[4] = {pw.x, pw.y, pw.z, pw.w};
-    uint32_t r[8];
-    if (vec && valid == 8) {
-        noise8<MODE>(ns, off, 8, r);
-    } else {
-#pragma unroll
-        for (int j = 0; j < 8; ++j) r[j] = j < valid ? noise1<MODE>(ns, off + j) : 0u;
-    }
-    uint32_t op[8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-        const float uf = (j & 1) ? bf16_hi(u[j >> 1]) : bf16_lo(u[j >> 1]);
-        const float pf = (j & 1) ? bf16_hi(wp[j >> 1]) : bf16_lo(wp[j >> 1]);
-        const float t1 = uf * ap.scale;                                   // :70
-        float pj = pf * ap.decay;                                         // :72
-        pj = pj - ap.lr * t1;                                             // :73
-        op[j] = sr_bf16(pj, r[j]);                                        // :75-80
-    }
-    if (vec && valid == 8) {
-        st_nt4(P + off, u32x4_t{pack2(op[0], op[1]), pack2(op[2], op[3]), pack2(op[4], op[5]), pack2(op[6], op[7])});
-    } else {
-#pragma unroll
-        for (int j = 0; j < 8; ++j)
-            if (j < valid) P[off + j] = (uint16_t)op[j];
-    }
-}
-
 // Work-group -> (matrix, tile).  Consecutive work-group ids are dispatched
 // round-robin over the 8 XCDs (each with its own L2), so tiles that share
 // operand row blocks should run on one XCD at the same time:
@@ -153,7 +96,6 @@ __device__ __forceinline__ void apply_chunk(const ApplyTab &ap, uint16_t *P, con
 // GROUP_M tile-rows, column by column, taking the band's rows ti <= tj of each
 // column.  Either way a run of consecutive tiles covers a compact block of
 // tile-rows and tile-columns.
-constexpr int NXCD = 8;
 constexpr int GROUP_M = 4;
 constexpr int PER_XCD_TILES = 64;
 constexpr int PERSIST_MAX = 32;   // tiles per persistent work-group, at most
@@ -213,18 +155,6 @@ __device__ __forceinline__ void locate_tile(const GemmArgs &a, int v, int64_t &b
     n0 = tj * BN;
 }
 
-// Wait until at most N vector memory operations of this wave are outstanding
-// (s_waitcnt: vmcnt in bits 3:0 and 15:14; expcnt and lgkmcnt at their maxima).
-// Vector memory operations complete in issue order, so every operation issued
-// before the last N has completed.
-template <int N>
-__device__ __forceinline__ void wait_vm() {
-    static_assert(N >= 0 && N < 64, "vmcnt is 6 bits");
-    __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | (15 << 8) | ((N >> 4) << 14));
-}
-
-typedef __attribute__((address_space(3))) void lds_void_t;
-
 // LDS: four variables of 32 KiB, one per slab: P stage 0, P stage 1, Q stage
 // 0, Q stage 1.  Separate variables tell the compiler that
 // the fragment reads of one stage do not alias the direct-to-LDS loads into
@@ -259,22 +189,6 @@ static_assert(4 * EST_BYTES <= SLAB_BYTES, "epilogue staging fits the stage-1 va
 //   GM_KK      P, Q K-major everywhere (the weight gradient dW = dY^T X of
 //              row-major activations)
 enum : int { GM_RR = 0, GM_RK = 1, GM_TRI_P = 2, GM_TRI_PQ = 3, GM_KK = 4 };
-
-// Epilogues of the Newton-Schulz products.  The iteration keeps A, B' and X
-// in bf16 between products; the diagonals of A and B' are the largest
-// entries of those matrices (B' carries a = 3.4445 on it), so their bf16
-// rounding is the largest rounding error of the iteration.  These epilogues
-// carry the rounding residual of every diagonal element in fp32 to the next
-// product:
-//   EPI_A  A = alpha X X^T:  rho[m] = A_mm - bf16(A_mm)                 (resid)
-//   EPI_B  B' = alpha (A A) + beta A + diag I with the diagonal corrected
-//          for rho to first order, B'_mm += rho[m] (beta + 2 alpha A_mm)
-//          (d/dA_mm of beta A_mm + alpha (A A)_mm with A_mm dominant):
-//          r[m] = B'_mm - bf16(B'_mm)                                   (resid)
-//   EPI_X  X' = alpha (B' X + bf16(r[m]) X), the second term as MFMAs of the diagonal
-//          block (see mmdiag)
-// EPI_NONE is the plain alpha P Q^T + beta C + diag I of the diagnostic GEMMs.
-enum : int { EPI_NONE = 0, EPI_A = 1, EPI_B = 2, EPI_X = 3 };
 
 // SRACC >= 0: D is a bf16 accumulator and the store adds to it with stochastic
 // rounding (noise mode SRACC), as msr_sr_accum does with the RNE bf16 product.
@@ -1282,9 +1196,10 @@ static inline int64_t round_up(int64_t x, int64_t m) { return (x + m - 1) / m * 
 
 struct NSLayout {
     int64_t m, n, mp, np;
+    int tile;         // 256 (ns_gemm.hip), or 64 / 128 (tile_gemm.hip); mp and np are multiples of it
     bool transposed;
     size_t off_x[2], off_a, off_b, off_part, off_alpha, off_rho, off_r, off_tpart, off_rexp, off_ctr, total;
-    int64_t ntiles;   // 64 x 64 tiles of the padded update (prologue sums of squares)
+    int64_t ntiles;   // 64 x 64 tiles of the update padded to 256 (prologue sums of squares)
 };
 
 static NSLayout ns_layout(int64_t batch, int64_t rows, int64_t cols) {
@@ -1292,10 +1207,14 @@ static NSLayout ns_layout(int64_t batch, int64_t rows, int64_t cols) {
     L.transposed = rows > cols;
     L.m = L.transposed ? cols : rows;
     L.n = L.transposed ? rows : cols;
-    L.mp = round_up(L.m, 256);
-    L.np = round_up(L.n, 256);
-    const size_t xs = (size_t)batch * L.mp * L.np * 2;
-    const size_t as = (size_t)batch * L.mp * L.mp * 2;
+    L.tile = ns_tile_choice(batch, L.m, L.n);
+    L.mp = round_up(L.m, L.tile);
+    L.np = round_up(L.n, L.tile);
+    // sized for 256-wide tiles whatever the tile, so that a workspace for a batch also serves
+    // every smaller one
+    const int64_t m256 = round_up(L.m, 256), n256 = round_up(L.n, 256);
+    const size_t xs = (size_t)batch * m256 * n256 * 2;
+    const size_t as = (size_t)batch * m256 * m256 * 2;
     size_t o = 0;
     auto take = [&](size_t s) { size_t r = o; o += (s + 255) & ~(size_t)255; return r; };
     L.off_x[0] = take(xs);
@@ -1304,9 +1223,9 @@ static NSLayout ns_layout(int64_t batch, int64_t rows, int64_t cols) {
     L.off_b = take(as);
     L.off_part = take((size_t)batch * NPART * 4);
     L.off_alpha = take((size_t)batch * 2 * 4);     // alphas of the first A and X' products
-    L.off_rho = take((size_t)batch * L.mp * 4);    // residuals of A's diagonal
-    L.off_r = take((size_t)batch * L.mp * 4);      // residuals of B''s diagonal
-    L.ntiles = (L.mp / 64) * (L.np / 64);
+    L.off_rho = take((size_t)batch * m256 * 4);    // residuals of A's diagonal
+    L.off_r = take((size_t)batch * m256 * 4);      // residuals of B''s diagonal
+    L.ntiles = (m256 / 64) * (n256 / 64);
     L.off_tpart = take((size_t)batch * L.ntiles * 4);   // tile sums of squares of the update
     L.off_rexp = take((size_t)batch * 4);               // prologue scale exponents
     L.off_ctr = take(16 * 4);                           // the GEMMs' dynamic tile counters
@@ -1569,6 +1488,18 @@ int msr_linear_wgrad_sr_accum(uint16_t *acc, const uint16_t *x, int64_t ldx, con
     a.zero_init = zero_init != 0;
     a.ns.key = seed_key(seed, 0);
     a.ns.inject = inject;
+    const int T = wgrad_tile_choice(a.M, a.N, a.K);
+    if (T != 256 && std::max(xb, yb) < (size_t(1) << 31)) {
+        TileArgs t = {};
+        t.P = dy; t.ldp = ldy;
+        t.Q = x; t.ldq = ldx;
+        t.D = acc; t.ldd = in_features;
+        t.M = a.M; t.N = a.N; t.K = a.K;
+        t.alpha = 1.0f;
+        t.zero_init = a.zero_init;
+        t.ns = a.ns;
+        return launch_tile_gemm(T, TILE_W, TILE_D, noise_mode, t, 1, nullptr, (hipStream_t)stream);
+    }
     return launch_gemm(a, 1, (hipStream_t)stream);
 }
 
@@ -1640,8 +1571,10 @@ static int ns_prologue_part(const NSPart &pt, uint16_t *X0, float *tpart, const 
         a.T = transposed ? x0 : nullptr; a.ldT = Rp; a.sT = xs;
         a.Rp = Rp; a.Cp = Cp;
         a.tpart = tpart + (pt.b0 + b0) * L.ntiles;
-        a.ntx = Cp / 64; a.ntiles = L.ntiles;
-        const dim3 grid((unsigned)(Cp / 64), (unsigned)(Rp / 64), (unsigned)nb);
+        // the tile sums are indexed over the extents padded to 256 whatever the products'
+        // tile, so the norm (and every result) does not depend on the batch
+        a.ntx = round_up(cols, 256) / 64; a.ntiles = L.ntiles;
+        const dim3 grid((unsigned)a.ntx, (unsigned)(round_up(rows, 256) / 64), (unsigned)nb);
         if (!pp) {
             a.in = pt.in + b0 * numel;
             if (vec) hipLaunchKernelGGL((ns_prologue_kernel<SRC_COPY, NOISE_TRITON, false, false, true>), grid, dim3(256), 0, s, a);
@@ -1682,6 +1615,83 @@ static int ns_prologue_finish(int64_t batch, uint16_t *X0, float *tpart, float *
     return check_launch("ns_rescale_kernel");
 }
 
+// The iterations and the last product of ns_run_parts in 64- or 128-wide tiles
+// (tile_gemm.hip): A and B' are stored whole.
+static int ns_tile_products(const NSPart *parts, int n_parts, int64_t batch, int32_t steps, float a_coef, float b_coef,
+                            float c_coef, uint16_t *const X[2], uint16_t *A, uint16_t *B, const float *alphas,
+                            float *rho, float *rr, const NSLayout &L, hipStream_t s) {
+    const int64_t xs = L.mp * L.np, as = L.mp * L.mp;
+    const int mp = (int)L.mp, np = (int)L.np;
+    int rc = MSR_OK, cur = 0;
+    for (int it = 0; it < steps; ++it) {
+        TileArgs g = {};
+        g.sv = mp;
+        g.P = g.Q = X[cur]; g.ldp = g.ldq = np; g.sP = g.sQ = xs;
+        g.D = A; g.ldd = mp; g.sD = as;
+        g.M = g.N = mp; g.K = np;
+        g.alpha = 1.0f;
+        g.alpha_b = it == 0 ? alphas : nullptr;   // s0^2 x0 x0^T
+        g.resid = rho;
+        if ((rc = launch_tile_gemm(L.tile, TILE_A, TILE_WS, 0, g, batch, nullptr, s))) return rc;
+        g.P = g.Q = g.C = A; g.ldp = g.ldq = g.ldc = mp; g.sP = g.sQ = g.sC = as;
+        g.D = B;
+        g.K = mp;
+        g.alpha = c_coef; g.beta = b_coef; g.diag = a_coef;
+        g.alpha_b = nullptr;
+        g.rvec = rho; g.resid = rr;
+        if ((rc = launch_tile_gemm(L.tile, TILE_B, TILE_WS, 0, g, batch, nullptr, s))) return rc;
+        g.P = B;
+        g.Q = X[cur]; g.ldq = np; g.sQ = xs;
+        g.C = nullptr;
+        g.N = np;
+        g.alpha = 1.0f; g.beta = 0.0f; g.diag = 0.0f;
+        g.alpha_b = it == 0 ? alphas + batch : nullptr;   // s0 (B' x0 + r x0)
+        g.rvec = rr; g.resid = nullptr;
+        if (it != steps - 1) {
+            g.D = X[cur ^ 1]; g.ldd = np; g.sD = xs;
+            if ((rc = launch_tile_gemm(L.tile, TILE_X, TILE_WS, 0, g, batch, nullptr, s))) return rc;
+            cur ^= 1;
+            continue;
+        }
+        for (int i = 0; i < n_parts; ++i) {   // the last product, per part: its output layout and update
+            const NSPart &pt = parts[i];
+            const int64_t numel = pt.rows * pt.cols;
+            const bool wide = pt.rows <= pt.cols;
+            const NSApply *ap = pt.ap;
+            const int64_t per = ap ? APPLY_MAX : std::max<int64_t>(pt.batch, 1);
+            for (int64_t b0 = 0; b0 < pt.batch; b0 += per) {
+                const int64_t nb = std::min(per, pt.batch - b0), at = pt.b0 + b0;
+                TileArgs ga = g;
+                ga.P += at * as;
+                ga.Q += at * xs;
+                ga.alpha_b = g.alpha_b ? g.alpha_b + at : nullptr;
+                ga.rvec += at * mp;
+                ga.Mv = (int)L.m; ga.Nv = (int)L.n;
+                bool vec = pt.cols % 8 == 0 && (ap || (aligned(pt.out, 16) && numel % 8 == 0));
+                ApplyTab tab;
+                if (ap) {
+                    for (int64_t j = 0; j < nb; ++j) {
+                        tab.p[j] = ap->params[b0 + j];
+                        tab.seed[j] = ap->seeds[b0 + j];
+                        vec = vec && aligned(tab.p[j], 16);
+                    }
+                    tab.inject = ap->inject ? ap->inject + b0 * numel : nullptr;
+                    tab.numel = numel;
+                    tab.lr = ap->lr;
+                    tab.decay = 1.0f - ap->lr * ap->weight_decay;          // :72
+                    tab.scale = ap->scale;
+                }
+                if (wide) { ga.D = ap ? nullptr : pt.out + b0 * numel; ga.ldd = pt.cols; ga.sD = numel; }
+                else { ga.D = nullptr; ga.DT = ap ? nullptr : pt.out + b0 * numel; ga.lddt = pt.cols; ga.sDT = numel; }
+                ga.d_vec = ga.dt_vec = vec;
+                const int out = ap ? (wide ? TILE_PD : TILE_PT) : (wide ? TILE_D : TILE_DT);
+                if ((rc = launch_tile_gemm(L.tile, TILE_X, out, ap ? ap->noise_mode : 0, ga, nb, ap ? &tab : nullptr, s))) return rc;
+            }
+        }
+    }
+    return MSR_OK;
+}
+
 // Newton-Schulz (steps >= 1) of the `batch` matrices of `parts` (which cover
 // [0, batch) in order): one prologue per part, the iterations over the whole
 // batch, and the last product per part.  Arguments are validated by the callers.
@@ -1702,6 +1712,7 @@ static int ns_run_parts(const NSPart *parts, int n_parts, int64_t batch, int32_t
         if ((rc = ns_prologue_part(parts[i], X[0], tpart, L, s))) return rc;
     if ((rc = ns_prologue_finish(batch, X[0], tpart, alphas, (int *)(ws + L.off_rexp), tile_ctr, L, s))) return rc;
 
+    if (L.tile != 256) return ns_tile_products(parts, n_parts, batch, steps, a_coef, b_coef, c_coef, X, A, B, alphas, rho, rr, L, s);
     const int mp = (int)L.mp, np = (int)L.np;
     int cur = 0;
     for (int it = 0; it < steps; ++it) {
