@@ -104,6 +104,26 @@ int msr_adamw_bf16_step(uint16_t *p, const uint16_t *g, uint16_t *ema, uint16_t 
                         float bias_correction, float bias_correction_sqrt, uint32_t seed,
                         int32_t noise_mode, const uint16_t *inject, msr_stream_t stream);
 
+/* The same for many tensors of one parameter group in one launch (up to 56 per launch, split
+ * internally); equal, bit for bit, to one call per item in order.  form MSR_ADAMW: each item as
+ * msr_adamw_bf16_step (m, v: ema, ema_sq; bc1, bc2: bias_correction, bias_correction_sqrt).
+ * form MSR_ADAMW_8BIT16: each item as msr_adamw8bit_step with quantized = 0 (m, v: the bf16
+ * states; bc1, bc2 as there).  items: HOST array.  noise_mode: MSR_NOISE_TRITON or
+ * MSR_NOISE_PHILOX8. */
+typedef struct msr_adamw_item {
+    uint16_t *p;
+    const uint16_t *g;
+    uint16_t *m, *v;
+    int64_t n;
+    float bc1, bc2;
+    uint32_t seed;
+    int32_t reserved;   /* 0 */
+} msr_adamw_item;
+#define MSR_ADAMW 0
+#define MSR_ADAMW_8BIT16 1
+int msr_adamw_multi(const msr_adamw_item *items, int32_t count, int32_t form, float lr, float beta1,
+                    float beta2, float eps, float weight_decay, int32_t noise_mode, msr_stream_t stream);
+
 /* ---------------------------------------------------------------------------
  * Gradient centralization of TritonAdamW, on the device.
  * Replaces the host-issued torch ops of muon_sr/triton_adamw.py:179-187

@@ -9,6 +9,7 @@ from __future__ import annotations
 import contextlib
 import ctypes
 import random
+import struct
 import threading
 
 import torch
@@ -22,25 +23,56 @@ def _seed(step: int, param_idx: int) -> int:
     return (step * 2654435761 ^ param_idx * 1234567891) & 0xFFFFFFFF
 
 
-def _adamw_step(p: torch.Tensor, g: torch.Tensor, ema: torch.Tensor, ema_sq: torch.Tensor,
-                lr: float, beta1: float, beta2: float, eps: float, weight_decay: float,
-                step: int, param_idx: int) -> None:
-    """One fused AdamW step on one tensor (muon_sr/triton_adamw.py:75-114).
+class _AdamWBatch:
+    """The bf16-moment AdamW steps of one parameter group, launched many tensors at a time
+    (msr_adamw_multi; muon_sr/triton_adamw.py:75-114 launches one kernel per tensor).  Steps run
+    in the order they were added wherever they share memory.  ``form``: _lib.ADAMW, or
+    _lib.ADAMW_8BIT16 for the bf16-moment tensors of the 8-bit optimizer.
+
+    A caller adds in a ``try`` and flushes in its ``finally``, so that an error at one parameter
+    leaves the earlier ones stepped, as one launch per parameter would."""
+
+    _PACK = struct.Struct("=QQQQqffIi").pack   # msr_adamw_item
+    MAX_KEPT_BYTES = 256 << 20   # gradient copies (made contiguous, or centred) held until their launch
+
+    def __init__(self, form, lr, beta1, beta2, eps, weight_decay):
+        self.form, self.hyper = form, (lr, beta1, beta2, eps, weight_decay)
+        self.items, self.kept, self.kept_bytes, self.stream, self.device = [], [], 0, None, None
+
+    def add(self, p, g, m, v, bc1, bc2, seed, copied=False):
+        """One tensor's step; ``copied``: nothing but the batch holds ``g``."""
+        device, stream = p.get_device(), _lib.stream_of(p)
+        if self.items and (device != self.device or stream != self.stream):
+            self.flush()
+        self.device, self.stream = device, stream
+        self.items.append(self._PACK(p.data_ptr(), g.data_ptr(), m.data_ptr(), v.data_ptr(), p.numel(), bc1, bc2, seed, 0))
+        if copied:
+            self.kept.append(g)
+            self.kept_bytes += g.numel() * g.element_size()
+            if self.kept_bytes >= self.MAX_KEPT_BYTES:
+                self.flush()
+
+    def flush(self):
+        if not self.items:
+            return
+        items, self.items = self.items, []
+        rc = _lib.lib().msr_adamw_multi(b"".join(items), len(items), self.form, *self.hyper, _lib.noise_mode(), self.stream)
+        self.kept, self.kept_bytes = [], 0
+        _lib.check(rc, "msr_adamw_multi")
+
+
+def _adamw_add(batch, p, g, ema, ema_sq, beta1, beta2, step, param_idx, copied=False):
+    """Adds the AdamW step of one tensor (muon_sr/triton_adamw.py:75-114).
 
     Bias corrections are Python doubles, passed to the kernel as fp32 (as a
     compiled Triton launch passes Python floats).
     """
-    bias_correction = 1.0 - beta1 ** step
-    bias_correction_sqrt = (1.0 - beta2 ** step) ** 0.5
     _lib.require_gpu(p, "TritonAdamW", RuntimeError)
     if not p.is_contiguous():
         raise RuntimeError("TritonAdamW requires contiguous parameters")
-    g = g.contiguous()
-    L = _lib.lib()
-    rc = L.msr_adamw_bf16_step(p.data_ptr(), g.data_ptr(), ema.data_ptr(), ema_sq.data_ptr(), p.numel(),
-                               lr, beta1, beta2, eps, weight_decay, bias_correction, bias_correction_sqrt,
-                               _seed(step, param_idx), _lib.noise_mode(), None, _lib.stream_of(p))
-    _lib.check(rc, "msr_adamw_bf16_step")
+    if not g.is_contiguous():
+        g, copied = g.contiguous(), True
+    batch.add(p, g, ema, ema_sq, 1.0 - beta1 ** step, (1.0 - beta2 ** step) ** 0.5, _seed(step, param_idx), copied)
 
 
 def centralize(grad: torch.Tensor, strength: float) -> torch.Tensor:
@@ -96,35 +128,39 @@ class TritonAdamW(Optimizer):
             eps = group["eps"]
             weight_decay = group["weight_decay"]
             centralization = group["centralization"]
-
-            for i, p in enumerate(group["params"]):
-                assert p.dtype == torch.bfloat16, "only bfloat16 is supported."
-                if p.grad is None:
-                    continue
-                grad = p.grad
-                if grad.is_sparse:
-                    raise RuntimeError("TritonAdamW does not support sparse gradients")
-
-                state = self.state[p]
-                if len(state) == 0:
-                    state["step"] = 0
-                    state["ema"] = torch.zeros_like(p.data, dtype=torch.bfloat16)
-                    state["ema_squared"] = torch.zeros_like(p.data, dtype=torch.bfloat16)
-
-                state["step"] += 1
-
-                # gradient centralization (muon_sr/triton_adamw.py:179-187): one fused
-                # device pass instead of the reference's five torch ops
-                if centralization != 0:
-                    _lib.require_gpu(p, "TritonAdamW", RuntimeError)
-                    grad = centralize(grad, centralization)
-
-                with torch.no_grad():
-                    _adamw_step(p=p.data, g=grad, ema=state["ema"], ema_sq=state["ema_squared"],
-                                lr=lr, beta1=beta1, beta2=beta2, eps=eps, weight_decay=weight_decay,
-                                step=state["step"], param_idx=group_offset + i)
+            batch = _AdamWBatch(_lib.ADAMW, lr, beta1, beta2, eps, weight_decay)
+            try:
+                self._step_group(group, group_offset, beta1, beta2, centralization, batch)
+            finally:
+                batch.flush()
 
         return loss
+
+    def _step_group(self, group, group_offset, beta1, beta2, centralization, batch):
+        for i, p in enumerate(group["params"]):
+            assert p.dtype == torch.bfloat16, "only bfloat16 is supported."
+            grad = p.grad
+            if grad is None:
+                continue
+            if grad.is_sparse:
+                raise RuntimeError("TritonAdamW does not support sparse gradients")
+
+            state = self.state[p]
+            if len(state) == 0:
+                state["step"] = 0
+                state["ema"] = torch.zeros_like(p.data, dtype=torch.bfloat16)
+                state["ema_squared"] = torch.zeros_like(p.data, dtype=torch.bfloat16)
+
+            state["step"] += 1
+
+            # gradient centralization (muon_sr/triton_adamw.py:179-187): one fused
+            # device pass instead of the reference's five torch ops
+            if centralization != 0:
+                _lib.require_gpu(p, "TritonAdamW", RuntimeError)
+                grad = centralize(grad, centralization)
+
+            _adamw_add(batch, p, grad, state["ema"], state["ema_squared"], beta1, beta2, state["step"],
+                       group_offset + i, copied=centralization != 0)
 
 
 class _AccumQueue:

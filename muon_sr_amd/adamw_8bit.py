@@ -14,6 +14,7 @@ import torch
 from torch.optim import Optimizer
 
 from . import _lib
+from .adamw import _AdamWBatch
 
 
 def create_dynamic_map(signed: bool = True) -> torch.Tensor:
@@ -83,10 +84,14 @@ def quant_table(state):
     return t.data_ptr()
 
 
-def adamw8bit_launch(p, g, state, lr, beta1, beta2, eps, weight_decay, seed):
-    """One fused 8-bit (or bf16-moment) step of one tensor with state from ``init_8bit_state``."""
+def adamw8bit_launch(p, g, state, lr, beta1, beta2, eps, weight_decay, seed, batch=None):
+    """One fused 8-bit (or bf16-moment) step of one tensor with state from ``init_8bit_state``.
+    ``batch``: the step's _AdamWBatch (form ADAMW_8BIT16), which takes the bf16-moment tensors."""
     n = state["step"]
     quant = state["optim_bits"] == 8
+    if not quant and batch is not None:
+        batch.add(p, g, state["state1"], state["state2"], 1 - beta1 ** n, 1 - beta2 ** n, seed)
+        return
     get = lambda k: state[k].data_ptr() if k in state else None  # noqa: E731
     qt = quant_table(state) if quant else None
     rc = _lib.lib().msr_adamw8bit_step(
@@ -233,28 +238,34 @@ class TritonAdamW8bit(Optimizer):
         for group in self.param_groups:
             self._validate_group(group)
             b1, b2 = group["betas"]
-            for p in group["params"]:
-                param_index = index
-                index += 1
-                if p.grad is None:
-                    continue
-                if p.dtype != torch.bfloat16 or not p.is_cuda:
-                    raise ValueError("TritonAdamW8bit requires CUDA BF16 parameters")
-                g = p.grad
-                if g.is_sparse or not p.is_contiguous() or not g.is_contiguous():
-                    raise ValueError("Parameters/gradients must be contiguous and dense")
-                if not p.numel():
-                    continue
-                state = self.state[p]
-                if not state:
-                    state.update(self._init_state(p, group))
-                expected_bits = 16 if p.numel() < group["min_8bit_size"] else group["optim_bits"]
-                if state["block_size"] != group["block_size"] or state["optim_bits"] != expected_bits:
-                    raise ValueError("Cannot change quantization configuration after state initialization")
-                state["step"] += 1
-                seed = step_seed(state["step"], param_index)
-                adamw8bit_launch(p, g, state, group["lr"], b1, b2, group["eps"], group["weight_decay"], seed)
+            batch = _AdamWBatch(_lib.ADAMW_8BIT16, group["lr"], b1, b2, group["eps"], group["weight_decay"])
+            try:
+                self._step_group(group, index, b1, b2, batch)
+            finally:
+                batch.flush()
+            index += len(group["params"])
         return loss
+
+    def _step_group(self, group, index, b1, b2, batch):
+        for param_index, p in enumerate(group["params"], index):
+            g = p.grad
+            if g is None:
+                continue
+            if p.dtype != torch.bfloat16 or not p.is_cuda:
+                raise ValueError("TritonAdamW8bit requires CUDA BF16 parameters")
+            if g.is_sparse or not p.is_contiguous() or not g.is_contiguous():
+                raise ValueError("Parameters/gradients must be contiguous and dense")
+            if not p.numel():
+                continue
+            state = self.state[p]
+            if not state:
+                state.update(self._init_state(p, group))
+            expected_bits = 16 if p.numel() < group["min_8bit_size"] else group["optim_bits"]
+            if state["block_size"] != group["block_size"] or state["optim_bits"] != expected_bits:
+                raise ValueError("Cannot change quantization configuration after state initialization")
+            state["step"] += 1
+            seed = step_seed(state["step"], param_index)
+            adamw8bit_launch(p, g, state, group["lr"], b1, b2, group["eps"], group["weight_decay"], seed, batch)
 
     def load_state_dict(self, state_dict):
         """Restore uint8 codes and fp32 scales without torch's cast to the

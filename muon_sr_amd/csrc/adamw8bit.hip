@@ -1,5 +1,5 @@
 // 8-bit blockwise AdamW for gfx950 (muon_sr/triton_adamw_8bit.py:27-99): the fused
-// quantized step, the bf16-moment step of excluded tensors, the quantizer
+// quantized step (the bf16-moment step of excluded tensors: adamw16.hip), the quantizer
 // diagnostics and the quantizer tables.
 #include <cmath>
 #include <cstdarg>
@@ -32,7 +32,7 @@ struct Adam8Args {
     int64_t n;
     int64_t qb0;   // first quantization block this launch handles (the rest of the tensor is done elsewhere)
     float lr, b1, b2, eps, wd, bc1, bc2;
-    Noise ns_p, ns_m, ns_v;
+    Noise ns_p;
 };
 
 struct Adam8Consts {
@@ -568,52 +568,6 @@ __global__ __launch_bounds__(F8_THREADS) void stream8_probe_kernel(Adam8Args a, 
     }
 }
 
-// Excluded tensors: bf16 moments with SR on both moment stores (:90-99).
-template <int MODE, bool VEC>
-__global__ __launch_bounds__(THREADS) void adamw8bit_bf16_kernel(Adam8Args a) {
-    const Adam8Consts c = adam8_consts(a);
-    uint16_t *m16 = static_cast<uint16_t *>(a.s1);
-    uint16_t *v16 = static_cast<uint16_t *>(a.s2);
-    const int64_t groups = (a.n + 7) >> 3;
-    for (int64_t t = (int64_t)blockIdx.x * THREADS + threadIdx.x; t < groups; t += (int64_t)gridDim.x * THREADS) {
-        const int64_t o0 = t << 3;
-        const int valid = clamp_valid(a.n, o0);
-        uint32_t wp[4], wg[4], wm[4], wv[4];
-        load_bf16x8<VEC>(a.p, o0, valid, wp);
-        load_bf16x8<VEC>(a.g, o0, valid, wg);
-        load_bf16x8<VEC>(m16, o0, valid, wm);
-        load_bf16x8<VEC>(v16, o0, valid, wv);
-        float p[8], g[8], m[8], v[8];
-        unpack8(wp, p); unpack8(wg, g); unpack8(wm, m); unpack8(wv, v);
-        uint32_t rp[8], rm[8], rv[8];
-        noise8<MODE>(a.ns_p, o0, valid, rp);
-        noise8<MODE>(a.ns_m, o0, valid, rm);
-        noise8<MODE>(a.ns_v, o0, valid, rv);
-        uint32_t op[8], om[8], ov[8];
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const bool fin = fabsf(g[j]) < __builtin_huge_valf();
-            const float mj = fin ? a.b1 * m[j] + c.one_m_b1 * g[j] : 0.0f;
-            const float vj = fin ? a.b2 * v[j] + (c.one_m_b2 * g[j]) * g[j] : 0.0f;
-            const float upd = (p[j] - (c.step_c * mj) / (sqrtf(vj) + c.eps_c)) * c.decay;
-            const uint32_t pin = (j & 1) ? (wp[j >> 1] >> 16) : (wp[j >> 1] & 0xffffu);
-            op[j] = fin ? sr_bf16(upd, rp[j]) : pin;
-            om[j] = sr_bf16(mj, rm[j]);
-            ov[j] = sr_bf16(vj, rv[j]);
-        }
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            wp[j] = pack2(op[2 * j], op[2 * j + 1]);
-            wm[j] = pack2(om[2 * j], om[2 * j + 1]);
-            wv[j] = pack2(ov[2 * j], ov[2 * j + 1]);
-        }
-        store_bf16x8<VEC>(a.p, o0, valid, wp);
-        store_bf16x8<VEC>(m16, o0, valid, wm);
-        store_bf16x8<VEC>(v16, o0, valid, wv);
-    }
-}
-
-
 __global__ __launch_bounds__(THREADS) void quantize_kernel(const float *x, uint8_t *out, int64_t n,
                                                           const float *qmap, int is_signed, const QuantTable *qt) {
     __shared__ float q[256];
@@ -824,8 +778,6 @@ int msr_adamw8bit_step(uint16_t *p, const uint16_t *g, void *state1, void *state
     if (a.qtable && !aligned(a.qtable, 16)) { set_error("msr_adamw8bit_step: qtable must be 16-byte aligned"); return MSR_ERR_ALIGN; }
     a.lr = lr; a.b1 = beta1; a.b2 = beta2; a.eps = eps; a.wd = weight_decay; a.bc1 = bc1; a.bc2 = bc2;
     a.ns_p = make_noise(seed, 0, inject, n);
-    a.ns_m = make_noise(seed, 1, inject, n);
-    a.ns_v = make_noise(seed, 2, inject, n);
     hipStream_t s = (hipStream_t)stream;
     if (quantized) {
         const bool vec = aligned(p, 16) && aligned(g, 16) && aligned(state1, 8) && aligned(state2, 8);
@@ -844,10 +796,8 @@ int msr_adamw8bit_step(uint16_t *p, const uint16_t *g, void *state1, void *state
         default: launch_quant<4096>(noise_mode, vec, a, s, nblocks); break;
         }
     } else {
-        const bool vec = aligned(p, 16) && aligned(g, 16) && aligned(state1, 16) && aligned(state2, 16);
-        const unsigned grid = grid_for((n + 7) / 8, THREADS);
-        if (vec) { MSR_DISPATCH_NOISE(noise_mode, M, hipLaunchKernelGGL((adamw8bit_bf16_kernel<M, true>), dim3(grid), dim3(THREADS), 0, s, a)); }
-        else { MSR_DISPATCH_NOISE(noise_mode, M, hipLaunchKernelGGL((adamw8bit_bf16_kernel<M, false>), dim3(grid), dim3(THREADS), 0, s, a)); }
+        const msr_adamw_item it{p, g, static_cast<uint16_t *>(state1), static_cast<uint16_t *>(state2), n, bc1, bc2, seed, 0};
+        return adamw16_launch(MSR_ADAMW_8BIT16, &it, 1, lr, beta1, beta2, eps, weight_decay, noise_mode, inject, s);
     }
     return check_launch("msr_adamw8bit_step");
 }

@@ -22,6 +22,10 @@ constexpr int MSR_OK = 0;
 void set_error(const char *fmt, ...);
 int check_launch(const char *what);
 
+// One launch of the bf16-moment AdamW steps (adamw16.hip): at most 56 items, none empty.
+int adamw16_launch(int form, const msr_adamw_item *items, int32_t count, float lr, float b1, float b2, float eps, float wd,
+                   int32_t mode, const uint16_t *inject, hipStream_t s);
+
 // ---------------------------------------------------------------------------
 // bf16 helpers
 // ---------------------------------------------------------------------------

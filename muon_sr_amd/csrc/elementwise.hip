@@ -1,11 +1,8 @@
-// Memory-bound optimizer kernels for gfx950: SR gradient accumulation, bf16-
-// moment AdamW and the Muon momentum/update passes (8-bit AdamW: adamw8bit.hip).
+// Memory-bound optimizer kernels for gfx950: SR gradient accumulation and the Muon
+// momentum/update passes (AdamW: adamw16.hip, adamw8bit.hip).
 //
 // Each thread owns 8 consecutive elements (one 16-byte bf16 vector), so a
-// wave64 streams 1 KiB of every bf16 operand per access.  The quantized AdamW
-// kernel assigns block/8 consecutive threads to one quantization block and
-// reduces the block absmax with cross-lane shuffles (LDS across waves for
-// blocks above 512 elements).
+// wave64 streams 1 KiB of every bf16 operand per access.
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
@@ -161,65 +158,6 @@ __global__ __launch_bounds__(ACC_THREADS) void sr_accum_multi_kernel(AccumMultiA
             case ACC_VEC | ACC_F32: accum_tile<MODE, true, false, true>(acc, grad, ns, n, g0); break;
             default: accum_tile<MODE, true, true, true>(acc, grad, ns, n, g0); break;
         }
-    }
-}
-
-// ---------------------------------------------------------------------------
-// BF16-moment AdamW   (muon_sr/triton_adamw.py:9-72)
-// ---------------------------------------------------------------------------
-
-struct AdamWArgs {
-    uint16_t *p;
-    const uint16_t *g;
-    uint16_t *ema;
-    uint16_t *ema_sq;
-    int64_t n;
-    float lr, beta1, beta2, eps, wd, bc, bcs;
-    Noise ns_ema, ns_ema_sq, ns_p;
-};
-
-template <int MODE, bool VEC>
-__global__ __launch_bounds__(THREADS) void adamw_bf16_kernel(AdamWArgs a) {
-    const float one_m_b1 = 1.0f - a.beta1;
-    const float one_m_b2 = 1.0f - a.beta2;
-    const float step_size = a.lr / a.bc;
-    const float decay = 1.0f - a.lr * a.wd;
-    const int64_t groups = (a.n + 7) >> 3;
-    for (int64_t t = (int64_t)blockIdx.x * THREADS + threadIdx.x; t < groups; t += (int64_t)gridDim.x * THREADS) {
-        const int64_t o0 = t << 3;
-        const int valid = clamp_valid(a.n, o0);
-        uint32_t wp[4], wg[4], we[4], ws[4];
-        load_bf16x8<VEC>(a.p, o0, valid, wp);
-        load_bf16x8<VEC>(a.g, o0, valid, wg);
-        load_bf16x8<VEC>(a.ema, o0, valid, we);
-        load_bf16x8<VEC>(a.ema_sq, o0, valid, ws);
-        float p[8], g[8], e[8], s[8];
-        unpack8(wp, p); unpack8(wg, g); unpack8(we, e); unpack8(ws, s);
-        uint32_t re[8], rs[8], rp[8];
-        noise8<MODE>(a.ns_ema, o0, valid, re);
-        noise8<MODE>(a.ns_ema_sq, o0, valid, rs);
-        noise8<MODE>(a.ns_p, o0, valid, rp);
-        uint32_t oe[8], os[8], op[8];
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            float ej = a.beta1 * e[j] + one_m_b1 * g[j];
-            float sj = a.beta2 * s[j] + (one_m_b2 * g[j]) * g[j];
-            float denom = sqrtf(sj) / a.bcs + a.eps;
-            float pj = p[j] * decay;
-            pj = pj - (step_size * ej) / denom;
-            oe[j] = sr_bf16(ej, re[j]);
-            os[j] = sr_bf16(sj, rs[j]);
-            op[j] = sr_bf16(pj, rp[j]);
-        }
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            we[j] = pack2(oe[2 * j], oe[2 * j + 1]);
-            ws[j] = pack2(os[2 * j], os[2 * j + 1]);
-            wp[j] = pack2(op[2 * j], op[2 * j + 1]);
-        }
-        store_bf16x8<VEC>(a.ema, o0, valid, we);
-        store_bf16x8<VEC>(a.ema_sq, o0, valid, ws);
-        store_bf16x8<VEC>(a.p, o0, valid, wp);
     }
 }
 
@@ -456,37 +394,6 @@ int msr_sr_accum_multi(const msr_accum_item *items, int32_t count, int32_t noise
         if (rc) return rc;
     }
     return MSR_OK;
-}
-
-int msr_adamw_bf16_step(uint16_t *p, const uint16_t *g, uint16_t *ema, uint16_t *ema_sq, int64_t n, float lr,
-                        float beta1, float beta2, float eps, float weight_decay, float bias_correction,
-                        float bias_correction_sqrt, uint32_t seed, int32_t noise_mode, const uint16_t *inject,
-                        msr_stream_t stream) {
-    if (n < 0 || (n > 0 && (!p || !g || !ema || !ema_sq))) { set_error("msr_adamw_bf16_step: bad arguments"); return MSR_ERR_ARG; }
-    MSR_CHECK_MODE(noise_mode, inject);
-    {
-        const void *ops[4] = {p, g, ema, ema_sq};
-        for (int i = 0; i < 4; ++i)
-            for (int j = i + 1; j < 4; ++j)
-                if (partial_overlap(ops[i], 2 * (size_t)n, ops[j], 2 * (size_t)n)) {
-                    set_error("msr_adamw_bf16_step: operands %d and %d overlap", i, j);
-                    return MSR_ERR_OVERLAP;
-                }
-    }
-    if (n == 0) return MSR_OK;
-    AdamWArgs a;
-    a.p = p; a.g = g; a.ema = ema; a.ema_sq = ema_sq; a.n = n;
-    a.lr = lr; a.beta1 = beta1; a.beta2 = beta2; a.eps = eps; a.wd = weight_decay;
-    a.bc = bias_correction; a.bcs = bias_correction_sqrt;
-    a.ns_ema = make_noise(seed, 0, inject, n);
-    a.ns_ema_sq = make_noise(seed, 1, inject, n);
-    a.ns_p = make_noise(seed, 2, inject, n);
-    const bool vec = aligned(p, 16) && aligned(g, 16) && aligned(ema, 16) && aligned(ema_sq, 16);
-    const unsigned grid = grid_for((n + 7) / 8, THREADS);
-    hipStream_t s = (hipStream_t)stream;
-    if (vec) { MSR_DISPATCH_NOISE(noise_mode, M, hipLaunchKernelGGL((adamw_bf16_kernel<M, true>), dim3(grid), dim3(THREADS), 0, s, a)); }
-    else { MSR_DISPATCH_NOISE(noise_mode, M, hipLaunchKernelGGL((adamw_bf16_kernel<M, false>), dim3(grid), dim3(THREADS), 0, s, a)); }
-    return check_launch("msr_adamw_bf16_step");
 }
 
 int msr_muon_prepare(const void *const *grads, int32_t grad_is_f32, uint16_t *buf, uint16_t *out, int64_t numel_each,

@@ -31,7 +31,7 @@ import torch
 from torch.optim import Optimizer
 
 from . import _lib
-from .adamw import _adamw_step
+from .adamw import _adamw_add, _AdamWBatch
 from .adamw_8bit import adamw8bit_launch, init_8bit_state, split_8bit_state, TritonAdamW8bit
 
 NS_COEFFS = (3.4445, -4.7750, 2.0315)
@@ -593,29 +593,33 @@ class TritonMuonSRWithAuxAdam(_StackedBufsMixin, Optimizer):
                 if eight_bit:
                     TritonAdamW8bit._validate_group(group)   # as TritonAdamW8bit.step (triton_adamw_8bit.py:175)
 
-                for i, p in enumerate(group["params"]):
-                    assert p.dtype == torch.bfloat16, "only bfloat16 is supported."
-                    if p.grad is None:
-                        continue
-                    if p.grad.is_sparse:
-                        raise RuntimeError("TritonMuonSRWithAuxAdam does not support sparse gradients")
-                    state = self.state[p]
-                    if eight_bit:
-                        self._step_8bit(p, group, state, lr, beta1, beta2, eps, weight_decay, group_offset + i)
-                        continue
-                    if "format_version" in state:   # an 8-bit state in a group no longer set to optim_bits=8
-                        raise ValueError("Cannot change quantization configuration after state initialization")
-                    if len(state) == 0:
-                        state["step"] = 0
-                        state["ema"] = torch.zeros_like(p, dtype=torch.bfloat16, memory_format=torch.contiguous_format)
-                        state["ema_squared"] = torch.zeros_like(p, dtype=torch.bfloat16,
-                                                                memory_format=torch.contiguous_format)
-                    state["step"] += 1
-                    _adamw_step(p=p.data, g=p.grad, ema=state["ema"], ema_sq=state["ema_squared"],
-                                lr=lr, beta1=beta1, beta2=beta2, eps=eps, weight_decay=weight_decay,
-                                step=state["step"], param_idx=group_offset + i)
+                batch = _AdamWBatch(_lib.ADAMW_8BIT16 if eight_bit else _lib.ADAMW, lr, beta1, beta2, eps, weight_decay)
+                try:
+                    self._step_adamw(group, group_offset, beta1, beta2, eight_bit, batch)
+                finally:
+                    batch.flush()
 
         return loss
+
+    def _step_adamw(self, group, group_offset, beta1, beta2, eight_bit, batch):
+        for i, p in enumerate(group["params"]):
+            assert p.dtype == torch.bfloat16, "only bfloat16 is supported."
+            if p.grad is None:
+                continue
+            if p.grad.is_sparse:
+                raise RuntimeError("TritonMuonSRWithAuxAdam does not support sparse gradients")
+            state = self.state[p]
+            if eight_bit:
+                self._step_8bit(p, group, state, beta1, beta2, group_offset + i, batch)
+                continue
+            if "format_version" in state:   # an 8-bit state in a group no longer set to optim_bits=8
+                raise ValueError("Cannot change quantization configuration after state initialization")
+            if len(state) == 0:
+                state["step"] = 0
+                state["ema"] = torch.zeros_like(p, dtype=torch.bfloat16, memory_format=torch.contiguous_format)
+                state["ema_squared"] = torch.zeros_like(p, dtype=torch.bfloat16, memory_format=torch.contiguous_format)
+            state["step"] += 1
+            _adamw_add(batch, p, p.grad, state["ema"], state["ema_squared"], beta1, beta2, state["step"], group_offset + i)
 
     def load_state_dict(self, state_dict):
         """As torch's, except that the states of ``optim_bits=8`` AdamW groups keep
@@ -629,7 +633,7 @@ class TritonMuonSRWithAuxAdam(_StackedBufsMixin, Optimizer):
         super().load_state_dict(stripped)
         restore(self.state)
 
-    def _step_8bit(self, p, group, state, lr, beta1, beta2, eps, weight_decay, param_index):
+    def _step_8bit(self, p, group, state, beta1, beta2, param_index, batch):
         """8-bit AdamW group step: the TritonAdamW8bit update with seed index group_offset + i."""
         _lib.require_gpu(p, "TritonMuonSRWithAuxAdam", ValueError)
         g = p.grad
@@ -647,4 +651,4 @@ class TritonMuonSRWithAuxAdam(_StackedBufsMixin, Optimizer):
             raise ValueError("Cannot change quantization configuration after state initialization")
         state["step"] += 1
         seed = (state["step"] * 2654435761 ^ param_index * 1234567891) & 0xFFFFFFFF
-        adamw8bit_launch(p.data, g, state, lr, beta1, beta2, eps, weight_decay, seed)
+        adamw8bit_launch(p.data, g, state, group["lr"], beta1, beta2, group["eps"], group["weight_decay"], seed, batch)
