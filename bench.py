@@ -123,7 +123,7 @@ def bench_adamw8bit(steps, warmup, n=N8):
         p.grad = grads[it % 4]; it += 1
         opt.step()
     sync()
-    with LaunchTimer("msr_adamw8bit_step") as lt:
+    with LaunchTimer("msr_adamw8bit_multi") as lt:
         t0 = time.perf_counter()
         lt.on = True
         for _ in range(steps):

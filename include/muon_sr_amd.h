@@ -177,6 +177,25 @@ int msr_adamw8bit_step(uint16_t *p, const uint16_t *g, void *state1, void *state
                        float bc1, float bc2, uint32_t seed,
                        int32_t noise_mode, const uint16_t *inject, msr_stream_t stream);
 
+/* The quantized step for many tensors of one parameter group in one launch (up to 56 per
+ * launch, split internally): equal, bit for bit, to one msr_adamw8bit_step(quantized = 1) per
+ * item in order, with the same codebooks, block, hyperparameters and bias corrections.  Tensors
+ * that the fast kernel does not take (other codebooks, blocks outside 64-512, unaligned
+ * operands) run one launch each.  items: HOST array.  noise_mode: MSR_NOISE_TRITON or
+ * MSR_NOISE_PHILOX8. */
+typedef struct msr_adam8_item {
+    uint16_t *p;
+    const uint16_t *g;
+    uint8_t *state1, *state2;       /* codes [n] */
+    float *absmax1, *absmax2;       /* block scales [ceil(n/block)] */
+    int64_t n;
+    uint32_t seed;
+    int32_t reserved;               /* 0 */
+} msr_adam8_item;
+int msr_adamw8bit_multi(const msr_adam8_item *items, int32_t count, const float *qmap1, const float *qmap2,
+                        const void *qtable, int32_t block, float lr, float beta1, float beta2, float eps,
+                        float weight_decay, float bc1, float bc2, int32_t noise_mode, msr_stream_t stream);
+
 /* ---------------------------------------------------------------------------
  * (b) Muon momentum prologue over one shape group.
  * Replaces the grad->stack copy and the _muon_prepare_kernel launch of

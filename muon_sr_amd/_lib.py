@@ -36,6 +36,13 @@ class AdamWItem(ctypes.Structure):
                 ("reserved", ctypes.c_int32)]
 
 
+class Adam8Item(ctypes.Structure):
+    """msr_adam8_item (include/muon_sr_amd.h)."""
+    _fields_ = [("p", ctypes.c_void_p), ("g", ctypes.c_void_p), ("state1", ctypes.c_void_p),
+                ("state2", ctypes.c_void_p), ("absmax1", ctypes.c_void_p), ("absmax2", ctypes.c_void_p),
+                ("n", ctypes.c_int64), ("seed", ctypes.c_uint32), ("reserved", ctypes.c_int32)]
+
+
 ADAMW = 0
 ADAMW_8BIT16 = 1
 ACCUM_ZERO_INIT = 1
@@ -62,6 +69,7 @@ SIGNATURES = {
     "msr_centralize_bf16_noalloc": (ctypes.c_int, [_P, _P, _I64, _I64, _F, _P]),
     "msr_adamw8bit_step": (ctypes.c_int, [_P, _P, _P, _P, _P, _P, _P, _P, _P, _I64, _I32, _I32,
                                           _F, _F, _F, _F, _F, _F, _F, _U32, _I32, _P, _P]),
+    "msr_adamw8bit_multi": (ctypes.c_int, [_P, _I32, _P, _P, _P, _I32, _F, _F, _F, _F, _F, _F, _F, _I32, _P]),
     "msr_muon_prepare": (ctypes.c_int, [_P, _I32, _P, _P, _I64, _I32, _F, _I32, _U32, _I32, _P, _P]),
     "msr_muon_apply": (ctypes.c_int, [_P, _P, _I64, _I32, _F, _F, _F, _P, _I32, _P, _P]),
     "msr_ns_workspace_bytes": (ctypes.c_int, [_I64, _I64, _I64, _SIZE_P]),

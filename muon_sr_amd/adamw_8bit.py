@@ -3,11 +3,12 @@
 Drop-in for ``muon_sr.triton_adamw_8bit.TritonAdamW8bit`` (bab2min/muon_sr
 0.1.2, muon_sr/triton_adamw_8bit.py:102-241): same constructor, param-group
 keys, validation errors, state format (``format_version=2``) and seeds.  The
-step runs one fused gfx950 kernel per tensor (libmuon_sr_amd.so).
+step runs fused gfx950 kernels over many tensors at a time (libmuon_sr_amd.so).
 """
 from __future__ import annotations
 
 import math
+import struct
 import weakref
 
 import torch
@@ -84,22 +85,57 @@ def quant_table(state):
     return t.data_ptr()
 
 
-def adamw8bit_launch(p, g, state, lr, beta1, beta2, eps, weight_decay, seed, batch=None):
-    """One fused 8-bit (or bf16-moment) step of one tensor with state from ``init_8bit_state``.
-    ``batch``: the step's _AdamWBatch (form ADAMW_8BIT16), which takes the bf16-moment tensors."""
-    n = state["step"]
-    quant = state["optim_bits"] == 8
-    if not quant and batch is not None:
-        batch.add(p, g, state["state1"], state["state2"], 1 - beta1 ** n, 1 - beta2 ** n, seed)
-        return
-    get = lambda k: state[k].data_ptr() if k in state else None  # noqa: E731
-    qt = quant_table(state) if quant else None
-    rc = _lib.lib().msr_adamw8bit_step(
-        p.data_ptr(), g.data_ptr(), state["state1"].data_ptr(), state["state2"].data_ptr(),
-        get("absmax1"), get("absmax2"), get("qmap1"), get("qmap2"), qt, p.numel(), state["block_size"], int(quant),
-        lr, beta1, beta2, eps, weight_decay, 1 - beta1 ** n, 1 - beta2 ** n, seed,
-        _lib.noise_mode(), None, _lib.stream_of(p))
-    _lib.check(rc, "msr_adamw8bit_step")
+class _Adam8Batch:
+    """The 8-bit steps of one parameter group, launched many tensors at a time: quantized ones by
+    msr_adamw8bit_multi, bf16-moment ones by msr_adamw_multi (the reference launches one kernel
+    per tensor, muon_sr/triton_adamw_8bit.py:196-205).  Added in a ``try`` and flushed in its
+    ``finally``, as _AdamWBatch."""
+
+    _PACK = struct.Struct("=QQQQQQqIi").pack   # msr_adam8_item
+
+    def __init__(self, lr, beta1, beta2, eps, weight_decay):
+        self.hyper = (lr, beta1, beta2, eps, weight_decay)
+        self.b16 = _AdamWBatch(_lib.ADAMW_8BIT16, *self.hyper)
+        self.items, self.key = [], None
+
+    def add(self, p, g, state, seed):
+        """One tensor's step with a state from ``init_8bit_state``."""
+        n = state["step"]
+        _, beta1, beta2, _, _ = self.hyper
+        if state["optim_bits"] != 8:
+            self.b16.add(p, g, state["state1"], state["state2"], 1 - beta1 ** n, 1 - beta2 ** n, seed)
+            return
+        # what the tensors of a launch share
+        key = (state["qmap1"].data_ptr(), state["qmap2"].data_ptr(), quant_table(state), state["block_size"], n,
+               p.get_device(), _lib.stream_of(p))
+        if key != self.key:
+            self._flush8()
+            self.key = key
+        self.items.append(self._PACK(p.data_ptr(), g.data_ptr(), state["state1"].data_ptr(), state["state2"].data_ptr(),
+                                     state["absmax1"].data_ptr(), state["absmax2"].data_ptr(), p.numel(), seed, 0))
+
+    def _flush8(self):
+        if not self.items:
+            return
+        items, self.items = self.items, []
+        q1, q2, qt, block, n, _, stream = self.key
+        lr, beta1, beta2, eps, weight_decay = self.hyper
+        rc = _lib.lib().msr_adamw8bit_multi(b"".join(items), len(items), q1, q2, qt, block, lr, beta1, beta2, eps,
+                                            weight_decay, 1 - beta1 ** n, 1 - beta2 ** n, _lib.noise_mode(), stream)
+        _lib.check(rc, "msr_adamw8bit_multi")
+
+    def flush(self):
+        try:
+            self._flush8()
+        finally:
+            self.b16.flush()
+
+
+def adamw8bit_launch(p, g, state, lr, beta1, beta2, eps, weight_decay, seed):
+    """One fused 8-bit (or bf16-moment) step of one tensor with state from ``init_8bit_state``."""
+    batch = _Adam8Batch(lr, beta1, beta2, eps, weight_decay)
+    batch.add(p, g, state, seed)
+    batch.flush()
 
 
 def init_8bit_state(p, block_size, optim_bits, min_8bit_size, maps):
@@ -238,15 +274,15 @@ class TritonAdamW8bit(Optimizer):
         for group in self.param_groups:
             self._validate_group(group)
             b1, b2 = group["betas"]
-            batch = _AdamWBatch(_lib.ADAMW_8BIT16, group["lr"], b1, b2, group["eps"], group["weight_decay"])
+            batch = _Adam8Batch(group["lr"], b1, b2, group["eps"], group["weight_decay"])
             try:
-                self._step_group(group, index, b1, b2, batch)
+                self._step_group(group, index, batch)
             finally:
                 batch.flush()
             index += len(group["params"])
         return loss
 
-    def _step_group(self, group, index, b1, b2, batch):
+    def _step_group(self, group, index, batch):
         for param_index, p in enumerate(group["params"], index):
             g = p.grad
             if g is None:
@@ -264,8 +300,7 @@ class TritonAdamW8bit(Optimizer):
             if state["block_size"] != group["block_size"] or state["optim_bits"] != expected_bits:
                 raise ValueError("Cannot change quantization configuration after state initialization")
             state["step"] += 1
-            seed = step_seed(state["step"], param_index)
-            adamw8bit_launch(p, g, state, group["lr"], b1, b2, group["eps"], group["weight_decay"], seed, batch)
+            batch.add(p, g, state, step_seed(state["step"], param_index))
 
     def load_state_dict(self, state_dict):
         """Restore uint8 codes and fp32 scales without torch's cast to the

@@ -254,22 +254,15 @@ int adamw16_launch(int form, const msr_adamw_item *items, int32_t count, float l
     return check_launch("adamw16_kernel");
 }
 
-// Whether some memory that one item writes is touched by another item: such items run in
-// launches of their own, in order.
 static bool items_conflict(const msr_adamw_item *items, int32_t count) {
-    struct Range { uintptr_t lo, hi; int32_t item; bool write; };
-    Range r[4 * A16_MAXT];
+    ItemRange r[4 * A16_MAXT];
     int n = 0;
     for (int32_t i = 0; i < count; ++i) {
         const size_t b = 2 * (size_t)items[i].n;
         const void *q[4] = {items[i].p, items[i].m, items[i].v, items[i].g};
         for (int k = 0; k < 4; ++k) r[n++] = {(uintptr_t)q[k], (uintptr_t)q[k] + b, i, k < 3};
     }
-    std::sort(r, r + n, [](const Range &x, const Range &y) { return x.lo < y.lo; });
-    for (int i = 0; i < n; ++i)
-        for (int j = i + 1; j < n && r[j].lo < r[i].hi; ++j)
-            if (r[i].item != r[j].item && (r[i].write || r[j].write)) return true;
-    return false;
+    return ranges_conflict(r, n);
 }
 
 // Every item's own operands distinct (or the same buffer, updated in place).

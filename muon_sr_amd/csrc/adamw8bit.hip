@@ -30,7 +30,6 @@ struct Adam8Args {
     const float *qmap2;
     const QuantTable *qtable;
     int64_t n;
-    int64_t qb0;   // first quantization block this launch handles (the rest of the tensor is done elsewhere)
     float lr, b1, b2, eps, wd, bc1, bc2;
     Noise ns_p;
 };
@@ -109,10 +108,10 @@ __global__ __launch_bounds__((BLOCK / 8 > THREADS) ? BLOCK / 8 : THREADS) void a
         r.vs = ok ? a.absmax2[qb] : 0.0f;
     };
 
-    int64_t qb = a.qb0 + (int64_t)blockIdx.x * QB_PER_WG + sub;
+    int64_t qb = (int64_t)blockIdx.x * QB_PER_WG + sub;
     Raw nxt;
     fetch(qb, nxt);
-    for (int64_t qb0 = a.qb0 + (int64_t)blockIdx.x * QB_PER_WG; qb0 < nblocks; qb0 += stride, qb += stride) {
+    for (int64_t qb0 = (int64_t)blockIdx.x * QB_PER_WG; qb0 < nblocks; qb0 += stride, qb += stride) {
         const Raw cur = nxt;
         if (qb0 + stride < nblocks) fetch(qb + stride, nxt);
         const bool qb_ok = qb < nblocks;
@@ -201,34 +200,57 @@ __global__ __launch_bounds__((BLOCK / 8 > THREADS) ? BLOCK / 8 : THREADS) void a
 }
 
 // ---------------------------------------------------------------------------
-// Fast 8-bit step: block 256, standard codebooks, full 16-byte-aligned blocks.
+// Fast 8-bit step: blocks of 64 to 512, standard codebooks, 16-byte-aligned tensors, many
+// tensors per launch.
 //
-// A wave owns two quantization blocks (64 lanes x 8 elements) per iteration
-// and walks the tensor in a grid-stride loop, fetching its next pair while it
-// computes the current one.  Per pair the wave first forms the new moments and
-// the two block maxima, then takes one of two branches, uniformly:
-//  * fast: every gradient finite, max v' < 2^62, both block divisors in
-//    [2^-60, 2) and every update numerator |step_c * m'| zero or in
-//    [2^-90, 2^60).  The update uses sqrt_rn and div_upd, the requantization
-//    quotients use rcp_rn/div_rn and the codes come from the flat table; all of
-//    these equal the IEEE operations on these ranges (see common.hpp);
-//  * exact: anything else (non-finite gradients, extreme moments) goes through
-//    the reference arithmetic with IEEE sqrt/division, the double-precision
+// A wave owns a chunk of 512 elements (64 lanes x 8: 8 blocks of 64 down to one of 512) per
+// iteration and walks the launch's chunks (those of all its tensors, one after the other) in a
+// grid-stride loop, fetching its next chunk while it computes the current one.  Per chunk the
+// wave first forms the new moments and the block maxima, then takes one of two branches, uniformly:
+//  * fast: every gradient finite, max v' < 2^62, the block divisors in [2^-60, 2) and every
+//    update numerator |step_c * m'| zero or in [2^-90, 2^60).  The update uses sqrt_rn and
+//    div_upd, the requantization quotients use rcp_rn/div_rn and the codes come from the flat
+//    table; all of these equal the IEEE operations on these ranges (see common.hpp);
+//  * exact: anything else (non-finite gradients, extreme moments, a tensor's last partial chunk)
+//    goes through the reference arithmetic with IEEE sqrt/division, the double-precision
 //    quotients and the reference search, as in adamw8bit_quant_kernel.
 // Both branches produce the reference's bits; the fast one with about half
 // the VALU work.
+//
+// Measured: 2^28 elements in one tensor 543 us (4.97 TB/s; VALU issue bounds it).  The 73 tensors
+// of an 8-layer d = 2048 model (56 of 4-11 M elements on 8-bit states) 1705 us as one launch per
+// tensor, each staging the 38 KiB tables and filling and draining the chip, 1005 us as one;
+// blocks of 64, six tensors of 5-30 M elements with the reference's noise, 297 us on the general
+// kernel (double-precision quotients, two-level table), 205 us here.
 // ---------------------------------------------------------------------------
 
 #ifndef MSR_F8_WAVES
 #define MSR_F8_WAVES 4
 #endif
-#ifndef MSR_F8_NP
-#define MSR_F8_NP 1
-#endif
 constexpr int F8_THREADS = 64 * MSR_F8_WAVES;
-constexpr int F8_NP = MSR_F8_NP;             // adjacent pairs a wave takes per iteration
-constexpr int F8_PAIR = 512;                 // elements of a pair (2 blocks of 256: 64 lanes x 8)
-constexpr int F8_DEFER = 64;                 // pairs a wave defers to its exact pass before flushing
+constexpr int F8_CHUNK = 512;                // elements of a chunk (64 lanes x 8)
+constexpr int F8_DEFER = 64;                 // chunks a wave defers to its exact pass before flushing
+constexpr int F8_MAXT = 56;                  // tensors per launch (4 KiB of kernel arguments)
+
+struct F8Item {
+    uint16_t *p;
+    const uint16_t *g;
+    uint8_t *s1, *s2;
+    float *a1, *a2;
+    int64_t n;
+    uint32_t seed, pad;
+};
+struct F8Args {
+    int count;
+    float b1, b2;
+    Adam8Consts c;
+    const float *qmap1, *qmap2;
+    const QuantTable *qtable;
+    const uint16_t *inject;          // NOISE_INJECT (one tensor)
+    uint32_t cstart[F8_MAXT + 1];    // tensor t owns the launch's whole chunks [cstart[t], cstart[t + 1])
+    F8Item it[F8_MAXT];
+};
+static_assert(sizeof(F8Args) <= 4096, "kernel arguments");
 
 struct Raw8 {
     u32x4_t p, g;
@@ -253,16 +275,45 @@ __device__ __forceinline__ u32x4_t with_word(u32x4_t w, int k, uint32_t x) {
     return w;
 }
 
-// The reference arithmetic for one full pair: the rare branch of the fast
-// kernel.  Element loops stay rolled and the moments are recomputed for the
+__device__ __forceinline__ Noise f8_noise(const F8Args &a, const F8Item &it) {
+    Noise ns;
+    ns.key = seed_key(it.seed, 0);
+    ns.inject = a.inject;
+    return ns;
+}
+
+// The reference arithmetic for one chunk, which may be a tensor's last, partial one: the rare
+// branch of the fast kernel.  Element loops stay rolled and the moments are recomputed for the
 // requantization pass, so this branch needs fewer registers than the fast one
 // and does not lower the kernel's occupancy.
-template <int MODE>
-__device__ __forceinline__ void adam8_pair_exact(const Adam8Args &a, const Raw8 &cur, int64_t o0, int64_t qb,
-                                                 const float *q1s, const float *q2s) {
-    const Adam8Consts c = adam8_consts(a);
-    uint8_t *m8 = static_cast<uint8_t *>(a.s1);
-    uint8_t *v8 = static_cast<uint8_t *>(a.s2);
+template <int MODE, int LB>
+__device__ __forceinline__ void adam8_chunk_exact(const F8Args &a, const F8Item &it, int64_t lc, uint32_t lane,
+                                                  const float *q1s, const float *q2s) {
+    const Adam8Consts &c = a.c;
+    const Noise ns = f8_noise(a, it);
+    const int64_t o0 = lc * F8_CHUNK + lane * 8;
+    const int valid = clamp_valid(it.n, o0);
+    const int64_t qb = lc * (64 / LB) + lane / LB;
+    const bool has = qb * (8 * LB) < it.n;       // the lane's block exists
+    Raw8 cur;
+    if (valid == 8) {
+        cur.p = ld_nt4(it.p + o0);
+        cur.g = ld_nt4(it.g + o0);
+        cur.mc = ld_nt2(it.s1 + o0);
+        cur.vc = ld_nt2(it.s2 + o0);
+    } else {
+        uint32_t wp[4], wg[4], cm[8], cv[8];
+        load_bf16x8<false>(it.p, o0, valid, wp);
+        load_bf16x8<false>(it.g, o0, valid, wg);
+        load_u8x8<false>(it.s1, o0, valid, 127u, cm);
+        load_u8x8<false>(it.s2, o0, valid, 0u, cv);
+        cur.p = u32x4_t{wp[0], wp[1], wp[2], wp[3]};
+        cur.g = u32x4_t{wg[0], wg[1], wg[2], wg[3]};
+        cur.mc = u32x2_t{cm[0] | cm[1] << 8 | cm[2] << 16 | cm[3] << 24, cm[4] | cm[5] << 8 | cm[6] << 16 | cm[7] << 24};
+        cur.vc = u32x2_t{cv[0] | cv[1] << 8 | cv[2] << 16 | cv[3] << 24, cv[4] | cv[5] << 8 | cv[6] << 16 | cv[7] << 24};
+    }
+    cur.ms = has ? it.a1[qb] : 0.0f;
+    cur.vs = has ? it.a2[qb] : 0.0f;
     // moments of element j, with non-finite gradients masked (:65-72)
     auto moments = [&](int j, float &mj, float &vj, float &gj, bool &fin) {
         const uint32_t gw = word_at(cur.g, j >> 1);
@@ -283,15 +334,23 @@ __device__ __forceinline__ void adam8_pair_exact(const Adam8Args &a, const Raw8 
         const uint32_t pw = word_at(cur.p, j >> 1);
         const float pj = (j & 1) ? bf16_hi(pw) : bf16_lo(pw);
         const float upd = (pj - (c.step_c * mj) / (sqrtf(vj) + c.eps_c)) * c.decay;   // :74
-        const uint32_t op = fin ? sr_bf16(upd, noise1<MODE>(a.ns_p, o0 + j)) : ((pw >> (16 * (j & 1))) & 0xffffu);  // :75-78
+        const uint32_t rn = MODE == NOISE_INJECT && j >= valid ? 0u : noise1<MODE>(ns, o0 + j);
+        const uint32_t op = fin ? sr_bf16(upd, rn) : ((pw >> (16 * (j & 1))) & 0xffffu);  // :75-78
         const uint32_t ow = word_at(pout, j >> 1);
         pout = with_word(pout, j >> 1, (j & 1) ? ((ow & 0xffffu) | (op << 16)) : ((ow & 0xffff0000u) | op));
-        mmax = fmaxf(mmax, fabsf(mj));
-        vmax = fmaxf(vmax, fabsf(vj));
+        if (j < valid) {
+            mmax = fmaxf(mmax, fabsf(mj));
+            vmax = fmaxf(vmax, fabsf(vj));
+        }
     }
-    st_nt4(a.p + o0, pout);
+    if (valid == 8) {
+        st_nt4(it.p + o0, pout);
+    } else {
+        const uint32_t w[4] = {pout.x, pout.y, pout.z, pout.w};
+        store_bf16x8<false>(it.p, o0, valid, w);
+    }
 #pragma unroll
-    for (int off = 16; off >= 1; off >>= 1) {                                // :80-81
+    for (int off = LB / 2; off >= 1; off >>= 1) {                            // :80-81
         mmax = fmaxf(mmax, __shfl_xor(mmax, off, 64));
         vmax = fmaxf(vmax, __shfl_xor(vmax, off, 64));
     }
@@ -310,11 +369,21 @@ __device__ __forceinline__ void adam8_pair_exact(const Adam8Args &a, const Raw8 
         const uint32_t sh = 8u * (uint32_t)(j & 3);
         if (j < 4) { mc0 |= mc << sh; vc0 |= vc << sh; } else { mc1 |= mc << sh; vc1 |= vc << sh; }
     }
-    st_nt2(m8 + o0, u32x2_t{mc0, mc1});
-    st_nt2(v8 + o0, u32x2_t{vc0, vc1});
-    if ((threadIdx.x & 31) == 0) {
-        a.absmax1[qb] = mmax;                                                // :86
-        a.absmax2[qb] = vmax;                                                // :87
+    if (valid == 8) {
+        st_nt2(it.s1 + o0, u32x2_t{mc0, mc1});
+        st_nt2(it.s2 + o0, u32x2_t{vc0, vc1});
+    } else {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            if (j < valid) {
+                it.s1[o0 + j] = (uint8_t)((j < 4 ? mc0 : mc1) >> (8 * (j & 3)));
+                it.s2[o0 + j] = (uint8_t)((j < 4 ? vc0 : vc1) >> (8 * (j & 3)));
+            }
+        }
+    }
+    if (has && lane % LB == 0) {
+        it.a1[qb] = mmax;                                                    // :86
+        it.a2[qb] = vmax;                                                    // :87
     }
 }
 
@@ -325,8 +394,8 @@ struct F8Consts {
     int32_t tm1;
 };
 
-__device__ __forceinline__ F8Consts f8_consts(const Adam8Args &a) {
-    const Adam8Consts c = adam8_consts(a);
+__device__ __forceinline__ F8Consts f8_consts(const F8Args &a) {
+    const Adam8Consts &c = a.c;
     F8Consts k;
     k.b1 = vgpr(a.b1); k.omb1 = vgpr(c.one_m_b1); k.b2 = vgpr(a.b2); k.omb2 = vgpr(c.one_m_b2);
     k.step_c = vgpr(c.step_c); k.eps_c = vgpr(c.eps_c); k.decay = vgpr(c.decay);
@@ -339,123 +408,100 @@ __device__ __forceinline__ F8Consts f8_consts(const Adam8Args &a) {
     return k;
 }
 
-// NP adjacent pairs of quantization blocks (pair pr0 + q: the wave's 64 lanes x 8 elements)
-// on the fast branch.  Returns the mask of the pairs done; a pair whose bit is clear needs
-// the exact arithmetic in some lane and has written nothing (the caller defers it to
-// adam8_pair_exact).  The pairs' instruction chains are independent, so with NP > 1 the
-// scheduler interleaves them: one wave keeps NP pairs of latency in flight.
-template <int MODE, int NP>
-__device__ __forceinline__ uint32_t adam8_pairs_fast(const Adam8Args &a, const F8Consts &k, const Raw8 (&raw)[NP],
-                                                     int64_t pr0, uint32_t lane, const float *q1s, const float *q2s,
-                                                     const uint32_t *s_flat) {
-    float p[NP][8], m[NP][8], v[NP][8], mx[NP], vx[NP];
-    int32_t neg[NP];
+// Chunk lc of a tensor (the wave's 64 lanes x 8 elements) on the fast branch.  Returns whether
+// it was done; otherwise it needs the exact arithmetic in some lane and has written
+// nothing (the caller defers it to adam8_chunk_exact).
+template <int MODE, int LB>
+__device__ __forceinline__ bool adam8_chunk_fast(const F8Args &a, const F8Item &it, const F8Consts &k, const Raw8 &raw,
+                                                 int64_t lc, uint32_t lane, const float *q1s, const float *q2s,
+                                                 const uint32_t *s_flat) {
+    float p[8], g[8], m[8], v[8];
 #pragma unroll
-    for (int q = 0; q < NP; ++q) {
-        float g[8];
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            p[q][j] = bf16_at(raw[q].p, j);
-            g[j] = bf16_at(raw[q].g, j);
-        }
-        // a sum of the 8 gradients is finite iff all of them are (or it overflows: exact)
-        const float gsum = ((g[0] + g[1]) + (g[2] + g[3])) + ((g[4] + g[5]) + (g[6] + g[7]));
-        float mxq = 0.0f, vxq = 0.0f;
-        uint32_t mnz = 0xffffffffu;   // min of 2 bits(|m|) - 2: (bits of the smallest nonzero |m|) - 1, times 2
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const float mq = q1s[byte_of(raw[q].mc, j)] * raw[q].ms;               // :65
-            const float vq = q2s[byte_of(raw[q].vc, j)] * raw[q].vs;               // :66
-            m[q][j] = k.b1 * mq + k.omb1 * g[j];                                   // :71
-            v[q][j] = k.b2 * vq + (k.omb2 * g[j]) * g[j];                          // :72
-            mxq = fmaxf(mxq, fabsf(m[q][j]));
-            vxq = fmaxf(vxq, v[q][j]);
-            mnz = min(mnz, (__float_as_uint(m[q][j]) << 1) - 2u);                  // +-0 gives 0xfffffffe
-        }
-        halfwave_max2(mxq, vxq);                                                   // :80-81
-        mx[q] = mxq;
-        vx[q] = vxq;
-        const float md = mxq > 0.0f ? mxq : 1.0f;                                  // :82
-        const float vd = vxq > 0.0f ? vxq : 1.0f;                                  // :83
-        // Fast-branch conditions as sign bits of differences of non-negative bit patterns:
-        // finite gradients and block scales, vs >= +0 (then m' is finite or +-inf and v' >= 0
-        // finite or +inf, never NaN, so the maxima above are exact), max v' < 2^62, both
-        // divisors in [2^-60, 2) and the update's numerators |step_c * m'| zero or in
-        // [2^-90, 2^60) (the block maximum of |m'| bounds them from above).
-        const int32_t FMAX = 0x7f7fffff, DLO = 0x21800000, DHI = 0x3fffffff, VXHI = 0x5e7fffff;
-        const int32_t NHI = 0x5d7fffff;   // bits(2^60) - 1
-        const int32_t gsb = (int32_t)(__float_as_uint(gsum) & 0x7fffffffu);
-        const int32_t msb = (int32_t)(__float_as_uint(raw[q].ms) & 0x7fffffffu);
-        const int32_t vsb = (int32_t)__float_as_uint(raw[q].vs), vxb = (int32_t)__float_as_uint(vxq);
-        const int32_t mdb = (int32_t)__float_as_uint(md), vdb = (int32_t)__float_as_uint(vd);
-        const int32_t nxb = (int32_t)__float_as_uint(k.step_abs * mxq), mnb = (int32_t)(mnz >> 1);
-        neg[q] = (FMAX - gsb) | (FMAX - msb) | vsb | (FMAX - vsb) | (VXHI - vxb) | (mdb - DLO) |
-                 (DHI - mdb) | (vdb - DLO) | (DHI - vdb) | (NHI - nxb) | (mnb - k.tm1);
+    for (int j = 0; j < 8; ++j) {
+        p[j] = bf16_at(raw.p, j);
+        g[j] = bf16_at(raw.g, j);
     }
-    uint32_t ok = 0;
+    // a sum of the 8 gradients is finite iff all of them are (or it overflows: exact)
+    const float gsum = ((g[0] + g[1]) + (g[2] + g[3])) + ((g[4] + g[5]) + (g[6] + g[7]));
+    float mx = 0.0f, vx = 0.0f;
+    uint32_t mnz = 0xffffffffu;   // min of 2 bits(|m|) - 2: (bits of the smallest nonzero |m|) - 1, times 2
 #pragma unroll
-    for (int q = 0; q < NP; ++q)
-        if (__builtin_amdgcn_ballot_w64(neg[q] < 0) == 0) ok |= 1u << q;
-    // the update, its SR store and the requantization of pair q
-    auto finish = [&](int q) {
-        const int64_t o0 = (pr0 + q) * F8_PAIR + lane * 8;
-        uint32_t rp[8], w[8];
-        noise8<MODE>(a.ns_p, o0, 8, rp);
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const float den = __builtin_fmaf(sqrt_rn_x2p32(v[q][j]), 0x1p-32f, k.eps_c);   // :74 sqrt(v) + eps
-            const float upd = (p[q][j] - div_upd(k.step_c * m[q][j], den)) * k.decay;
-            w[j] = __float_as_uint(upd) + rp[j];                                           // :75-78 (SR)
-        }
-        stu_nt4(a.p + (pr0 + q) * F8_PAIR, lane * 16u,
-                u32x4_t{__builtin_amdgcn_perm(w[1], w[0], 0x07060302u), __builtin_amdgcn_perm(w[3], w[2], 0x07060302u),
-                        __builtin_amdgcn_perm(w[5], w[4], 0x07060302u), __builtin_amdgcn_perm(w[7], w[6], 0x07060302u)});
-        const float md = mx[q] > 0.0f ? mx[q] : 1.0f, vd = vx[q] > 0.0f ? vx[q] : 1.0f;
-        const float ym = rcp_rn(md), yv = rcp_rn(vd);
-        uint32_t rm[8], rv[8];
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            rm[j] = qf_signed(div_rn(m[q][j], md, ym), s_flat, k.lo1, k.scap);            // :82,84
-            rv[j] = qf_unsigned(div_rn(v[q][j], vd, yv), s_flat + QF_SIGNED, k.lo1);     // :83,85
-        }
-        stu_nt2(static_cast<uint8_t *>(a.s1) + (pr0 + q) * F8_PAIR, lane * 8u,
-                u32x2_t{pack_codes(rm[0], rm[1], rm[2], rm[3]), pack_codes(rm[4], rm[5], rm[6], rm[7])});
-        stu_nt2(static_cast<uint8_t *>(a.s2) + (pr0 + q) * F8_PAIR, lane * 8u,
-                u32x2_t{pack_codes(rv[0], rv[1], rv[2], rv[3]), pack_codes(rv[4], rv[5], rv[6], rv[7])});
-        if ((lane & 31) == 0) {
-            stu_f32(a.absmax1 + (pr0 + q) * 2, (lane >> 5) * 4u, mx[q]);         // :86
-            stu_f32(a.absmax2 + (pr0 + q) * 2, (lane >> 5) * 4u, vx[q]);         // :87
-        }
-    };
-    constexpr uint32_t ALL = (1u << NP) - 1u;
-    if (ok == ALL) {
-#pragma unroll
-        for (int q = 0; q < NP; ++q) finish(q);
-    } else {
-#pragma unroll
-        for (int q = 0; q < NP; ++q)
-            if ((ok >> q) & 1u) finish(q);
+    for (int j = 0; j < 8; ++j) {
+        const float mq = q1s[byte_of(raw.mc, j)] * raw.ms;                     // :65
+        const float vq = q2s[byte_of(raw.vc, j)] * raw.vs;                     // :66
+        m[j] = k.b1 * mq + k.omb1 * g[j];                                      // :71
+        v[j] = k.b2 * vq + (k.omb2 * g[j]) * g[j];                             // :72
+        mx = fmaxf(mx, fabsf(m[j]));
+        vx = fmaxf(vx, v[j]);
+        mnz = min(mnz, (__float_as_uint(m[j]) << 1) - 2u);                     // +-0 gives 0xfffffffe
     }
-    return ok;
+    group_max2<LB>(mx, vx);                                                    // :80-81
+    const float md = mx > 0.0f ? mx : 1.0f;                                    // :82
+    const float vd = vx > 0.0f ? vx : 1.0f;                                    // :83
+    // Fast-branch conditions as sign bits of differences of non-negative bit patterns:
+    // finite gradients and block scales, vs >= +0 (then m' is finite or +-inf and v' >= 0
+    // finite or +inf, never NaN, so the maxima above are exact), max v' < 2^62, both
+    // divisors in [2^-60, 2) and the update's numerators |step_c * m'| zero or in
+    // [2^-90, 2^60) (the block maximum of |m'| bounds them from above).
+    const int32_t FMAX = 0x7f7fffff, DLO = 0x21800000, DHI = 0x3fffffff, VXHI = 0x5e7fffff;
+    const int32_t NHI = 0x5d7fffff;   // bits(2^60) - 1
+    const int32_t gsb = (int32_t)(__float_as_uint(gsum) & 0x7fffffffu);
+    const int32_t msb = (int32_t)(__float_as_uint(raw.ms) & 0x7fffffffu);
+    const int32_t vsb = (int32_t)__float_as_uint(raw.vs), vxb = (int32_t)__float_as_uint(vx);
+    const int32_t mdb = (int32_t)__float_as_uint(md), vdb = (int32_t)__float_as_uint(vd);
+    const int32_t nxb = (int32_t)__float_as_uint(k.step_abs * mx), mnb = (int32_t)(mnz >> 1);
+    const int32_t neg = (FMAX - gsb) | (FMAX - msb) | vsb | (FMAX - vsb) | (VXHI - vxb) | (mdb - DLO) |
+                        (DHI - mdb) | (vdb - DLO) | (DHI - vdb) | (NHI - nxb) | (mnb - k.tm1);
+    if (__builtin_amdgcn_ballot_w64(neg < 0) != 0) return false;
+    // the update, its SR store and the requantization
+    const int64_t base = lc * F8_CHUNK, o0 = base + lane * 8;
+    uint32_t rp[8], w[8];
+    noise8<MODE>(f8_noise(a, it), o0, 8, rp);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        const float den = __builtin_fmaf(sqrt_rn_x2p32(v[j]), 0x1p-32f, k.eps_c);              // :74 sqrt(v) + eps
+        const float upd = (p[j] - div_upd(k.step_c * m[j], den)) * k.decay;
+        w[j] = __float_as_uint(upd) + rp[j];                                                   // :75-78 (SR)
+    }
+    stu_nt4(it.p + base, lane * 16u,
+            u32x4_t{__builtin_amdgcn_perm(w[1], w[0], 0x07060302u), __builtin_amdgcn_perm(w[3], w[2], 0x07060302u),
+                    __builtin_amdgcn_perm(w[5], w[4], 0x07060302u), __builtin_amdgcn_perm(w[7], w[6], 0x07060302u)});
+    const float ym = rcp_rn(md), yv = rcp_rn(vd);
+    uint32_t rm[8], rv[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        rm[j] = qf_signed(div_rn(m[j], md, ym), s_flat, k.lo1, k.scap);            // :82,84
+        rv[j] = qf_unsigned(div_rn(v[j], vd, yv), s_flat + QF_SIGNED, k.lo1);     // :83,85
+    }
+    stu_nt2(it.s1 + base, lane * 8u,
+            u32x2_t{pack_codes(rm[0], rm[1], rm[2], rm[3]), pack_codes(rm[4], rm[5], rm[6], rm[7])});
+    stu_nt2(it.s2 + base, lane * 8u,
+            u32x2_t{pack_codes(rv[0], rv[1], rv[2], rv[3]), pack_codes(rv[4], rv[5], rv[6], rv[7])});
+    if (lane % LB == 0) {
+        stu_f32(it.a1 + lc * (64 / LB), (lane / LB) * 4u, mx);               // :86
+        stu_f32(it.a2 + lc * (64 / LB), (lane / LB) * 4u, vx);               // :87
+    }
+    return true;
 }
 
-// Raw inputs of pair pr (wave-uniform), loaded into VGPRs: buffer loads from the pair's
-// base address, so the address arithmetic runs on the scalar unit.
-__device__ __forceinline__ Raw8 fetch_pair(const Adam8Args &a, int64_t pr, uint32_t lane) {
+// Raw inputs of chunk lc (wave-uniform) of a tensor, loaded into VGPRs: buffer loads from the
+// chunk's base address, so the address arithmetic runs on the scalar unit.
+template <int LB>
+__device__ __forceinline__ Raw8 fetch_chunk(const F8Item &it, int64_t lc, uint32_t lane) {
     Raw8 r;
-    r.p = ldu_nt4(a.p + pr * F8_PAIR, lane * 16u);
-    r.g = ldu_nt4(a.g + pr * F8_PAIR, lane * 16u);
-    r.mc = ldu_nt2(static_cast<const uint8_t *>(a.s1) + pr * F8_PAIR, lane * 8u);
-    r.vc = ldu_nt2(static_cast<const uint8_t *>(a.s2) + pr * F8_PAIR, lane * 8u);
-    r.ms = ldu_f32(a.absmax1 + pr * 2, (lane >> 5) * 4u);
-    r.vs = ldu_f32(a.absmax2 + pr * 2, (lane >> 5) * 4u);
+    r.p = ldu_nt4(it.p + lc * F8_CHUNK, lane * 16u);
+    r.g = ldu_nt4(it.g + lc * F8_CHUNK, lane * 16u);
+    r.mc = ldu_nt2(it.s1 + lc * F8_CHUNK, lane * 8u);
+    r.vc = ldu_nt2(it.s2 + lc * F8_CHUNK, lane * 8u);
+    r.ms = ldu_f32(it.a1 + lc * (64 / LB), (lane / LB) * 4u);
+    r.vs = ldu_f32(it.a2 + lc * (64 / LB), (lane / LB) * 4u);
     return r;
 }
 
-// The pairs a wave walks: pr, pr + stride, ... below end (groups of np adjacent pairs).
+// The whole chunks a wave walks: c, c + stride, ... below the launch's count.
 // The work-groups of one XCD take runs of MSR_F8_XCD_RUN consecutive places of the
 // grid-stride order (-1: a run of g / 8, the XCD's whole share of each sweep).  A run of 4
-// work-groups is 16 pairs, one 128-byte line of each block-scale array, which is then
+// work-groups is 16 chunks, one 128-byte line of each block-scale array at block 256, which is then
 // written from one XCD's L2 rather than from four.  Measured on 2^28 elements (A/B in one
 // process, bit-exact): the step 2.4 % faster than places in dispatch order (runs of 32
 // and g / 8: 1.4 % and 0 %), the access-pattern probe at 16 waves per CU 8.5 % faster.
@@ -463,25 +509,23 @@ __device__ __forceinline__ Raw8 fetch_pair(const Adam8Args &a, int64_t pr, uint3
 #define MSR_F8_XCD_RUN 4
 #endif
 struct F8Walk {
-    int64_t pr, end, stride;
+    int64_t c, stride;
 };
-__device__ __forceinline__ F8Walk f8_walk(int64_t npairs, int wave, int np) {
+__device__ __forceinline__ F8Walk f8_walk(int wave) {
     const int64_t b = blockIdx.x, g = gridDim.x;
     constexpr int W = F8_THREADS / 64;
     const int64_t run = MSR_F8_XCD_RUN >= 0 ? MSR_F8_XCD_RUN : ((g & 7) == 0 ? g / 8 : 0);
-    F8Walk w;
-    w.pr = (xcd_place(b, g, run) * W + wave) * np;
-    w.end = npairs;
-    w.stride = g * W * np;
-    return w;
+    return F8Walk{xcd_place(b, g, run) * W + wave, g * W};
 }
 
 // Four waves per SIMD (16 per CU) hide the branch's latency chains: at most 128 VGPRs.
 #ifndef MSR_F8_MIN_WAVES
 #define MSR_F8_MIN_WAVES 4
 #endif
-template <int MODE>
-__global__ __launch_bounds__(F8_THREADS, MSR_F8_MIN_WAVES) void adamw8bit_fast_kernel(Adam8Args a, int64_t npairs) {
+// MULTI: more than one tensor (a launch of one keeps its pointers and Philox key schedule out of
+// the loop: 1.6 % on 2^28 elements).
+template <int MODE, int LB, bool MULTI>
+__global__ __launch_bounds__(F8_THREADS, MSR_F8_MIN_WAVES) void adamw8bit_fast_kernel(F8Args a) {
     __shared__ float q1s[256], q2s[256];
     __shared__ uint32_t s_flat[QF_TOTAL];
     __shared__ uint32_t s_deferred[F8_THREADS / 64][F8_DEFER];
@@ -493,77 +537,92 @@ __global__ __launch_bounds__(F8_THREADS, MSR_F8_MIN_WAVES) void adamw8bit_fast_k
     __syncthreads();
     const F8Consts k = f8_consts(a);
     const uint32_t lane = threadIdx.x & 63u;
-    // the pair index is wave-uniform: addresses are a scalar base plus a fixed lane offset.
-    // Each wave takes F8_NP adjacent pairs per iteration (npairs is a multiple of F8_NP).
+    // the chunk index is wave-uniform: addresses are a scalar base plus a fixed lane offset
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    const F8Walk walk = f8_walk(npairs, wave, F8_NP);
-    const int64_t wstride = walk.stride, pend = walk.end;
-    int64_t pr = walk.pr;
+    const F8Walk walk = f8_walk(wave);
+    const uint32_t stride = (uint32_t)walk.stride, end = a.cstart[MULTI ? a.count : 1];
+    uint32_t c = (uint32_t)walk.c;
+    // The tensor of a chunk stays in scalar registers and is read again only where the walk
+    // enters another one.
+    struct Tensor {
+        F8Item it;
+        uint32_t c0, c1;
+        int t;
+    };
+    auto enter = [&](uint32_t x, Tensor &w) {   // the tensor of chunk x, not before w's
+        while (x >= w.c1) {
+            ++w.t;
+            w.c0 = w.c1;
+            w.c1 = a.cstart[w.t + 1];
+        }
+        w.it = a.it[w.t];
+    };
     uint32_t *deferred = s_deferred[wave];
+    Tensor wn{a.it[0], 0u, a.cstart[1], 0};
     for (;;) {
         int ndef = 0;
-        Raw8 nxt[F8_NP];
-        if (pr < pend) {
-#pragma unroll
-            for (int q = 0; q < F8_NP; ++q) nxt[q] = fetch_pair(a, pr + q, lane);
+        Raw8 nxt;
+        if (c < end) {
+            if (MULTI && c >= wn.c1) enter(c, wn);
+            nxt = fetch_chunk<LB>(wn.it, c - wn.c0, lane);
         }
-        for (; pr < pend; pr += wstride) {
-            Raw8 raw[F8_NP];
-#pragma unroll
-            for (int q = 0; q < F8_NP; ++q) raw[q] = nxt[q];
-            if (pr + wstride < pend) {
-#pragma unroll
-                for (int q = 0; q < F8_NP; ++q) nxt[q] = fetch_pair(a, pr + wstride + q, lane);
+        Tensor w = wn;
+        for (; c < end; c += stride) {
+            const Raw8 raw = nxt;
+            if (MULTI && w.t != wn.t) w = wn;
+            if (c + stride < end) {
+                if (MULTI && c + stride >= wn.c1) enter(c + stride, wn);
+                nxt = fetch_chunk<LB>(wn.it, c + stride - wn.c0, lane);
             }
-            const uint32_t ok = adam8_pairs_fast<MODE, F8_NP>(a, k, raw, pr, lane, q1s, q2s, s_flat);
-            if (ok == (1u << F8_NP) - 1u) continue;
-#pragma unroll
-            for (int q = 0; q < F8_NP; ++q) {
-                if ((ok >> q) & 1u) continue;
-                if (lane == 0) deferred[ndef] = (uint32_t)(pr + q);
-                ++ndef;
-            }
-            if (ndef > F8_DEFER - F8_NP) {
-                pr += wstride;
+            if (adam8_chunk_fast<MODE, LB>(a, w.it, k, raw, c - w.c0, lane, q1s, q2s, s_flat)) continue;
+            if (lane == 0) deferred[ndef] = c;
+            if (++ndef == F8_DEFER) {
+                c += stride;
                 break;
             }
         }
         __builtin_amdgcn_wave_barrier();   // lane 0's list writes precede the wave's reads
         for (int i = 0; i < ndef; ++i) {
-            const int64_t pe = (int64_t)__builtin_amdgcn_readfirstlane(deferred[i]);
-            adam8_pair_exact<MODE>(a, fetch_pair(a, pe, lane), pe * F8_PAIR + lane * 8, pe * 2 + (lane >> 5), q1s, q2s);
+            const uint32_t ce = (uint32_t)__builtin_amdgcn_readfirstlane((int)deferred[i]);
+            Tensor wd{a.it[0], 0u, a.cstart[1], 0};
+            if (MULTI && ce >= wd.c1) enter(ce, wd);
+            adam8_chunk_exact<MODE, LB>(a, wd.it, ce - wd.c0, lane, q1s, q2s);
         }
-        if (pr >= pend) break;
+        if (c >= end) break;
+    }
+    // the tensors' last, partial chunks, spread over the waves from the last one down
+    for (int64_t t = walk.stride - 1 - walk.c; t < a.count; t += walk.stride) {
+        const F8Item &it = a.it[t];
+        if (it.n % F8_CHUNK) adam8_chunk_exact<MODE, LB>(a, it, it.n / F8_CHUNK, lane, q1s, q2s);
     }
 }
 
 // Streaming probe of the fast kernel's memory accesses (a measurement aid, no counterpart
-// in the reference): the same pair walk, loads and stores as adamw8bit_fast_kernel (read p,
+// in the reference): the same chunk walk, loads and stores as adamw8bit_fast_kernel at block 256 (read p,
 // g 16 B and the m, v codes 8 B per lane, and the two block scales; write p, m, v and the
 // scales), with one integer operation per word in place of the arithmetic.  Its rate is what
 // the memory system delivers for this pattern at a given grid and occupancy (set by the
 // dynamic LDS of each work-group); the step cannot stream faster.
-__global__ __launch_bounds__(F8_THREADS) void stream8_probe_kernel(Adam8Args a, int64_t npairs) {
+__global__ __launch_bounds__(F8_THREADS) void stream8_probe_kernel(F8Item it, int64_t chunks) {
     extern __shared__ uint32_t occupancy_pad[];
     const uint32_t lane = threadIdx.x & 63u;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    const F8Walk walk = f8_walk(npairs, wave, 1);
-    const int64_t wstride = walk.stride, pend = walk.end;
-    int64_t pr = walk.pr;
-    if (pr >= pend) return;
-    Raw8 nxt = fetch_pair(a, pr, lane);
-    for (; pr < pend; pr += wstride) {
+    const F8Walk walk = f8_walk(wave);
+    int64_t c = walk.c;
+    if (c >= chunks) return;
+    Raw8 nxt = fetch_chunk<32>(it, c, lane);
+    for (; c < chunks; c += walk.stride) {
         const Raw8 raw = nxt;
-        if (pr + wstride < pend) nxt = fetch_pair(a, pr + wstride, lane);
-        const int64_t o0 = pr * F8_PAIR + lane * 8;
+        if (c + walk.stride < chunks) nxt = fetch_chunk<32>(it, c + walk.stride, lane);
+        const int64_t o0 = c * F8_CHUNK + lane * 8;
         const u32x4_t pw = raw.p ^ raw.g;
-        st_nt4(a.p + o0, pw);
-        st_nt2(static_cast<uint8_t *>(a.s1) + o0, u32x2_t{raw.mc.x ^ 0x01010101u, raw.mc.y ^ 0x01010101u});
-        st_nt2(static_cast<uint8_t *>(a.s2) + o0, u32x2_t{raw.vc.x + 0x01010101u, raw.vc.y + 0x01010101u});
+        st_nt4(it.p + o0, pw);
+        st_nt2(it.s1 + o0, u32x2_t{raw.mc.x ^ 0x01010101u, raw.mc.y ^ 0x01010101u});
+        st_nt2(it.s2 + o0, u32x2_t{raw.vc.x + 0x01010101u, raw.vc.y + 0x01010101u});
         if ((lane & 31) == 0) {
-            const int64_t qb = pr * 2 + (lane >> 5);
-            a.absmax1[qb] = raw.ms + 1.0f;
-            a.absmax2[qb] = raw.vs * 0.5f;
+            const int64_t qb = c * 2 + (lane >> 5);
+            it.a1[qb] = raw.ms + 1.0f;
+            it.a2[qb] = raw.vs * 0.5f;
         }
     }
 }
@@ -719,7 +778,7 @@ static void launch_quant(int mode, bool vec, const Adam8Args &a, hipStream_t s, 
     constexpr int TPB = BLOCK / 8;
     constexpr int WG = TPB > THREADS ? TPB : THREADS;
     constexpr int QB_PER_WG = WG / TPB;
-    const unsigned grid = grid_for(nblocks - a.qb0, QB_PER_WG, 256 * 8);
+    const unsigned grid = grid_for(nblocks, QB_PER_WG, 256 * 8);
     const bool qtab = a.qtable != nullptr;
     if (mode == NOISE_TRITON) launch_quant_mode<NOISE_TRITON, BLOCK>(vec, qtab, a, s, grid, WG);
     else if (mode == NOISE_PHILOX8) launch_quant_mode<NOISE_PHILOX8, BLOCK>(vec, qtab, a, s, grid, WG);
@@ -730,19 +789,135 @@ static void launch_quant(int mode, bool vec, const Adam8Args &a, hipStream_t s, 
 #define MSR_F8_GRID_CAP 2048   // twice the resident work-groups (4 per CU on 256 CUs): measured best
 #endif
 
-// Fast kernel over the first 2 * npairs blocks (block 256); returns blocks done.
-static int64_t launch_fast8(int mode, const Adam8Args &a, hipStream_t s, int64_t nfull) {
-    const int64_t npairs = nfull / (2 * F8_NP) * F8_NP;   // whole groups of F8_NP pairs; the rest goes to the general kernel
-    if (npairs == 0 || npairs >= ((int64_t)1 << 31)) return 0;   // deferred pairs are recorded as int32
-    // the update's divisor sqrt(v') + eps_c must lie in [2^-60, 2^32) (sqrt(v') < 2^31 is
-    // checked per pair), and step_c must be finite: the same fp32 arithmetic as adam8_consts
-    const float sqrt_bc2 = sqrtf(a.bc2), eps_c = sqrt_bc2 * a.eps, step_c = (a.lr * sqrt_bc2) / a.bc1;
-    if (!(eps_c >= 0x1p-60f && eps_c <= 0x1p30f) || !std::isfinite(step_c)) return 0;
-    const unsigned grid = grid_for(npairs / F8_NP, F8_THREADS / 64, MSR_F8_GRID_CAP);
-    if (mode == NOISE_TRITON) hipLaunchKernelGGL((adamw8bit_fast_kernel<NOISE_TRITON>), dim3(grid), dim3(F8_THREADS), 0, s, a, npairs);
-    else if (mode == NOISE_PHILOX8) hipLaunchKernelGGL((adamw8bit_fast_kernel<NOISE_PHILOX8>), dim3(grid), dim3(F8_THREADS), 0, s, a, npairs);
-    else hipLaunchKernelGGL((adamw8bit_fast_kernel<NOISE_INJECT>), dim3(grid), dim3(F8_THREADS), 0, s, a, npairs);
-    return 2 * npairs;
+// Hyperparameters and codebooks of one parameter group.
+struct Adam8Group {
+    const float *qmap1, *qmap2;
+    const QuantTable *qtable;
+    int32_t block;
+    float lr, b1, b2, eps, wd, bc1, bc2;
+    int32_t mode;
+    const uint16_t *inject;
+};
+
+// Whether the fast kernel takes this tensor: standard codebooks, a block of 64 to 512, aligned
+// operands, an update divisor sqrt(v') + eps_c in [2^-60, 2^32) (sqrt(v') < 2^31 is checked per
+// chunk) and a finite step_c.
+static bool fast8_fits(const Adam8Group &g, const Adam8Consts &c, const msr_adam8_item &x) {
+    return g.qtable && g.block >= 64 && g.block <= 512 && aligned(x.p, 16) && aligned(x.g, 16) && aligned(x.state1, 8) &&
+           aligned(x.state2, 8) && c.eps_c >= 0x1p-60f && c.eps_c <= 0x1p30f && std::isfinite(c.step_c) &&
+           x.n < ((int64_t)1 << 39);
+}
+
+// The fp32 arithmetic of adam8_consts, on the host.
+static Adam8Consts host_consts(const Adam8Group &g) {
+    Adam8Consts c;
+    const float sqrt_bc2 = sqrtf(g.bc2);
+    c.one_m_b1 = 1.0f - g.b1;
+    c.one_m_b2 = 1.0f - g.b2;
+    c.step_c = (g.lr * sqrt_bc2) / g.bc1;
+    c.eps_c = sqrt_bc2 * g.eps;
+    c.decay = 1.0f - g.lr * g.wd;
+    return c;
+}
+
+template <int LB>
+static void launch_fast8_lb(int mode, const F8Args &a, unsigned grid, hipStream_t s) {
+#define F8_LAUNCH(MODE, MULTI) hipLaunchKernelGGL((adamw8bit_fast_kernel<MODE, LB, MULTI>), dim3(grid), dim3(F8_THREADS), 0, s, a)
+    if (mode == NOISE_INJECT) F8_LAUNCH(NOISE_INJECT, false);   // one tensor
+    else if (mode == NOISE_TRITON) { if (a.count > 1) F8_LAUNCH(NOISE_TRITON, true); else F8_LAUNCH(NOISE_TRITON, false); }
+    else { if (a.count > 1) F8_LAUNCH(NOISE_PHILOX8, true); else F8_LAUNCH(NOISE_PHILOX8, false); }
+#undef F8_LAUNCH
+}
+
+// One launch of the fast kernel over `count` (<= F8_MAXT) tensors that it takes, none empty.
+static int launch_fast8(const Adam8Group &g, const Adam8Consts &c, const msr_adam8_item *items, int32_t count, hipStream_t s) {
+    F8Args a;
+    a.count = count;
+    a.b1 = g.b1; a.b2 = g.b2; a.c = c;
+    a.qmap1 = g.qmap1; a.qmap2 = g.qmap2; a.qtable = g.qtable; a.inject = g.inject;
+    uint64_t chunks = 0;
+    for (int32_t i = 0; i < count; ++i) {
+        const msr_adam8_item &x = items[i];
+        a.cstart[i] = (uint32_t)chunks;
+        a.it[i] = F8Item{x.p, x.g, x.state1, x.state2, x.absmax1, x.absmax2, x.n, x.seed, 0};
+        chunks += (uint64_t)(x.n / F8_CHUNK);
+    }
+    if (chunks >= (1ull << 31)) {   // chunk numbers are 32-bit: halves
+        if (count < 2) { set_error("adamw8bit: a tensor of 2^31 chunks or more"); return MSR_ERR_ARG; }
+        const int rc = launch_fast8(g, c, items, count / 2, s);
+        return rc ? rc : launch_fast8(g, c, items + count / 2, count - count / 2, s);
+    }
+    a.cstart[count] = (uint32_t)chunks;
+    const unsigned grid = grid_for((int64_t)chunks, F8_THREADS / 64, MSR_F8_GRID_CAP);
+    switch (g.block) {
+    case 64: launch_fast8_lb<8>(g.mode, a, grid, s); break;
+    case 128: launch_fast8_lb<16>(g.mode, a, grid, s); break;
+    case 256: launch_fast8_lb<32>(g.mode, a, grid, s); break;
+    default: launch_fast8_lb<64>(g.mode, a, grid, s); break;
+    }
+    return check_launch("adamw8bit_fast_kernel");
+}
+
+// One tensor on the general kernel.
+static int launch_general8(const Adam8Group &g, const msr_adam8_item &x, hipStream_t s) {
+    Adam8Args a;
+    a.p = x.p; a.g = x.g; a.s1 = x.state1; a.s2 = x.state2; a.absmax1 = x.absmax1; a.absmax2 = x.absmax2;
+    a.qmap1 = g.qmap1; a.qmap2 = g.qmap2; a.qtable = g.qtable; a.n = x.n;
+    a.lr = g.lr; a.b1 = g.b1; a.b2 = g.b2; a.eps = g.eps; a.wd = g.wd; a.bc1 = g.bc1; a.bc2 = g.bc2;
+    a.ns_p = make_noise(x.seed, 0, g.inject, x.n);
+    const bool vec = aligned(x.p, 16) && aligned(x.g, 16) && aligned(x.state1, 8) && aligned(x.state2, 8);
+    const int64_t nblocks = (x.n + g.block - 1) / g.block;
+    switch (g.block) {
+    case 32: launch_quant<32>(g.mode, vec, a, s, nblocks); break;
+    case 64: launch_quant<64>(g.mode, vec, a, s, nblocks); break;
+    case 128: launch_quant<128>(g.mode, vec, a, s, nblocks); break;
+    case 256: launch_quant<256>(g.mode, vec, a, s, nblocks); break;
+    case 512: launch_quant<512>(g.mode, vec, a, s, nblocks); break;
+    case 1024: launch_quant<1024>(g.mode, vec, a, s, nblocks); break;
+    case 2048: launch_quant<2048>(g.mode, vec, a, s, nblocks); break;
+    default: launch_quant<4096>(g.mode, vec, a, s, nblocks); break;
+    }
+    return check_launch("adamw8bit_quant_kernel");
+}
+
+static int check_item8(const msr_adam8_item &x, int32_t block, const char *name, int32_t i) {
+    if (x.n < 0 || (x.n > 0 && (!x.p || !x.g || !x.state1 || !x.state2 || !x.absmax1 || !x.absmax2))) {
+        set_error("%s: bad arguments in item %d", name, (int)i);
+        return MSR_ERR_ARG;
+    }
+    const size_t n = (size_t)x.n, ab = 4 * ((n + block - 1) / block);
+    const void *ops[6] = {x.p, x.g, x.state1, x.state2, x.absmax1, x.absmax2};
+    const size_t len[6] = {2 * n, 2 * n, n, n, ab, ab};
+    for (int k = 0; k < 6; ++k)
+        for (int l = k + 1; l < 6; ++l)
+            if (partial_overlap(ops[k], len[k], ops[l], len[l])) {
+                set_error("%s: operands %d and %d of item %d overlap", name, k, l, (int)i);
+                return MSR_ERR_OVERLAP;
+            }
+    return MSR_OK;
+}
+
+static int check_group8(const Adam8Group &g, const char *name) {
+    if (g.block < 32 || g.block > 4096 || (g.block & (g.block - 1))) {
+        set_error("%s: block %d is not a power of two in [32, 4096]", name, (int)g.block);
+        return MSR_ERR_ARG;
+    }
+    if (!g.qmap1 || !g.qmap2) { set_error("%s: quantized state needs absmax and qmaps", name); return MSR_ERR_ARG; }
+    if (g.qtable && !aligned(g.qtable, 16)) { set_error("%s: qtable must be 16-byte aligned", name); return MSR_ERR_ALIGN; }
+    return MSR_OK;
+}
+
+static bool items_conflict(const msr_adam8_item *items, int32_t count, int32_t block) {
+    ItemRange r[6 * F8_MAXT];
+    int n = 0;
+    for (int32_t i = 0; i < count; ++i) {
+        const msr_adam8_item &x = items[i];
+        const size_t e = (size_t)x.n, ab = 4 * ((e + block - 1) / block);
+        const void *q[6] = {x.p, x.state1, x.state2, x.absmax1, x.absmax2, x.g};
+        const size_t len[6] = {2 * e, e, e, ab, ab, 2 * e};
+        for (int k = 0; k < 6; ++k) r[n++] = {(uintptr_t)q[k], (uintptr_t)q[k] + len[k], i, k < 5};
+    }
+    return ranges_conflict(r, n);
 }
 
 extern "C" {
@@ -760,52 +935,67 @@ int msr_adamw8bit_step(uint16_t *p, const uint16_t *g, void *state1, void *state
     if (quantized && (!absmax1 || !absmax2 || !qmap1 || !qmap2)) { set_error("msr_adamw8bit_step: quantized state needs absmax and qmaps"); return MSR_ERR_ARG; }
     MSR_CHECK_MODE(noise_mode, inject);
     if (n == 0) return MSR_OK;
-    {
-        const size_t sb = (quantized ? 1 : 2) * (size_t)n, ab = 4 * (size_t)((n + block - 1) / block);
-        const void *ops[6] = {p, g, state1, state2, quantized ? absmax1 : nullptr, quantized ? absmax2 : nullptr};
-        const size_t len[6] = {2 * (size_t)n, 2 * (size_t)n, sb, sb, ab, ab};
-        for (int i = 0; i < 6; ++i)
-            for (int j = i + 1; j < 6; ++j)
-                if (partial_overlap(ops[i], len[i], ops[j], len[j])) {
+    hipStream_t s = (hipStream_t)stream;
+    if (!quantized) {
+        const void *ops[4] = {p, g, state1, state2};
+        for (int i = 0; i < 4; ++i)
+            for (int j = i + 1; j < 4; ++j)
+                if (partial_overlap(ops[i], 2 * (size_t)n, ops[j], 2 * (size_t)n)) {
                     set_error("msr_adamw8bit_step: operands %d and %d overlap", i, j);
                     return MSR_ERR_OVERLAP;
                 }
-    }
-    Adam8Args a;
-    a.p = p; a.g = g; a.s1 = state1; a.s2 = state2; a.absmax1 = absmax1; a.absmax2 = absmax2;
-    a.qmap1 = qmap1; a.qmap2 = qmap2; a.n = n; a.qb0 = 0;
-    a.qtable = static_cast<const QuantTable *>(qtable);
-    if (a.qtable && !aligned(a.qtable, 16)) { set_error("msr_adamw8bit_step: qtable must be 16-byte aligned"); return MSR_ERR_ALIGN; }
-    a.lr = lr; a.b1 = beta1; a.b2 = beta2; a.eps = eps; a.wd = weight_decay; a.bc1 = bc1; a.bc2 = bc2;
-    a.ns_p = make_noise(seed, 0, inject, n);
-    hipStream_t s = (hipStream_t)stream;
-    if (quantized) {
-        const bool vec = aligned(p, 16) && aligned(g, 16) && aligned(state1, 8) && aligned(state2, 8);
-        const int64_t nblocks = (n + block - 1) / block;
-        // standard codebooks, block 256, aligned: the fast kernel takes the full block pairs
-        if (block == 256 && a.qtable && vec) a.qb0 = launch_fast8(noise_mode, a, s, n / 256);
-        if (a.qb0 == nblocks) return check_launch("msr_adamw8bit_step");
-        switch (block) {
-        case 32: launch_quant<32>(noise_mode, vec, a, s, nblocks); break;
-        case 64: launch_quant<64>(noise_mode, vec, a, s, nblocks); break;
-        case 128: launch_quant<128>(noise_mode, vec, a, s, nblocks); break;
-        case 256: launch_quant<256>(noise_mode, vec, a, s, nblocks); break;
-        case 512: launch_quant<512>(noise_mode, vec, a, s, nblocks); break;
-        case 1024: launch_quant<1024>(noise_mode, vec, a, s, nblocks); break;
-        case 2048: launch_quant<2048>(noise_mode, vec, a, s, nblocks); break;
-        default: launch_quant<4096>(noise_mode, vec, a, s, nblocks); break;
-        }
-    } else {
         const msr_adamw_item it{p, g, static_cast<uint16_t *>(state1), static_cast<uint16_t *>(state2), n, bc1, bc2, seed, 0};
         return adamw16_launch(MSR_ADAMW_8BIT16, &it, 1, lr, beta1, beta2, eps, weight_decay, noise_mode, inject, s);
     }
-    return check_launch("msr_adamw8bit_step");
+    const Adam8Group grp{qmap1, qmap2, static_cast<const QuantTable *>(qtable), block, lr, beta1, beta2, eps, weight_decay,
+                         bc1, bc2, noise_mode, inject};
+    const msr_adam8_item it{p, g, static_cast<uint8_t *>(state1), static_cast<uint8_t *>(state2), absmax1, absmax2, n, seed, 0};
+    int rc = check_group8(grp, "msr_adamw8bit_step");
+    if (!rc) rc = check_item8(it, block, "msr_adamw8bit_step", 0);
+    if (rc) return rc;
+    const Adam8Consts c = host_consts(grp);
+    return fast8_fits(grp, c, it) ? launch_fast8(grp, c, &it, 1, s) : launch_general8(grp, it, s);
+}
+
+int msr_adamw8bit_multi(const msr_adam8_item *items, int32_t count, const float *qmap1, const float *qmap2,
+                        const void *qtable, int32_t block, float lr, float beta1, float beta2, float eps,
+                        float weight_decay, float bc1, float bc2, int32_t noise_mode, msr_stream_t stream) {
+    if (count < 0 || (count > 0 && !items)) { set_error("msr_adamw8bit_multi: bad arguments"); return MSR_ERR_ARG; }
+    if (noise_mode != NOISE_TRITON && noise_mode != NOISE_PHILOX8) {
+        set_error("msr_adamw8bit_multi: noise_mode must be TRITON or PHILOX8 (got %d)", (int)noise_mode);
+        return MSR_ERR_ARG;
+    }
+    const Adam8Group grp{qmap1, qmap2, static_cast<const QuantTable *>(qtable), block, lr, beta1, beta2, eps, weight_decay,
+                         bc1, bc2, noise_mode, nullptr};
+    int rc = check_group8(grp, "msr_adamw8bit_multi");
+    for (int32_t i = 0; i < count && !rc; ++i) rc = check_item8(items[i], block, "msr_adamw8bit_multi", i);
+    if (rc) return rc;
+    const Adam8Consts c = host_consts(grp);
+    hipStream_t s = (hipStream_t)stream;
+    for (int32_t i = 0; i < count;) {
+        msr_adam8_item run[F8_MAXT], fit[F8_MAXT];
+        int32_t n = 0, nfit = 0;
+        for (; i < count && n < F8_MAXT; ++i)
+            if (items[i].n > 0) run[n++] = items[i];
+        const bool apart = n > 1 && items_conflict(run, n, block);
+        for (int32_t j = 0; j < n; ++j) {
+            if (!fast8_fits(grp, c, run[j])) {
+                if ((rc = launch_general8(grp, run[j], s))) return rc;
+            } else if (apart) {
+                if ((rc = launch_fast8(grp, c, run + j, 1, s))) return rc;
+            } else {
+                fit[nfit++] = run[j];
+            }
+        }
+        if (nfit > 0 && (rc = launch_fast8(grp, c, fit, nfit, s))) return rc;
+    }
+    return MSR_OK;
 }
 
 int msr_stream_probe8(uint16_t *p, const uint16_t *g, uint8_t *state1, uint8_t *state2, float *absmax1,
                       float *absmax2, int64_t n, int32_t grid, int32_t lds_bytes, msr_stream_t stream) {
-    if (n <= 0 || n % F8_PAIR || !p || !g || !state1 || !state2 || !absmax1 || !absmax2) {
-        set_error("msr_stream_probe8: n must be a positive multiple of %d and every pointer set", F8_PAIR);
+    if (n <= 0 || n % F8_CHUNK || !p || !g || !state1 || !state2 || !absmax1 || !absmax2) {
+        set_error("msr_stream_probe8: n must be a positive multiple of %d and every pointer set", F8_CHUNK);
         return MSR_ERR_ARG;
     }
     if (!aligned(p, 16) || !aligned(g, 16) || !aligned(state1, 8) || !aligned(state2, 8)) {
@@ -816,10 +1006,9 @@ int msr_stream_probe8(uint16_t *p, const uint16_t *g, uint8_t *state1, uint8_t *
         set_error("msr_stream_probe8: grid %d not in [1, 2^20] or lds_bytes %d not in [0, 64 KiB]", (int)grid, (int)lds_bytes);
         return MSR_ERR_ARG;
     }
-    Adam8Args a = {};
-    a.p = p; a.g = g; a.s1 = state1; a.s2 = state2; a.absmax1 = absmax1; a.absmax2 = absmax2; a.n = n;
+    const F8Item it{p, g, state1, state2, absmax1, absmax2, n, 0, 0};
     hipLaunchKernelGGL(stream8_probe_kernel, dim3((unsigned)grid), dim3(F8_THREADS), (unsigned)lds_bytes,
-                       (hipStream_t)stream, a, n / F8_PAIR);
+                       (hipStream_t)stream, it, n / F8_CHUNK);
     return check_launch("msr_stream_probe8");
 }
 

@@ -7,6 +7,7 @@
 
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include <algorithm>
 
 #include "../../include/muon_sr_amd.h"
 
@@ -425,28 +426,44 @@ __device__ __forceinline__ uint32_t pack_codes(uint32_t r0, uint32_t r1, uint32_
     return lo | hi;
 }
 
-// Maxima of two non-negative, NaN-free fp32 values over each 32-lane half of a
-// wave64 (integer order equals float order there).  Rows of 16 lanes reduce
-// with DPP (quad_perm [1,0,3,2] and [2,3,0,1], row_ror 4 and 8); then
-// v_permlane16_swap(a, b) returns rows (a0, b0, a2, b2) and (a1, b1, a3, b3), so
-// one swap and a max leave rows (A01, B01, A23, B23), and a swap of that value
-// with itself spreads A and B over both rows of their half.
+// Maxima of two non-negative, NaN-free fp32 values over each group of LB = 8, 16, 32 or 64
+// lanes of a wave64 (integer order equals float order there), in every lane of the group.  Rows
+// of 16 lanes reduce with DPP (quad_perm [1,0,3,2] and [2,3,0,1], then row_half_mirror, or
+// row_ror 4 and 8); then v_permlane16_swap(a, b) returns rows (a0, b0, a2, b2) and (a1, b1, a3,
+// b3), so one swap and a max leave rows (A01, B01, A23, B23), a v_permlane32_swap of that value
+// with itself the whole wave's (A, B, A, B), and a v_permlane16_swap with itself spreads A and B
+// over the rows.
 template <int CTRL>
 __device__ __forceinline__ uint32_t dpp_max_u32(uint32_t x) {
     return max(x, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, CTRL, 0xf, 0xf, true));
 }
 
-__device__ __forceinline__ void halfwave_max2(float &a, float &b) {
+template <int LB>
+__device__ __forceinline__ void group_max2(float &a, float &b) {
+    static_assert(LB == 8 || LB == 16 || LB == 32 || LB == 64, "lanes per group");
     uint32_t x = __float_as_uint(a), y = __float_as_uint(b);
     x = dpp_max_u32<0xB1>(x); y = dpp_max_u32<0xB1>(y);
     x = dpp_max_u32<0x4E>(x); y = dpp_max_u32<0x4E>(y);
-    x = dpp_max_u32<0x124>(x); y = dpp_max_u32<0x124>(y);
-    x = dpp_max_u32<0x128>(x); y = dpp_max_u32<0x128>(y);
-    const auto s = __builtin_amdgcn_permlane16_swap(x, y, false, false);
-    const uint32_t c = max((uint32_t)s[0], (uint32_t)s[1]);
-    const auto t = __builtin_amdgcn_permlane16_swap(c, c, false, false);
-    a = __uint_as_float(t[0]);
-    b = __uint_as_float(t[1]);
+    if constexpr (LB == 8) {
+        x = dpp_max_u32<0x141>(x); y = dpp_max_u32<0x141>(y);
+    } else {
+        x = dpp_max_u32<0x124>(x); y = dpp_max_u32<0x124>(y);
+        x = dpp_max_u32<0x128>(x); y = dpp_max_u32<0x128>(y);
+    }
+    if constexpr (LB <= 16) {
+        a = __uint_as_float(x);
+        b = __uint_as_float(y);
+    } else {
+        const auto s = __builtin_amdgcn_permlane16_swap(x, y, false, false);
+        uint32_t c = max((uint32_t)s[0], (uint32_t)s[1]);
+        if constexpr (LB == 64) {
+            const auto w = __builtin_amdgcn_permlane32_swap(c, c, false, false);
+            c = max((uint32_t)w[0], (uint32_t)w[1]);
+        }
+        const auto t = __builtin_amdgcn_permlane16_swap(c, c, false, false);
+        a = __uint_as_float(t[0]);
+        b = __uint_as_float(t[1]);
+    }
 }
 
 inline bool aligned(const void *p, uintptr_t a) { return ((uintptr_t)p & (a - 1)) == 0; }
@@ -463,6 +480,21 @@ inline bool partial_overlap(const void *a, size_t na, const void *b, size_t nb) 
     return x < y + nb && y < x + na;
 }
 
+
+// A memory range of one item of a launch, and whether some memory that one item writes is
+// touched by another (such items run in launches of their own, in order).
+struct ItemRange {
+    uintptr_t lo, hi;
+    int32_t item;
+    bool write;
+};
+inline bool ranges_conflict(ItemRange *r, int n) {
+    std::sort(r, r + n, [](const ItemRange &x, const ItemRange &y) { return x.lo < y.lo; });
+    for (int i = 0; i < n; ++i)
+        for (int j = i + 1; j < n && r[j].lo < r[i].hi; ++j)
+            if (r[i].item != r[j].item && (r[i].write || r[j].write)) return true;
+    return false;
+}
 
 // Grid size for a grid-stride loop over `work` items with `threads` per block.
 inline unsigned grid_for(int64_t work, int threads, int64_t cap = 256 * 32) {

@@ -32,7 +32,7 @@ from torch.optim import Optimizer
 
 from . import _lib
 from .adamw import _adamw_add, _AdamWBatch
-from .adamw_8bit import adamw8bit_launch, init_8bit_state, split_8bit_state, TritonAdamW8bit
+from .adamw_8bit import _Adam8Batch, init_8bit_state, split_8bit_state, TritonAdamW8bit
 
 NS_COEFFS = (3.4445, -4.7750, 2.0315)
 
@@ -593,7 +593,8 @@ class TritonMuonSRWithAuxAdam(_StackedBufsMixin, Optimizer):
                 if eight_bit:
                     TritonAdamW8bit._validate_group(group)   # as TritonAdamW8bit.step (triton_adamw_8bit.py:175)
 
-                batch = _AdamWBatch(_lib.ADAMW_8BIT16 if eight_bit else _lib.ADAMW, lr, beta1, beta2, eps, weight_decay)
+                hyper = (lr, beta1, beta2, eps, weight_decay)
+                batch = _Adam8Batch(*hyper) if eight_bit else _AdamWBatch(_lib.ADAMW, *hyper)
                 try:
                     self._step_adamw(group, group_offset, beta1, beta2, eight_bit, batch)
                 finally:
@@ -610,7 +611,7 @@ class TritonMuonSRWithAuxAdam(_StackedBufsMixin, Optimizer):
                 raise RuntimeError("TritonMuonSRWithAuxAdam does not support sparse gradients")
             state = self.state[p]
             if eight_bit:
-                self._step_8bit(p, group, state, beta1, beta2, group_offset + i, batch)
+                self._step_8bit(p, group, state, group_offset + i, batch)
                 continue
             if "format_version" in state:   # an 8-bit state in a group no longer set to optim_bits=8
                 raise ValueError("Cannot change quantization configuration after state initialization")
@@ -633,7 +634,7 @@ class TritonMuonSRWithAuxAdam(_StackedBufsMixin, Optimizer):
         super().load_state_dict(stripped)
         restore(self.state)
 
-    def _step_8bit(self, p, group, state, beta1, beta2, param_index, batch):
+    def _step_8bit(self, p, group, state, param_index, batch):
         """8-bit AdamW group step: the TritonAdamW8bit update with seed index group_offset + i."""
         _lib.require_gpu(p, "TritonMuonSRWithAuxAdam", ValueError)
         g = p.grad
@@ -651,4 +652,4 @@ class TritonMuonSRWithAuxAdam(_StackedBufsMixin, Optimizer):
             raise ValueError("Cannot change quantization configuration after state initialization")
         state["step"] += 1
         seed = (state["step"] * 2654435761 ^ param_index * 1234567891) & 0xFFFFFFFF
-        adamw8bit_launch(p.data, g, state, group["lr"], beta1, beta2, group["eps"], group["weight_decay"], seed, batch)
+        batch.add(p, g, state, seed)
