@@ -333,6 +333,29 @@ int msr_muon_fused_steps(const msr_muon_group *groups, int32_t n_groups, float b
                          int32_t noise_mode, void *workspace, size_t workspace_bytes, msr_stream_t stream);
 
 /* ---------------------------------------------------------------------------
+ * (b) The whole Muon step of matrices that are parameters of their own (momenta not stacked, a
+ * prepare seed each): one msr_muon_fused_step with batch 1, first 0 per matrix, as
+ * TritonMuonSR's per-parameter steps make it (_triton_muon_step, muon_sr/triton_muon_sr.py:88-120),
+ * with matrices of one Newton-Schulz shape sharing product launches.  Equal, bit for bit, to
+ * those calls in order; matrices that share memory which one of them writes run one by one.
+ * matrices: HOST array, any shapes.  The workspace is what msr_muon_each_workspace_bytes gives
+ * for the same list: the largest of the shared launches', bounded by them at 2^27 elements (or by
+ * one larger matrix).
+ * ------------------------------------------------------------------------- */
+typedef struct msr_muon_matrix {
+    const void *grad;              /* bf16, or fp32 with grad_f32 */
+    uint16_t *buf, *param;         /* momentum and parameter, [rows][cols] */
+    int64_t rows, cols;
+    uint32_t prepare_seed, apply_seed;
+    int32_t grad_f32;
+    float scale;                   /* sqrt(max(1, rows/cols)) */
+} msr_muon_matrix;
+int msr_muon_each_workspace_bytes(const msr_muon_matrix *matrices, int32_t count, size_t *bytes);
+int msr_muon_each(const msr_muon_matrix *matrices, int32_t count, float beta, int32_t nesterov, int32_t steps,
+                  float a, float b, float c, float lr, float weight_decay, int32_t noise_mode, void *workspace,
+                  size_t workspace_bytes, msr_stream_t stream);
+
+/* ---------------------------------------------------------------------------
  * Diagnostics (no counterpart in the reference; used by the parity tests).
  * ------------------------------------------------------------------------- */
 

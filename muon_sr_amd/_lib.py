@@ -56,6 +56,14 @@ class MuonGroup(ctypes.Structure):
                 ("rows", ctypes.c_int64), ("cols", ctypes.c_int64), ("prepare_seed", ctypes.c_uint32),
                 ("grads_f32", ctypes.c_int32), ("scale", ctypes.c_float)]
 
+
+class MuonMatrix(ctypes.Structure):
+    """msr_muon_matrix (include/muon_sr_amd.h)."""
+    _fields_ = [("grad", ctypes.c_void_p), ("buf", ctypes.c_void_p), ("param", ctypes.c_void_p),
+                ("rows", ctypes.c_int64), ("cols", ctypes.c_int64), ("prepare_seed", ctypes.c_uint32),
+                ("apply_seed", ctypes.c_uint32), ("grad_f32", ctypes.c_int32), ("scale", ctypes.c_float)]
+
+
 # name -> (restype, argtypes); mirrors include/muon_sr_amd.h
 SIGNATURES = {
     "msr_version": (ctypes.c_int, []),
@@ -80,6 +88,8 @@ SIGNATURES = {
                                            _P, _P, _P, _F, _F, _F, _I32, _P, _P, _P, ctypes.c_size_t, _P]),
     "msr_muon_fused_steps": (ctypes.c_int, [ctypes.POINTER(MuonGroup), _I32, _F, _I32, _I32, _F, _F, _F, _F, _F, _I32,
                                             _P, ctypes.c_size_t, _P]),
+    "msr_muon_each_workspace_bytes": (ctypes.c_int, [_P, _I32, _SIZE_P]),
+    "msr_muon_each": (ctypes.c_int, [_P, _I32, _F, _I32, _I32, _F, _F, _F, _F, _F, _I32, _P, ctypes.c_size_t, _P]),
     "msr_noise_fill": (ctypes.c_int, [_P, _I64, _I64, _U32, _U32, _I32, _P]),
     "msr_stream_probe8": (ctypes.c_int, [_P, _P, _P, _P, _P, _P, _I64, _I32, _I32, _P]),
     "msr_quantize": (ctypes.c_int, [_P, _P, _I64, _P, _I32, _P, _P]),

@@ -34,6 +34,8 @@
 // first slab, and its stores the next tile's first MFMAs.
 #include <algorithm>
 #include <atomic>
+#include <new>
+#include <tuple>
 #include <type_traits>
 #include <vector>
 
@@ -991,10 +993,11 @@ enum ProSrc : int { SRC_COPY = 0, SRC_PREPARE = 1 };
 struct PrologueArgs {
     const uint16_t *in;              // SRC_COPY: u, [batch][rows][cols] (matrix 0 of this launch)
     const void *grad[PRO_MAX];       // SRC_PREPARE: gradients (bf16, or fp32 with G32)
-    uint16_t *buf;                   // SRC_PREPARE: momentum of matrix 0 of this launch, [batch][rows][cols]
-    int64_t noise0;                  // SRC_PREPARE: noise offset of matrix 0 of this launch
+    uint16_t *buf[PRO_MAX];          // SRC_PREPARE: momenta
+    uint32_t seed[PRO_MAX];          // SRC_PREPARE: noise seeds
+    int64_t noise0, noise1;          // SRC_PREPARE: noise offset of matrix b of this launch: noise0 + b noise1
     float beta;
-    Noise ns;
+    const uint16_t *inject;          // SRC_PREPARE, NOISE_INJECT: indexed by the noise offset
     int64_t rows, cols;
     uint16_t *S; int64_t ldS, sS;    // X0 in the input layout (wide), or null
     uint16_t *T; int64_t ldT, sT;    // X0 = u^T (tall), or null
@@ -1023,6 +1026,12 @@ __global__ __launch_bounds__(256) void ns_prologue_kernel(PrologueArgs a) {
     const int j = threadIdx.x & 7, i0 = threadIdx.x >> 3;
     const float one_m_beta = 1.0f - a.beta;
     float s = 0.0f;
+    uint16_t *const buf = SRC == SRC_PREPARE ? a.buf[b] : nullptr;
+    Noise ns = {};
+    if constexpr (SRC == SRC_PREPARE) {
+        ns.key = seed_key((uint32_t)__builtin_amdgcn_readfirstlane((int)a.seed[b]), 0);
+        ns.inject = a.inject;
+    }
     // Both rows' loads are issued before any store: the momentum is updated in place, so
     // the compiler would not move row 1's loads above row 0's stores by itself.
     uint32_t ld0[2][4] = {}, ld1[2][4] = {};   // SRC_COPY: u; SRC_PREPARE: bf16 gradient, momentum
@@ -1042,7 +1051,7 @@ __global__ __launch_bounds__(256) void ns_prologue_kernel(PrologueArgs a) {
                     load_f32x8<VEC>(static_cast<const float *>(a.grad[b]) + offs[h], 0, valids[h], g32[h]);
                 else
                     load_bf16x8<VEC>(static_cast<const uint16_t *>(a.grad[b]) + offs[h], 0, valids[h], ld0[h]);
-                load_bf16x8<VEC>(a.buf + b * numel + offs[h], 0, valids[h], ld1[h]);
+                load_bf16x8<VEC>(buf + offs[h], 0, valids[h], ld1[h]);
             }
         }
     }
@@ -1066,15 +1075,15 @@ __global__ __launch_bounds__(256) void ns_prologue_kernel(PrologueArgs a) {
                 } else {
                     unpack8(ld0[h], gf);
                 }
-                uint16_t *bp = a.buf + b * numel + off;
+                uint16_t *bp = buf + off;
                 unpack8(ld1[h], bf);
-                const int64_t o0 = a.noise0 + b * numel + off;
+                const int64_t o0 = a.noise0 + b * a.noise1 + off;
                 uint32_t rn[8];
                 if (VEC || MODE != NOISE_PHILOX8) {
-                    noise8<MODE>(a.ns, o0, valid, rn);
+                    noise8<MODE>(ns, o0, valid, rn);
                 } else {
 #pragma unroll
-                    for (int k = 0; k < 8; ++k) rn[k] = (k < valid) ? noise1<MODE>(a.ns, o0 + k) : 0u;
+                    for (int k = 0; k < 8; ++k) rn[k] = (k < valid) ? noise1<MODE>(ns, o0 + k) : 0u;
                 }
                 float up[8];
                 uint32_t ob[8];
@@ -1520,17 +1529,21 @@ struct NSApply {
     const uint16_t *inject;
 };
 
-// The Muon momentum step that produces the update inside the prologue
-// (msr_muon_fused_step): gradients, the momentum of the call's matrix 0 and the
-// index of that matrix in its momentum stack (the noise counter's base).
+// The Muon momentum step that produces the update inside the prologue: gradients and
+// momenta of a part's matrices, either rows of one stack (msr_muon_fused_step: `buf` is matrix 0's,
+// `first` its index in the stack, the noise counter's base; one seed) or matrices of their own
+// (msr_muon_each: `bufs`, `seeds`, noise offsets from 0).
 struct NSPrepare {
     const void *const *grads;
     bool g32;
     uint16_t *buf;
     int64_t first;
+    uint32_t seed;
+    uint16_t *const *bufs;
+    const uint32_t *seeds;
     float beta;
     bool nesterov;
-    Noise ns;
+    const uint16_t *inject;   // indexed by the noise offset
     int noise_mode;
 };
 
@@ -1557,8 +1570,8 @@ static int ns_prologue_part(const NSPart &pt, uint16_t *X0, float *tpart, const 
     const NSPrepare *pp = pt.pp;
     bool vec = (cols % 8) == 0;
     if (pp) {
-        vec = vec && aligned(pp->buf, 16);
-        for (int64_t i = 0; i < pt.batch && vec; ++i) vec = aligned(pp->grads[i], 16);
+        vec = vec && (pp->bufs || aligned(pp->buf, 16));
+        for (int64_t i = 0; i < pt.batch && vec; ++i) vec = aligned(pp->grads[i], 16) && (!pp->bufs || aligned(pp->bufs[i], 16));
     } else {
         vec = vec && aligned(pt.in, 16);
     }
@@ -1580,11 +1593,15 @@ static int ns_prologue_part(const NSPart &pt, uint16_t *X0, float *tpart, const 
             if (vec) hipLaunchKernelGGL((ns_prologue_kernel<SRC_COPY, NOISE_TRITON, false, false, true>), grid, dim3(256), 0, s, a);
             else hipLaunchKernelGGL((ns_prologue_kernel<SRC_COPY, NOISE_TRITON, false, false, false>), grid, dim3(256), 0, s, a);
         } else {
-            for (int64_t i = 0; i < nb; ++i) a.grad[i] = pp->grads[b0 + i];
-            a.buf = pp->buf + b0 * numel;
-            a.noise0 = (pp->first + b0) * numel;
+            for (int64_t i = 0; i < nb; ++i) {
+                a.grad[i] = pp->grads[b0 + i];
+                a.buf[i] = pp->bufs ? pp->bufs[b0 + i] : pp->buf + (b0 + i) * numel;
+                a.seed[i] = pp->bufs ? pp->seeds[b0 + i] : pp->seed;
+            }
+            a.noise0 = pp->bufs ? 0 : (pp->first + b0) * numel;
+            a.noise1 = pp->bufs ? 0 : numel;
             a.beta = pp->beta;
-            a.ns = pp->ns;
+            a.inject = pp->inject;
 #define PRO_LAUNCH(NEST, G, V) MSR_DISPATCH_NOISE(pp->noise_mode, M, hipLaunchKernelGGL((ns_prologue_kernel<SRC_PREPARE, M, NEST, G, V>), grid, dim3(256), 0, s, a))
             if (pp->g32) {
                 if (pp->nesterov) { if (vec) { PRO_LAUNCH(true, true, true); } else { PRO_LAUNCH(true, true, false); } }
@@ -1970,10 +1987,9 @@ int msr_muon_fused_step(const void *const *grads, int32_t grads_f32, uint16_t *b
             }
         }
     }
-    Noise pns;
-    pns.key = seed_key(prepare_seed, 0);
-    pns.inject = inject_prepare;   // indexed by the element offset in the momentum stack
-    NSPrepare pp{grads, grads_f32 != 0, buf, first, beta, nesterov != 0, pns, (int)noise_mode};
+    // inject_prepare is indexed by the element offset in the momentum stack
+    NSPrepare pp{grads, grads_f32 != 0, buf, first, prepare_seed, nullptr, nullptr, beta, nesterov != 0, inject_prepare,
+                 (int)noise_mode};
     if (!params)
         return ns_run(nullptr, out, batch, rows, cols, steps, a_coef, b_coef, c_coef, workspace, L, (hipStream_t)stream,
                       nullptr, &pp);
@@ -2078,10 +2094,8 @@ int msr_muon_fused_steps(const msr_muon_group *groups, int32_t n_groups, float b
     int64_t b0 = 0;
     for (int32_t i = 0; i < n_groups; ++i) {
         const msr_muon_group &g = groups[i];
-        Noise pns;
-        pns.key = seed_key(g.prepare_seed, 0);
-        pns.inject = nullptr;
-        pps[i] = NSPrepare{g.grads, g.grads_f32 != 0, g.buf, g.first, beta, nesterov != 0, pns, (int)noise_mode};
+        pps[i] = NSPrepare{g.grads, g.grads_f32 != 0, g.buf, g.first, g.prepare_seed, nullptr, nullptr, beta, nesterov != 0,
+                           nullptr, (int)noise_mode};
         aps[i] = NSApply{g.params, g.apply_seeds, lr, weight_decay, g.scale, (int)noise_mode, nullptr};
         // the last product's store writes params[b]: `out` only marks the output layout (never accessed)
         parts[i] = NSPart{b0, g.batch, g.rows, g.cols, nullptr, static_cast<uint16_t *>(workspace), &aps[i], &pps[i]};
@@ -2089,6 +2103,154 @@ int msr_muon_fused_steps(const msr_muon_group *groups, int32_t n_groups, float b
     }
     return ns_run_parts(parts.data(), (int)n_groups, total, steps, a_coef, b_coef, c_coef, workspace, L,
                         (hipStream_t)stream);
+}
+
+}  // extern "C"
+
+// ---------------------------------------------------------------------------
+// Matrices of their own (msr_muon_each)
+// ---------------------------------------------------------------------------
+
+// Elements of the matrices that share a call's product launches: enough for 2048 x 2048 ones to
+// fill the chip many times over (32), while a 4096 x 14336 one, which fills it by itself, is
+// nearly alone; it bounds the workspace at about 1 GiB.
+constexpr int64_t EACH_NUMEL = int64_t(1) << 27;
+
+// The calls of a list of matrices: indices, grouped by Newton-Schulz shape (a tall matrix has the
+// shape of its transpose) and cut evenly into runs of at most EACH_NUMEL elements; inside a run
+// the matrices of one layout and gradient type are next to each other.
+static std::vector<std::vector<int32_t>> each_runs(const msr_muon_matrix *x, int32_t count) {
+    std::vector<int32_t> order((size_t)count);
+    for (int32_t i = 0; i < count; ++i) order[i] = i;
+    auto key = [&](int32_t i) {
+        return std::make_tuple(std::min(x[i].rows, x[i].cols), std::max(x[i].rows, x[i].cols), x[i].rows > x[i].cols, x[i].grad_f32 != 0);
+    };
+    std::stable_sort(order.begin(), order.end(), [&](int32_t a, int32_t b) { return key(a) < key(b); });
+    std::vector<std::vector<int32_t>> runs;
+    for (size_t i = 0; i < order.size();) {
+        size_t e = i;
+        auto shape = [&](int32_t k) { return std::make_pair(std::min(x[k].rows, x[k].cols), std::max(x[k].rows, x[k].cols)); };
+        while (e < order.size() && shape(order[e]) == shape(order[i])) ++e;
+        const int64_t numel = x[order[i]].rows * x[order[i]].cols, n = (int64_t)(e - i);
+        const int64_t most = std::max<int64_t>(1, EACH_NUMEL / numel), pieces = (n + most - 1) / most;
+        for (int64_t k = 0; k < pieces; ++k)
+            runs.emplace_back(order.begin() + i + n * k / pieces, order.begin() + i + n * (k + 1) / pieces);
+        i = e;
+    }
+    return runs;
+}
+
+static int each_check(const msr_muon_matrix *x, int32_t count, const char *name) {
+    if (count < 0 || (count > 0 && !x)) { set_error("%s: bad arguments", name); return MSR_ERR_ARG; }
+    for (int32_t i = 0; i < count; ++i) {
+        if (!x[i].grad || !x[i].buf || !x[i].param || x[i].rows <= 0 || x[i].cols <= 0 || x[i].rows > (1 << 30) || x[i].cols > (1 << 30)) {
+            set_error("%s: bad arguments in matrix %d", name, (int)i);
+            return MSR_ERR_ARG;
+        }
+    }
+    return MSR_OK;
+}
+
+static int each_run(const msr_muon_matrix *x, const std::vector<int32_t> &run, float beta, bool nesterov, int32_t steps,
+                    float a, float b, float c, float lr, float wd, int32_t mode, void *ws, size_t ws_bytes, hipStream_t s) {
+    const int64_t n = (int64_t)run.size();
+    const msr_muon_matrix &x0 = x[run[0]];
+    const NSLayout L = ns_layout(n, std::min(x0.rows, x0.cols), std::max(x0.rows, x0.cols));
+    if (!ws || ws_bytes < L.total) {
+        set_error("msr_muon_each: workspace of %zu bytes is smaller than the %zu required", ws_bytes, L.total);
+        return MSR_ERR_WORKSPACE;
+    }
+    std::vector<const void *> grads((size_t)n);
+    std::vector<uint16_t *> bufs((size_t)n), params((size_t)n);
+    std::vector<uint32_t> pseeds((size_t)n), aseeds((size_t)n);
+    for (int64_t i = 0; i < n; ++i) {
+        const msr_muon_matrix &m = x[run[i]];
+        grads[i] = m.grad; bufs[i] = m.buf; params[i] = m.param;
+        pseeds[i] = m.prepare_seed; aseeds[i] = m.apply_seed;
+    }
+    NSPrepare pps[4];
+    NSApply aps[4];
+    NSPart parts[4];   // wide and tall, bf16 and fp32 gradients
+    int np = 0;
+    for (int64_t i = 0; i < n;) {
+        const msr_muon_matrix &m = x[run[i]];
+        int64_t e = i;
+        while (e < n && x[run[e]].rows == m.rows && (x[run[e]].grad_f32 != 0) == (m.grad_f32 != 0)) ++e;
+        pps[np] = NSPrepare{&grads[i], m.grad_f32 != 0, nullptr, 0, 0u, &bufs[i], &pseeds[i], beta, nesterov, nullptr, (int)mode};
+        aps[np] = NSApply{&params[i], &aseeds[i], lr, wd, m.scale, (int)mode, nullptr};
+        // the last product's store writes the parameters: `out` only marks the layout (never accessed)
+        parts[np] = NSPart{i, e - i, m.rows, m.cols, nullptr, static_cast<uint16_t *>(ws), &aps[np], &pps[np]};
+        ++np;
+        i = e;
+    }
+    return ns_run_parts(parts, np, n, steps, a, b, c, ws, L, s);
+}
+
+extern "C" {
+
+int msr_muon_each_workspace_bytes(const msr_muon_matrix *matrices, int32_t count, size_t *bytes) {
+    const int rc = each_check(matrices, count, "msr_muon_each_workspace_bytes");
+    if (rc) return rc;
+    if (!bytes) { set_error("msr_muon_each_workspace_bytes: bad arguments"); return MSR_ERR_ARG; }
+    size_t most = 0;
+    try {
+        for (const auto &r : each_runs(matrices, count))
+            most = std::max(most, ns_layout((int64_t)r.size(), matrices[r[0]].rows, matrices[r[0]].cols).total);
+    } catch (const std::bad_alloc &) {
+        set_error("msr_muon_each_workspace_bytes: out of host memory");
+        return MSR_ERR_ARG;
+    }
+    *bytes = most;
+    return MSR_OK;
+}
+
+int msr_muon_each(const msr_muon_matrix *matrices, int32_t count, float beta, int32_t nesterov, int32_t steps, float a_coef,
+                  float b_coef, float c_coef, float lr, float weight_decay, int32_t noise_mode, void *workspace,
+                  size_t workspace_bytes, msr_stream_t stream) {
+    int rc = each_check(matrices, count, "msr_muon_each");
+    if (rc) return rc;
+    if (steps < 1 || (noise_mode != NOISE_TRITON && noise_mode != NOISE_PHILOX8)) {
+        set_error("msr_muon_each: bad arguments (steps must be >= 1, noise_mode TRITON or PHILOX8)");
+        return MSR_ERR_ARG;
+    }
+    if (count == 0) return MSR_OK;
+    hipStream_t s = (hipStream_t)stream;
+    try {
+        // a matrix's own operands and the workspace must not overlap; matrices that share
+        // memory which one of them writes run one after the other, in order
+        std::vector<ItemRange> r;
+        r.reserve(3 * (size_t)count);
+        for (int32_t i = 0; i < count; ++i) {
+            const msr_muon_matrix &m = matrices[i];
+            const size_t e = (size_t)m.rows * (size_t)m.cols;
+            const void *q[3] = {m.param, m.buf, m.grad};
+            const size_t len[3] = {2 * e, 2 * e, (m.grad_f32 ? 4 : 2) * e};
+            for (int k = 0; k < 3; ++k) {
+                const uintptr_t lo = (uintptr_t)q[k], hi = lo + len[k], w = (uintptr_t)workspace;
+                bool race = lo < w + workspace_bytes && w < hi;
+                for (int l = 0; l < k; ++l) race = race || (lo < (uintptr_t)q[l] + len[l] && (uintptr_t)q[l] < hi);
+                if (race) {
+                    set_error("msr_muon_each: operands of matrix %d overlap each other or the workspace", (int)i);
+                    return MSR_ERR_OVERLAP;
+                }
+                r.push_back({lo, hi, i, k < 2});
+            }
+        }
+        std::vector<std::vector<int32_t>> runs;
+        if (ranges_conflict(r.data(), (int)r.size())) {
+            for (int32_t i = 0; i < count; ++i) runs.push_back({i});
+        } else {
+            runs = each_runs(matrices, count);
+        }
+        for (const auto &run : runs)
+            if ((rc = each_run(matrices, run, beta, nesterov != 0, steps, a_coef, b_coef, c_coef, lr, weight_decay, noise_mode,
+                               workspace, workspace_bytes, s)))
+                return rc;
+    } catch (const std::bad_alloc &) {
+        set_error("msr_muon_each: out of host memory");
+        return MSR_ERR_ARG;
+    }
+    return MSR_OK;
 }
 
 }  // extern "C"

@@ -7,7 +7,7 @@ constructor signatures, param-group keys, state keys (``step``,
 shape-group order and checkpoint behaviour.
 
 One Muon step of a chunk of 2-D matrices of one shape is one library call
-(msr_muon_fused_step):
+(msr_muon_fused_step; msr_muon_each for a list of matrices whose momenta are not stacked):
   prologue  momentum lerp + nesterov, SR store of the momentum stack, RNE bf16
             update written straight into Newton-Schulz's first iterate with its
             sum of squares (grads read through a pointer table: no stack copy,
@@ -25,6 +25,7 @@ with ``optim_bits=8`` runs the blockwise 8-bit AdamW of TritonAdamW8bit
 """
 from __future__ import annotations
 
+import struct
 from collections import defaultdict
 
 import torch
@@ -293,17 +294,76 @@ def _check_param(p, name):
         raise RuntimeError(f"{name} requires contiguous parameters")
 
 
-def _muon_step(p, grad, buf, beta, nesterov, ns_steps, lr, weight_decay, step, param_idx):
-    """Single-param Muon step (muon_sr/triton_muon_sr.py:116-120)."""
-    grad = _grad_operand(grad)
-    if p.dim() == 2 and ns_steps >= 1:
-        _fused_step([grad], buf, 0, [p.data], beta, nesterov, _deterministic_seed(step, param_idx, salt=0), ns_steps,
-                    lr, weight_decay, _ns_scale(p.shape), [_deterministic_seed(step, param_idx, salt=1)])
-        return
-    update = torch.empty(p.shape, dtype=torch.bfloat16, device=p.device)
-    _run_prepare([grad], buf, update, beta, nesterov, _deterministic_seed(step, param_idx, salt=0))
-    _ns_apply(update.unsqueeze(0), [p.data], lr, weight_decay, _ns_scale(p.shape),
-              [_deterministic_seed(step, param_idx, salt=1)], ns_steps)
+class _MuonEach:
+    """The Muon steps of parameters whose momenta are not stacked, or whose shape group misses a
+    gradient: matrices of one Newton-Schulz shape share product launches (msr_muon_each), with
+    the seeds, noise offsets and results of one step per parameter
+    (_triton_muon_step, muon_sr/triton_muon_sr.py:116-120).
+
+    A caller adds in a ``try`` and flushes in its ``finally``, so that an error at one parameter
+    leaves the earlier ones stepped, as one step per parameter would."""
+
+    _PACK = struct.Struct("=QQQqqIIif").pack   # msr_muon_matrix
+    MAX_KEPT_BYTES = 256 << 20   # gradient copies (made contiguous or fp32) held until their launch
+
+    def __init__(self, beta, nesterov, ns_steps, lr, weight_decay):
+        self.beta, self.nesterov, self.ns_steps, self.lr, self.weight_decay = beta, nesterov, ns_steps, lr, weight_decay
+        self.items, self.kept, self.kept_bytes, self.device, self.stream = [], [], 0, None, None
+
+    def add(self, p, buf, step, param_idx):
+        grad = _grad_operand(p.grad)
+        seeds = [_deterministic_seed(step, param_idx, salt=salt) for salt in (0, 1)]
+        if p.dim() != 2 or self.ns_steps < 1 or not p.numel():
+            self._alone(p, grad, buf, *seeds)
+            return
+        device, stream = p.device, _lib.stream_of(p)
+        if self.items and (device != self.device or stream != self.stream):
+            self.flush()
+        self.device, self.stream = device, stream
+        self.items.append(self._PACK(grad.data_ptr(), buf.data_ptr(), p.data_ptr(), *p.shape, *seeds,
+                                     grad.dtype == torch.float32, _ns_scale(p.shape)))
+        if grad is not p.grad:
+            self.kept.append(grad)
+            self.kept_bytes += grad.numel() * grad.element_size()
+            if self.kept_bytes >= self.MAX_KEPT_BYTES:
+                self.flush()
+
+    def _alone(self, p, grad, buf, prepare_seed, apply_seed):
+        """Parameters of more than 2 dims, and ns_steps = 0."""
+        self.flush()   # parameters may share memory: keep the order
+        if p.dim() == 2 and self.ns_steps >= 1:   # an empty matrix, which the library refuses
+            _fused_step([grad], buf, 0, [p.data], self.beta, self.nesterov, prepare_seed, self.ns_steps, self.lr,
+                        self.weight_decay, 1.0, [apply_seed])
+            return
+        update = torch.empty(p.shape, dtype=torch.bfloat16, device=p.device)
+        _run_prepare([grad], buf, update, self.beta, self.nesterov, prepare_seed)
+        _ns_apply(update.unsqueeze(0), [p.data], self.lr, self.weight_decay, _ns_scale(p.shape), [apply_seed], self.ns_steps)
+
+    def _launch(self, items):
+        L = _lib.lib()
+        arr, n = b"".join(items), len(items)
+        nbytes = _lib.ctypes.c_size_t(0)
+        _lib.check(L.msr_muon_each_workspace_bytes(arr, n, _lib.ctypes.byref(nbytes)), "msr_muon_each_workspace_bytes")
+        try:
+            ws = torch.empty(nbytes.value, dtype=torch.uint8, device=self.device)
+        except torch.OutOfMemoryError:
+            if n == 1:
+                raise
+            for item in items:   # one by one, each with its own smaller workspace
+                self._launch([item])
+            return
+        rc = L.msr_muon_each(arr, n, self.beta, int(bool(self.nesterov)), self.ns_steps, *NS_COEFFS, self.lr,
+                             self.weight_decay, _lib.noise_mode(), ws.data_ptr(), nbytes.value, self.stream)
+        _lib.check(rc, "msr_muon_each")
+
+    def flush(self):
+        if not self.items:
+            return
+        items, self.items = self.items, []
+        try:
+            self._launch(items)
+        finally:
+            self.kept, self.kept_bytes = [], 0
 
 
 def _muon_batch_step(shape_groups, stacked_bufs, buf_indices, beta, nesterov, ns_steps, lr, weight_decay, step):
@@ -320,6 +380,7 @@ def _muon_batch_step(shape_groups, stacked_bufs, buf_indices, beta, nesterov, ns
     items = list(shape_groups.items())
     partners = _transposed_partners(items, ns_steps)
     calls = []   # the fused library calls of whole groups, run at the end by _run_calls
+    each = _MuonEach(beta, nesterov, ns_steps, lr, weight_decay)   # parameters of groups with missing gradients
 
     def whole_group(idx):   # the one chunk of a whole group, as the loop below makes it
         shape, grp = items[idx]
@@ -369,11 +430,13 @@ def _muon_batch_step(shape_groups, stacked_bufs, buf_indices, beta, nesterov, ns
                 _ns_apply(work[start:start + k], [p.data for p in chunk], lr, weight_decay, scale, seeds, ns_steps)
             del work
         else:
-            for p in active:
-                _check_param(p, "TritonMuonSR")
-                idx = buf_indices[id(p)]
-                _muon_step(p, p.grad, stacked_buf[idx], beta, nesterov, ns_steps, lr, weight_decay, step,
-                           shape_idx * 10000 + idx)
+            try:
+                for p in active:
+                    _check_param(p, "TritonMuonSR")
+                    idx = buf_indices[id(p)]
+                    each.add(p, stacked_buf[idx], step, shape_idx * 10000 + idx)
+            finally:
+                each.flush()
     by_device = {}
     for c in calls:
         by_device.setdefault(c[1][0].device, []).append(c)
@@ -403,6 +466,23 @@ def _init_stacked_bufs(params, device, state):
             p_state["momentum_buffer"] = stacked[i]
         stacked_bufs[shape] = stacked
     return dict(shape_groups), stacked_bufs, buf_indices
+
+
+def _muon_each_step(params, states, each, name):
+    """The parameters of a group without batch_ns, in order (muon_sr/triton_muon_sr.py:235-253)."""
+    for param_idx, p in enumerate(params):
+        assert p.dtype == torch.bfloat16, "only bfloat16 is supported."
+        if p.grad is None:
+            continue
+        if p.grad.is_sparse:
+            raise RuntimeError(f"{name} does not support sparse gradients")
+        _check_param(p, name)
+        state = states[p]
+        if len(state) == 0:
+            state["step"] = 0
+            state["momentum_buffer"] = torch.zeros_like(p, dtype=torch.bfloat16, memory_format=torch.contiguous_format)
+        state["step"] += 1
+        each.add(p, state["momentum_buffer"], state["step"], param_idx)
 
 
 class _StackedBufsMixin:
@@ -473,21 +553,11 @@ class TritonMuonSR(_StackedBufsMixin, Optimizer):
                 _muon_batch_step(shape_groups, stacked_bufs, buf_indices, beta, nesterov, ns_steps, lr,
                                  weight_decay, self._global_step)
             else:
-                for param_idx, p in enumerate(group["params"]):
-                    assert p.dtype == torch.bfloat16, "only bfloat16 is supported."
-                    if p.grad is None:
-                        continue
-                    if p.grad.is_sparse:
-                        raise RuntimeError("TritonMuonSR does not support sparse gradients")
-                    _check_param(p, "TritonMuonSR")
-                    state = self.state[p]
-                    if len(state) == 0:
-                        state["step"] = 0
-                        state["momentum_buffer"] = torch.zeros_like(p, dtype=torch.bfloat16,
-                                                                    memory_format=torch.contiguous_format)
-                    state["step"] += 1
-                    _muon_step(p, p.grad, state["momentum_buffer"], beta, nesterov, ns_steps, lr, weight_decay,
-                               state["step"], param_idx)
+                each = _MuonEach(beta, nesterov, ns_steps, lr, weight_decay)
+                try:
+                    _muon_each_step(group["params"], self.state, each, "TritonMuonSR")
+                finally:
+                    each.flush()
 
         return loss
 
@@ -569,21 +639,11 @@ class TritonMuonSRWithAuxAdam(_StackedBufsMixin, Optimizer):
                         _muon_batch_step(shape_groups, stacked_bufs, buf_indices, beta, nesterov, ns_steps, lr,
                                          weight_decay, self._global_step)
                     else:
-                        for param_idx, p in enumerate(group["params"]):
-                            assert p.dtype == torch.bfloat16, "only bfloat16 is supported."
-                            if p.grad is None:
-                                continue
-                            if p.grad.is_sparse:
-                                raise RuntimeError("TritonMuonSRWithAuxAdam does not support sparse gradients")
-                            _check_param(p, "TritonMuonSRWithAuxAdam")
-                            state = self.state[p]
-                            if len(state) == 0:
-                                state["step"] = 0
-                                state["momentum_buffer"] = torch.zeros_like(p, dtype=torch.bfloat16,
-                                                                            memory_format=torch.contiguous_format)
-                            state["step"] += 1
-                            _muon_step(p, p.grad, state["momentum_buffer"], beta, nesterov, ns_steps, lr,
-                                       weight_decay, state["step"], param_idx)
+                        each = _MuonEach(beta, nesterov, ns_steps, lr, weight_decay)
+                        try:
+                            _muon_each_step(group["params"], self.state, each, "TritonMuonSRWithAuxAdam")
+                        finally:
+                            each.flush()
             else:
                 lr = group["lr"]
                 beta1, beta2 = group["betas"]
