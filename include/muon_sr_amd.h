@@ -108,8 +108,11 @@ int msr_adamw_bf16_step(uint16_t *p, const uint16_t *g, uint16_t *ema, uint16_t 
  * internally); equal, bit for bit, to one call per item in order.  form MSR_ADAMW: each item as
  * msr_adamw_bf16_step (m, v: ema, ema_sq; bc1, bc2: bias_correction, bias_correction_sqrt).
  * form MSR_ADAMW_8BIT16: each item as msr_adamw8bit_step with quantized = 0 (m, v: the bf16
- * states; bc1, bc2 as there).  items: HOST array.  noise_mode: MSR_NOISE_TRITON or
- * MSR_NOISE_PHILOX8. */
+ * states; bc1, bc2 as there).  form MSR_ADAMW_CENTRALIZED: as MSR_ADAMW on the gradient that
+ * msr_centralize_bf16(rows of item.cols elements, strength) gives, without writing it; tensors
+ * 16-byte aligned, cols a multiple of 8 and at most MSR_ADAMW_CENTRAL_MAX_COLS (else
+ * MSR_ERR_ARG: centralize first).  strength is unused in the other forms.  items: HOST array.
+ * noise_mode: MSR_NOISE_TRITON or MSR_NOISE_PHILOX8. */
 typedef struct msr_adamw_item {
     uint16_t *p;
     const uint16_t *g;
@@ -117,12 +120,15 @@ typedef struct msr_adamw_item {
     int64_t n;
     float bc1, bc2;
     uint32_t seed;
-    int32_t reserved;   /* 0 */
+    int32_t cols;       /* MSR_ADAMW_CENTRALIZED: elements of a row; else unused */
 } msr_adamw_item;
 #define MSR_ADAMW 0
 #define MSR_ADAMW_8BIT16 1
-int msr_adamw_multi(const msr_adamw_item *items, int32_t count, int32_t form, float lr, float beta1,
-                    float beta2, float eps, float weight_decay, int32_t noise_mode, msr_stream_t stream);
+#define MSR_ADAMW_CENTRALIZED 2
+#define MSR_ADAMW_CENTRAL_MAX_COLS 4096
+int msr_adamw_multi(const msr_adamw_item *items, int32_t count, int32_t form, float strength, float lr,
+                    float beta1, float beta2, float eps, float weight_decay, int32_t noise_mode,
+                    msr_stream_t stream);
 
 /* ---------------------------------------------------------------------------
  * Gradient centralization of TritonAdamW, on the device.

@@ -33,7 +33,7 @@ class AdamWItem(ctypes.Structure):
     """msr_adamw_item (include/muon_sr_amd.h)."""
     _fields_ = [("p", ctypes.c_void_p), ("g", ctypes.c_void_p), ("m", ctypes.c_void_p), ("v", ctypes.c_void_p),
                 ("n", ctypes.c_int64), ("bc1", ctypes.c_float), ("bc2", ctypes.c_float), ("seed", ctypes.c_uint32),
-                ("reserved", ctypes.c_int32)]
+                ("cols", ctypes.c_int32)]
 
 
 class Adam8Item(ctypes.Structure):
@@ -45,6 +45,8 @@ class Adam8Item(ctypes.Structure):
 
 ADAMW = 0
 ADAMW_8BIT16 = 1
+ADAMW_CENTRALIZED = 2
+ADAMW_CENTRAL_MAX_COLS = 4096
 ACCUM_ZERO_INIT = 1
 ACCUM_GRAD_F32 = 2
 
@@ -71,7 +73,7 @@ SIGNATURES = {
     "msr_sr_accum": (ctypes.c_int, [_P, _P, _I32, _I64, _U32, _I32, _I32, _P, _P]),
     "msr_sr_accum_multi": (ctypes.c_int, [ctypes.POINTER(AccumItem), _I32, _I32, _P]),
     "msr_adamw_bf16_step": (ctypes.c_int, [_P, _P, _P, _P, _I64, _F, _F, _F, _F, _F, _F, _F, _U32, _I32, _P, _P]),
-    "msr_adamw_multi": (ctypes.c_int, [_P, _I32, _I32, _F, _F, _F, _F, _F, _I32, _P]),
+    "msr_adamw_multi": (ctypes.c_int, [_P, _I32, _I32, _F, _F, _F, _F, _F, _F, _I32, _P]),
     "msr_centralize_workspace_bytes": (ctypes.c_int, [_I64, _I64, _SIZE_P]),
     "msr_centralize_bf16": (ctypes.c_int, [_P, _P, _I64, _I64, _F, _P, ctypes.c_size_t, _P]),
     "msr_centralize_bf16_noalloc": (ctypes.c_int, [_P, _P, _I64, _I64, _F, _P]),

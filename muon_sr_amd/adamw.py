@@ -35,17 +35,18 @@ class _AdamWBatch:
     _PACK = struct.Struct("=QQQQqffIi").pack   # msr_adamw_item
     MAX_KEPT_BYTES = 256 << 20   # gradient copies (made contiguous, or centred) held until their launch
 
-    def __init__(self, form, lr, beta1, beta2, eps, weight_decay):
-        self.form, self.hyper = form, (lr, beta1, beta2, eps, weight_decay)
+    def __init__(self, form, lr, beta1, beta2, eps, weight_decay, centralization=0.0):
+        self.form, self.centralization, self.hyper = form, centralization, (lr, beta1, beta2, eps, weight_decay)
         self.items, self.kept, self.kept_bytes, self.stream, self.device = [], [], 0, None, None
 
-    def add(self, p, g, m, v, bc1, bc2, seed, copied=False):
-        """One tensor's step; ``copied``: nothing but the batch holds ``g``."""
+    def add(self, p, g, m, v, bc1, bc2, seed, copied=False, cols=0):
+        """One tensor's step; ``copied``: nothing but the batch holds ``g``; ``cols``: elements of a
+        row, with form ADAMW_CENTRALIZED."""
         device, stream = p.get_device(), _lib.stream_of(p)
         if self.items and (device != self.device or stream != self.stream):
             self.flush()
         self.device, self.stream = device, stream
-        self.items.append(self._PACK(p.data_ptr(), g.data_ptr(), m.data_ptr(), v.data_ptr(), p.numel(), bc1, bc2, seed, 0))
+        self.items.append(self._PACK(p.data_ptr(), g.data_ptr(), m.data_ptr(), v.data_ptr(), p.numel(), bc1, bc2, seed, cols))
         if copied:
             self.kept.append(g)
             self.kept_bytes += g.numel() * g.element_size()
@@ -56,12 +57,13 @@ class _AdamWBatch:
         if not self.items:
             return
         items, self.items = self.items, []
-        rc = _lib.lib().msr_adamw_multi(b"".join(items), len(items), self.form, *self.hyper, _lib.noise_mode(), self.stream)
+        rc = _lib.lib().msr_adamw_multi(b"".join(items), len(items), self.form, self.centralization, *self.hyper,
+                                        _lib.noise_mode(), self.stream)
         self.kept, self.kept_bytes = [], 0
         _lib.check(rc, "msr_adamw_multi")
 
 
-def _adamw_add(batch, p, g, ema, ema_sq, beta1, beta2, step, param_idx, copied=False):
+def _adamw_add(batch, p, g, ema, ema_sq, beta1, beta2, step, param_idx, copied=False, cols=0):
     """Adds the AdamW step of one tensor (muon_sr/triton_adamw.py:75-114).
 
     Bias corrections are Python doubles, passed to the kernel as fp32 (as a
@@ -72,7 +74,20 @@ def _adamw_add(batch, p, g, ema, ema_sq, beta1, beta2, step, param_idx, copied=F
         raise RuntimeError("TritonAdamW requires contiguous parameters")
     if not g.is_contiguous():
         g, copied = g.contiguous(), True
-    batch.add(p, g, ema, ema_sq, 1.0 - beta1 ** step, (1.0 - beta2 ** step) ** 0.5, _seed(step, param_idx), copied)
+    batch.add(p, g, ema, ema_sq, 1.0 - beta1 ** step, (1.0 - beta2 ** step) ** 0.5, _seed(step, param_idx), copied, cols)
+
+
+def _fused_central_cols(p, g, ema, ema_sq):
+    """Elements of a row of ``g`` (centralize's rows) where the centred step can run in one kernel
+    (msr_adamw_multi, form MSR_ADAMW_CENTRALIZED); 0 where the gradient is centred first."""
+    if g.dtype != torch.bfloat16 or not g.is_contiguous() or not p.is_contiguous() or not g.numel():
+        return 0
+    cols = g.numel() // g.shape[0] if g.dim() >= 2 else g.numel()
+    if cols % 8 or cols > _lib.ADAMW_CENTRAL_MAX_COLS or g.numel() != p.numel():
+        return 0
+    if (p.data_ptr() | g.data_ptr() | ema.data_ptr() | ema_sq.data_ptr()) % 16:
+        return 0
+    return cols
 
 
 def centralize(grad: torch.Tensor, strength: float) -> torch.Tensor:
@@ -129,14 +144,16 @@ class TritonAdamW(Optimizer):
             weight_decay = group["weight_decay"]
             centralization = group["centralization"]
             batch = _AdamWBatch(_lib.ADAMW, lr, beta1, beta2, eps, weight_decay)
+            central = _AdamWBatch(_lib.ADAMW_CENTRALIZED, lr, beta1, beta2, eps, weight_decay, centralization)
             try:
-                self._step_group(group, group_offset, beta1, beta2, centralization, batch)
+                self._step_group(group, group_offset, beta1, beta2, centralization, batch, central)
             finally:
+                central.flush()
                 batch.flush()
 
         return loss
 
-    def _step_group(self, group, group_offset, beta1, beta2, centralization, batch):
+    def _step_group(self, group, group_offset, beta1, beta2, centralization, batch, central):
         for i, p in enumerate(group["params"]):
             assert p.dtype == torch.bfloat16, "only bfloat16 is supported."
             grad = p.grad
@@ -153,10 +170,17 @@ class TritonAdamW(Optimizer):
 
             state["step"] += 1
 
-            # gradient centralization (muon_sr/triton_adamw.py:179-187): one fused
-            # device pass instead of the reference's five torch ops
+            # gradient centralization (muon_sr/triton_adamw.py:179-187): in the step itself, or
+            # one device pass before it, where the reference runs five torch ops
             if centralization != 0:
                 _lib.require_gpu(p, "TritonAdamW", RuntimeError)
+                cols = _fused_central_cols(p, grad, state["ema"], state["ema_squared"])
+                if cols:
+                    batch.flush()   # parameters may share memory: the two batches keep their order
+                    _adamw_add(central, p, grad, state["ema"], state["ema_squared"], beta1, beta2, state["step"],
+                               group_offset + i, cols=cols)
+                    continue
+                central.flush()
                 grad = centralize(grad, centralization)
 
             _adamw_add(batch, p, grad, state["ema"], state["ema_squared"], beta1, beta2, state["step"],

@@ -25,7 +25,7 @@ int check_launch(const char *what);
 
 // One launch of the bf16-moment AdamW steps (adamw16.hip): at most 56 items, none empty.
 int adamw16_launch(int form, const msr_adamw_item *items, int32_t count, float lr, float b1, float b2, float eps, float wd,
-                   int32_t mode, const uint16_t *inject, hipStream_t s);
+                   int32_t mode, const uint16_t *inject, hipStream_t s, bool central = false, float strength = 0.0f);
 
 // ---------------------------------------------------------------------------
 // bf16 helpers
