@@ -1205,7 +1205,7 @@ static inline int64_t round_up(int64_t x, int64_t m) { return (x + m - 1) / m * 
 
 struct NSLayout {
     int64_t m, n, mp, np;
-    int tile;         // 256 (ns_gemm.hip), or 64 / 128 (tile_gemm.hip); mp and np are multiples of it
+    int tile;         // mp and np are multiples of it: 256 (this file's kernel), or 64 / 128 (tile_gemm.hip)
     bool transposed;
     size_t off_x[2], off_a, off_b, off_part, off_alpha, off_rho, off_r, off_tpart, off_rexp, off_ctr, total;
     int64_t ntiles;   // 64 x 64 tiles of the update padded to 256 (prologue sums of squares)
@@ -1497,8 +1497,7 @@ int msr_linear_wgrad_sr_accum(uint16_t *acc, const uint16_t *x, int64_t ldx, con
     a.zero_init = zero_init != 0;
     a.ns.key = seed_key(seed, 0);
     a.ns.inject = inject;
-    const int T = wgrad_tile_choice(a.M, a.N, a.K);
-    if (T != 256 && std::max(xb, yb) < (size_t(1) << 31)) {
+    if (wgrad_takes_tiles(a.M, a.N, a.K) && std::max(xb, yb) < (size_t(1) << 31)) {
         TileArgs t = {};
         t.P = dy; t.ldp = ldy;
         t.Q = x; t.ldq = ldx;
@@ -1507,7 +1506,7 @@ int msr_linear_wgrad_sr_accum(uint16_t *acc, const uint16_t *x, int64_t ldx, con
         t.alpha = 1.0f;
         t.zero_init = a.zero_init;
         t.ns = a.ns;
-        return launch_tile_gemm(T, TILE_W, TILE_D, noise_mode, t, 1, nullptr, (hipStream_t)stream);
+        return launch_tile_gemm(TILE_W, TILE_D, noise_mode, t, 1, nullptr, (hipStream_t)stream);
     }
     return launch_gemm(a, 1, (hipStream_t)stream);
 }
@@ -1649,14 +1648,14 @@ static int ns_tile_products(const NSPart *parts, int n_parts, int64_t batch, int
         g.alpha = 1.0f;
         g.alpha_b = it == 0 ? alphas : nullptr;   // s0^2 x0 x0^T
         g.resid = rho;
-        if ((rc = launch_tile_gemm(L.tile, TILE_A, TILE_WS, 0, g, batch, nullptr, s))) return rc;
+        if ((rc = launch_tile_gemm(TILE_A, TILE_WS, 0, g, batch, nullptr, s))) return rc;
         g.P = g.Q = g.C = A; g.ldp = g.ldq = g.ldc = mp; g.sP = g.sQ = g.sC = as;
         g.D = B;
         g.K = mp;
         g.alpha = c_coef; g.beta = b_coef; g.diag = a_coef;
         g.alpha_b = nullptr;
         g.rvec = rho; g.resid = rr;
-        if ((rc = launch_tile_gemm(L.tile, TILE_B, TILE_WS, 0, g, batch, nullptr, s))) return rc;
+        if ((rc = launch_tile_gemm(TILE_B, TILE_WS, 0, g, batch, nullptr, s))) return rc;
         g.P = B;
         g.Q = X[cur]; g.ldq = np; g.sQ = xs;
         g.C = nullptr;
@@ -1666,7 +1665,7 @@ static int ns_tile_products(const NSPart *parts, int n_parts, int64_t batch, int
         g.rvec = rr; g.resid = nullptr;
         if (it != steps - 1) {
             g.D = X[cur ^ 1]; g.ldd = np; g.sD = xs;
-            if ((rc = launch_tile_gemm(L.tile, TILE_X, TILE_WS, 0, g, batch, nullptr, s))) return rc;
+            if ((rc = launch_tile_gemm(TILE_X, TILE_WS, 0, g, batch, nullptr, s))) return rc;
             cur ^= 1;
             continue;
         }
@@ -1702,7 +1701,7 @@ static int ns_tile_products(const NSPart *parts, int n_parts, int64_t batch, int
                 else { ga.D = nullptr; ga.DT = ap ? nullptr : pt.out + b0 * numel; ga.lddt = pt.cols; ga.sDT = numel; }
                 ga.d_vec = ga.dt_vec = vec;
                 const int out = ap ? (wide ? TILE_PD : TILE_PT) : (wide ? TILE_D : TILE_DT);
-                if ((rc = launch_tile_gemm(L.tile, TILE_X, out, ap ? ap->noise_mode : 0, ga, nb, ap ? &tab : nullptr, s))) return rc;
+                if ((rc = launch_tile_gemm(TILE_X, out, ap ? ap->noise_mode : 0, ga, nb, ap ? &tab : nullptr, s))) return rc;
             }
         }
     }

@@ -519,40 +519,72 @@ static int launch_tiles(int prod, int out, int mode, TileArgs &a, int64_t batch,
     return check_launch("tile_gemm_kernel");
 }
 
-int launch_tile_gemm(int T, int prod, int out, int mode, const TileArgs &a0, int64_t batch, const ApplyTab *tab,
-                     hipStream_t s) {
-    TileArgs a = a0;
-    if (batch == 0) return MSR_OK;
-    if (T == 64) return launch_tiles<64, 4>(prod, out, mode, a, batch, tab, s);
-    // T = 128: 4 stages (128 KiB of LDS, one work-group per CU) while every tile has a CU of its
-    // own, 2 stages (two work-groups per CU) beyond: 2048 x 2048 weight gradient of 4096 tokens
-    // (256 tiles) 35 against 48 us, Newton-Schulz of two 2048 x 2048 matrices (272 and 512 tiles)
-    // 538 against 448 us
-    const int64_t tm = a.M / 128, tn = a.N / 128, tiles = (prod == PR_A || prod == PR_B ? tm * (tm + 1) / 2 : tm * tn) * batch;
-    if (tiles <= TILE_CUS) return launch_tiles<128, 4>(prod, out, mode, a, batch, tab, s);
-    return launch_tiles<128, 2>(prod, out, mode, a, batch, tab, s);
+// Estimated time (us) of a product in `tiles` tiles of T (ring of S stages) over `slabs` K slabs:
+// rounds of the work-groups that run at once (LDS and registers allow 512 of 64/4, 768 of 64/2, 256
+// of 128/4 and 512 of 128/2), each the slabs plus a tile's start and end.  Fitted to kernel times
+// of A, B' and X' at 20 Newton-Schulz shapes (1-64 matrices of 256-2048 x 256-5632); the estimates
+// pick the fastest of the four, or one within 5 % of it, on nearly all.  Some of the times, us
+// (64/4, 64/2, 128/4, 128/2):
+//   40 tiles of 64 (12 of 128),  4 slabs   4.1   4.4   6.9   6.6
+//   168 (48),                   24 slabs   6.8   8.8  13.4  13.7
+//   528 (136),                  88 slabs  59.3  44.8  38.2  57.3
+//   576 (144),                  12 slabs  12.0   9.9  10.5  10.5
+//   1024 (256),                 32 slabs  30.9  30.6  20.6  24.3
+//   1152 (288),                  6 slabs  12.0  11.0  14.0   9.8
+//   8192 (2048),                16 slabs   121   105    90    72
+// 256-wide tiles (ns_gemm.hip): one work-group per CU.
+static double tile_cost(int T, int S, int64_t tiles, int64_t slabs) {
+    const double f = (double)tiles / TILE_CUS, k = (double)slabs;
+    // whole rounds of n work-groups, and a last one that is shorter when it leaves CUs less shared
+    auto rounds = [&](int64_t n, double least) {
+        const int64_t rest = tiles % n;
+        return (double)(tiles / n) + (rest ? least + (1.0 - least) * (double)rest / (double)n : 0.0);
+    };
+    if (T == 256) return 9.0 + 1.3 * k * (double)((tiles + TILE_CUS - 1) / TILE_CUS);
+    if (T == 64 && S == 4) return f <= 1.0 ? 3.4 + k * (0.13 + 0.13 * f) : 3.4 + rounds(512, 0.4) * (0.42 * k + 1.0);
+    if (T == 64) return 3.4 + std::max(0.5, f / 3.0) * (0.57 * k + 1.2);
+    if (S == 4) return 5.2 + (f <= 1.0 ? k * (0.33 + 0.17 * f) : rounds(TILE_CUS, 0.66) * (0.5 * k + 1.0));
+    return 5.0 + rounds(512, 0.45) * (0.98 * k + 1.2);
 }
 
-// Estimated time (us) of one product launch in T-wide tiles: work-groups in rounds over the
-// CUs, times K slabs of 64, times the measured time of a slab, plus the launch's fixed part.
-// Measured on Newton-Schulz of 1-12 matrices of 64 to 5632 rows and columns and on weight
-// gradients of 256-5632 features; the estimates are within 20 % of the measured times and pick
-// the fastest tile, or one within 3 % of it, on all of them (see tile_choice).
-static double tile_cost(int T, int64_t tiles, int64_t slabs) {
-    const double fill = (double)tiles / TILE_CUS;
-    if (T == 64) return 3.3 + (double)slabs * std::max(0.2, 0.24 * fill);
-    if (T == 128) {
-        if (tiles <= TILE_CUS) return 5.0 + (double)slabs * 0.49;
-        const int64_t full = tiles / (2 * TILE_CUS), rest = tiles % (2 * TILE_CUS);   // rounds of two per CU
-        return 5.0 + (double)slabs * (0.9 * (double)full + (rest == 0 ? 0.0 : rest <= TILE_CUS ? 0.55 : 0.55 + 0.35 * (double)(rest - TILE_CUS) / TILE_CUS));
+struct TileCfg {
+    int T, S;
+};
+constexpr TileCfg TILE_CFGS[4] = {{64, 4}, {64, 2}, {128, 4}, {128, 2}};
+
+// Tiles of an M x N product in T-wide tiles (upper ones only if symmetric).
+static int64_t tiles_of(int T, bool sym, int64_t M, int64_t N) {
+    const int64_t tm = M / T, tn = N / T;
+    return sym ? tm * (tm + 1) / 2 : tm * tn;
+}
+
+// The cheapest of the four for a product whose extents are multiples of 64.
+static TileCfg best_cfg(bool sym, int64_t M, int64_t N, int64_t K, int64_t batch, double *cost) {
+    TileCfg best = TILE_CFGS[0];
+    double least = -1.0;
+    for (const TileCfg &c : TILE_CFGS) {
+        if (M % c.T || N % c.T) continue;
+        const double t = tile_cost(c.T, c.S, tiles_of(c.T, sym, M, N) * batch, K / TBK);
+        if (least < 0.0 || t < least) { least = t; best = c; }
     }
-    return 9.0 + (double)slabs * 1.3 * (double)((tiles + TILE_CUS - 1) / TILE_CUS);
+    *cost = least;
+    return best;
+}
+
+int launch_tile_gemm(int prod, int out, int mode, const TileArgs &a0, int64_t batch, const ApplyTab *tab, hipStream_t s) {
+    TileArgs a = a0;
+    if (batch == 0) return MSR_OK;
+    double cost;
+    const TileCfg c = best_cfg(prod == PR_A || prod == PR_B, a.M, a.N, a.K, batch, &cost);
+    if (c.T == 64) return c.S == 4 ? launch_tiles<64, 4>(prod, out, mode, a, batch, tab, s) : launch_tiles<64, 2>(prod, out, mode, a, batch, tab, s);
+    return c.S == 4 ? launch_tiles<128, 4>(prod, out, mode, a, batch, tab, s) : launch_tiles<128, 2>(prod, out, mode, a, batch, tab, s);
 }
 
 static int64_t up(int64_t x, int64_t m) { return (x + m - 1) / m * m; }
 
-// Tile of a Newton-Schulz call (m <= n): the smallest estimate of one iteration's three
-// products, each with the padding that the tile brings.  Measured times in us (256 / 128 / 64):
+// Padding of a Newton-Schulz call (m <= n): the smallest estimate of one iteration's three
+// products, each in its best tile, with what the padding costs; 256 means the 256-wide kernel.
+// Measured times in us (all products 256 / 128 / 64 wide):
 //   4 of 256 x 256   165 / 104 / 65      1 of 2048 x 2048   710 / 286 / 371
 //   8 of 384 x 1536  351 / 170 / 121     2 of 2048 x 5632  1308 / 910 / 1333
 //   1 of 1024 x 1024 364 / 185 / 118     4 of 2048 x 2048   795 / 845 / 1126
@@ -561,27 +593,33 @@ int ns_tile_choice(int64_t batch, int64_t m, int64_t n) {
     int best = 256;
     double least = 0.0;
     for (int T : {256, 128, 64}) {
-        const int64_t mp = up(m, T), np = up(n, T), tm = mp / T, tn = np / T;
-        if (T != 256 && (tm * tn * batch >= (int64_t(1) << 28) || mp * np >= (int64_t(1) << 29))) continue;
-        const double c = tile_cost(T, tm * (tm + 1) / 2 * batch, np / TBK) + tile_cost(T, tm * (tm + 1) / 2 * batch, mp / TBK) +
-                         tile_cost(T, tm * tn * batch, mp / TBK);
+        const int64_t mp = up(m, T), np = up(n, T);
+        double c;
+        if (T == 256) {
+            const int64_t sym = tiles_of(256, true, mp, mp) * batch;
+            c = tile_cost(256, 2, sym, np / TBK) + tile_cost(256, 2, sym, mp / TBK) +
+                tile_cost(256, 2, tiles_of(256, false, mp, np) * batch, mp / TBK);
+        } else {
+            if (tiles_of(64, false, mp, np) * batch >= (int64_t(1) << 28) || mp * np >= (int64_t(1) << 29)) continue;
+            double ca, cb, cx;
+            best_cfg(true, mp, mp, np, batch, &ca);
+            best_cfg(true, mp, mp, mp, batch, &cb);
+            best_cfg(false, mp, np, mp, batch, &cx);
+            c = ca + cb + cx;
+        }
         if (T == 256 || c < least) { best = T; least = c; }
     }
     return best;
 }
 
-// Tile of a weight gradient M x N over K tokens (M, N multiples of 256).  Measured times in us
-// (256 / 128 / 64): 2048 x 2048 of 4096 tokens 78 / 35 / 66, 1024 x 4096 of 8192 139 / 62 / 129,
-// 768 x 768 of 8192 140 / 47 / 27, 5632 x 2048 of 4096 85 / 92 / 155, 4096 x 4096 of 2048
-// 60 / 66 / 94, 256 x 256 of 128 12 / 7.5 / 7.6.
-int wgrad_tile_choice(int64_t M, int64_t N, int64_t K) {
-    int best = 256;
-    double least = tile_cost(256, (M / 256) * (N / 256), K / TBK);
-    for (int T : {128, 64}) {
-        const double c = tile_cost(T, (M / T) * (N / T), K / TBK);
-        if (c < least) { best = T; least = c; }
-    }
-    return best;
+// Whether a weight gradient M x N over K tokens (M, N multiples of 256) takes these tiles rather
+// than the 256-wide ones.  Measured times in us (256 / 128 / 64): 2048 x 2048 of 4096 tokens
+// 78 / 35 / 66, 1024 x 4096 of 8192 139 / 62 / 129, 768 x 768 of 8192 140 / 47 / 27, 5632 x 2048
+// of 4096 85 / 92 / 155, 4096 x 4096 of 2048 60 / 66 / 94, 256 x 256 of 128 12 / 7.5 / 7.6.
+bool wgrad_takes_tiles(int64_t M, int64_t N, int64_t K) {
+    double c;
+    best_cfg(false, M, N, K, 1, &c);
+    return c < tile_cost(256, 2, (M / 256) * (N / 256), K / TBK);
 }
 
 }  // namespace msr

@@ -5,8 +5,8 @@
 
 namespace msr {
 
-// D = alpha P Q^T (+ beta C + diag I) of `batch` matrices; extents are multiples of the
-// tile, K of 64, and each operand matrix spans less than 2 GiB.
+// D = alpha P Q^T (+ beta C + diag I) of `batch` matrices; extents are multiples of 64,
+// and each operand matrix spans less than 2 GiB.
 struct TileArgs {
     const uint16_t *P; int64_t ldp, sP;
     const uint16_t *Q; int64_t ldq, sQ;
@@ -31,14 +31,13 @@ constexpr int64_t TILE_CUS = 256;   // work-groups that run at once, one per CU
 enum TileProd : int { TILE_A = 0, TILE_B = 1, TILE_X = 2, TILE_W = 3 };
 enum TileOut : int { TILE_WS = 0, TILE_D = 1, TILE_DT = 2, TILE_PD = 3, TILE_PT = 4 };
 
-// T: 64 or 128.  mode: noise mode of TILE_PD / TILE_PT (with `tab`, at most APPLY_MAX
-// matrices) and TILE_W.
-int launch_tile_gemm(int T, int prod, int out, int mode, const TileArgs &a, int64_t batch, const ApplyTab *tab,
-                     hipStream_t s);
+// mode: noise mode of TILE_PD / TILE_PT (with `tab`, at most APPLY_MAX matrices) and TILE_W.
+// The tile (64 or 128 wide, where the extents allow it) is the one with the least estimated time.
+int launch_tile_gemm(int prod, int out, int mode, const TileArgs &a, int64_t batch, const ApplyTab *tab, hipStream_t s);
 
-// The tile (64, 128 or 256) of a Newton-Schulz call of `batch` m x n matrices (m <= n), and
-// of a weight gradient M x N over K tokens.
+// What a Newton-Schulz call of `batch` m x n matrices (m <= n) pads to: 64 or 128 (these tiles),
+// or 256 (ns_gemm.hip's kernel); and whether a weight gradient M x N over K tokens takes these tiles.
 int ns_tile_choice(int64_t batch, int64_t m, int64_t n);
-int wgrad_tile_choice(int64_t M, int64_t N, int64_t K);
+bool wgrad_takes_tiles(int64_t M, int64_t N, int64_t K);
 
 }  // namespace msr
