@@ -980,11 +980,24 @@ __global__ __launch_bounds__(256) void normalize_kernel(const uint16_t *in, int6
 // Scaling: X0 = u / (||u||_F + 1e-7) is not rounded.  With e the exponent of
 // ||u||_F, X0 is kept as x0 = u when |e| <= PRO_ELIM (the first products then
 // multiply by s = 1 / (||u|| + 1e-7): A = s^2 x0 x0^T, X' = s (B' x0 + ...)),
-// else as x0 = u 2^-e with s0 = 2^e s (ns_rescale_kernel; bounded values keep
+// else as x0 = u 2^-e with s0 = 2^e s (ns_finalize_kernel; bounded values keep
 // products in range).  Both are the same numbers: bf16 products are exact in
 // fp32 and every fp32 rounding of the products commutes with the power-of-two
 // scale while no partial result leaves the normal range.
 // ---------------------------------------------------------------------------
+
+// The sum of 256 values, one per thread, by the tree that adds the upper half to the lower at
+// 128, 64, ... 1, in every thread of the first wave: the first two steps through LDS, the others by
+// shuffles (one barrier; eight with the whole tree in LDS).
+__device__ __forceinline__ float tree_sum256(float s, float *red) {
+    red[threadIdx.x] = s;
+    __syncthreads();
+    const int l = threadIdx.x & 63;
+    float v = (red[l] + red[l + 128]) + (red[l + 64] + red[l + 192]);
+#pragma unroll
+    for (int w = 32; w > 0; w >>= 1) v = v + __shfl_down(v, w, 64);
+    return __shfl(v, 0, 64);
+}
 
 constexpr int PRO_MAX = 96;       // matrices per prologue launch (kernel-argument table)
 constexpr int PRO_ELIM = 16;
@@ -1119,13 +1132,8 @@ __global__ __launch_bounds__(256) void ns_prologue_kernel(PrologueArgs a) {
             }
         }
     }
-    red[threadIdx.x] = s;
-    __syncthreads();
-    for (int wdt = 128; wdt > 0; wdt >>= 1) {
-        if (threadIdx.x < wdt) red[threadIdx.x] = red[threadIdx.x] + red[threadIdx.x + wdt];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) a.tpart[b * a.ntiles + ty * a.ntx + tx] = red[0];
+    const float sum = tree_sum256(s, red);   // its barrier also completes the tile in LDS
+    if (threadIdx.x == 0) a.tpart[b * a.ntiles + ty * a.ntx + tx] = sum;
     if (!a.T) return;
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
@@ -1147,25 +1155,21 @@ __global__ __launch_bounds__(256) void ns_prologue_kernel(PrologueArgs a) {
     }
 }
 
-// Per matrix b: ||u||_F from the tile sums, the first products' factors
-// alphas[b] = s^2, alphas[batch + b] = s, and rexp[b]: 0 when x0 = u, else -e
-// (ns_rescale_kernel scales x0 by 2^-e).  ||u|| >= 2^64 (inf) gives e = 127 and
-// s = 0 (u / inf = 0, as the reference's normalisation); NaN propagates.
+// Per matrix b: ||u||_F from the tile sums and the first products' factors
+// alphas[b] = s^2, alphas[batch + b] = s; x0 stays u, or becomes u 2^-e (its padded X0: n8 16-byte
+// chunks at X + b sX) where the exponent e is out of range.  ||u|| >= 2^64 (inf) gives e = 127
+// and s = 0 (u / inf = 0, as the reference's normalisation); NaN propagates.  `bpm` work-groups
+// per matrix each form the norm (tile sums are few and in L2: one launch, where a second one for the
+// rescale cost 4-6 us of a small call) and scale their share of X0.
 __global__ __launch_bounds__(256) void ns_finalize_kernel(const float *tpart, int64_t ntiles, int64_t batch,
-                                                          float *alphas, int *rexp, int *tile_ctr) {
+                                                          float *alphas, int *tile_ctr, uint16_t *X, int64_t sX,
+                                                          int64_t n8, int64_t bpm) {
     __shared__ float red[256];
-    const int64_t b = blockIdx.x;
-    if (b == 0 && threadIdx.x <= NXCD) tile_ctr[threadIdx.x] = 0;   // the GEMMs' tile counters start at zero
+    const int64_t b = blockIdx.x / bpm, part = blockIdx.x % bpm;
+    if (blockIdx.x == 0 && threadIdx.x <= NXCD) tile_ctr[threadIdx.x] = 0;   // the GEMMs' tile counters start at zero
     float s = 0.0f;
     for (int64_t t = threadIdx.x; t < ntiles; t += 256) s = s + tpart[b * ntiles + t];
-    red[threadIdx.x] = s;
-    __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-        if (threadIdx.x < w) red[threadIdx.x] = red[threadIdx.x] + red[threadIdx.x + w];
-        __syncthreads();
-    }
-    if (threadIdx.x != 0) return;
-    const float d = sqrtf(red[0]);
+    const float d = sqrtf(tree_sum256(s, red));
     int e = 0;
     float s0;
     if (d == __builtin_huge_valf()) {
@@ -1176,27 +1180,19 @@ __global__ __launch_bounds__(256) void ns_finalize_kernel(const float *tpart, in
         s0 = ldexpf(1.0f / (d + 1e-7f), e);
     }
     const bool scaled = e > PRO_ELIM || e < -PRO_ELIM;
-    const float f = scaled ? s0 : ldexpf(s0, -e);   // exact for |e| <= PRO_ELIM: 1 / (||u|| + 1e-7)
-    alphas[b] = f * f;
-    alphas[batch + b] = f;
-    rexp[b] = scaled ? -e : 0;
-}
-
-// x0 <- x0 2^rexp[b] over matrix b's padded X0 (n8 16-byte chunks at X + b sX),
-// for the matrices the finalisation marked; the others return at once.  `bpm`
-// work-groups per matrix: work-group g serves matrix g / bpm.
-__global__ __launch_bounds__(256) void ns_rescale_kernel(uint16_t *X, int64_t sX, int64_t n8, int64_t bpm,
-                                                         const int *rexp) {
-    const int64_t b = blockIdx.x / bpm, part = blockIdx.x % bpm;
-    const int ne = rexp[b];
-    if (ne == 0) return;
+    if (part == 0 && threadIdx.x == 0) {
+        const float f = scaled ? s0 : ldexpf(s0, -e);   // exact for |e| <= PRO_ELIM: 1 / (||u|| + 1e-7)
+        alphas[b] = f * f;
+        alphas[batch + b] = f;
+    }
+    if (!scaled) return;
     uint4 *x = reinterpret_cast<uint4 *>(X + b * sX);
     for (int64_t i = part * 256 + threadIdx.x; i < n8; i += bpm * 256) {
         const uint4 v = x[i];
         const uint32_t u[4] = {v.x, v.y, v.z, v.w};
         uint32_t o[4];
 #pragma unroll
-        for (int k = 0; k < 4; ++k) o[k] = rne_bf16x2(ldexpf(bf16_lo(u[k]), ne), ldexpf(bf16_hi(u[k]), ne));
+        for (int k = 0; k < 4; ++k) o[k] = rne_bf16x2(ldexpf(bf16_lo(u[k]), -e), ldexpf(bf16_hi(u[k]), -e));
         x[i] = make_uint4(o[0], o[1], o[2], o[3]);
     }
 }
@@ -1207,7 +1203,7 @@ struct NSLayout {
     int64_t m, n, mp, np;
     int tile;         // mp and np are multiples of it: 256 (this file's kernel), or 64 / 128 (tile_gemm.hip)
     bool transposed;
-    size_t off_x[2], off_a, off_b, off_part, off_alpha, off_rho, off_r, off_tpart, off_rexp, off_ctr, total;
+    size_t off_x[2], off_a, off_b, off_part, off_alpha, off_rho, off_r, off_tpart, off_ctr, total;
     int64_t ntiles;   // 64 x 64 tiles of the update padded to 256 (prologue sums of squares)
 };
 
@@ -1236,7 +1232,6 @@ static NSLayout ns_layout(int64_t batch, int64_t rows, int64_t cols) {
     L.off_r = take((size_t)batch * m256 * 4);      // residuals of B''s diagonal
     L.ntiles = (m256 / 64) * (n256 / 64);
     L.off_tpart = take((size_t)batch * L.ntiles * 4);   // tile sums of squares of the update
-    L.off_rexp = take((size_t)batch * 4);               // prologue scale exponents
     L.off_ctr = take(16 * 4);                           // the GEMMs' dynamic tile counters
     L.total = o;
     return L;
@@ -1619,16 +1614,13 @@ static int ns_prologue_part(const NSPart &pt, uint16_t *X0, float *tpart, const 
 
 // After the parts' prologues, over all `batch` matrices of the call: the first
 // products' factors and the rescale of out-of-range matrices.
-static int ns_prologue_finish(int64_t batch, uint16_t *X0, float *tpart, float *alphas, int *rexp, int *tile_ctr,
-                              const NSLayout &L, hipStream_t s) {
-    const int64_t xs = L.mp * L.np;
-    hipLaunchKernelGGL(ns_finalize_kernel, dim3((unsigned)batch), dim3(256), 0, s, tpart, L.ntiles, batch, alphas, rexp,
-                       tile_ctr);
-    int rc = check_launch("ns_finalize_kernel");
-    if (rc) return rc;
-    const int64_t n8 = xs / 8, bpm = std::min<int64_t>((n8 + 255) / 256, 64);
-    hipLaunchKernelGGL(ns_rescale_kernel, dim3((unsigned)(bpm * batch)), dim3(256), 0, s, X0, xs, n8, bpm, rexp);
-    return check_launch("ns_rescale_kernel");
+static int ns_prologue_finish(int64_t batch, uint16_t *X0, float *tpart, float *alphas, int *tile_ctr, const NSLayout &L,
+                              hipStream_t s) {
+    const int64_t xs = L.mp * L.np, n8 = xs / 8;
+    const int64_t bpm = std::min<int64_t>((n8 + 255) / 256, std::min<int64_t>(64, std::max<int64_t>(4, 1024 / batch)));
+    hipLaunchKernelGGL(ns_finalize_kernel, dim3((unsigned)(bpm * batch)), dim3(256), 0, s, tpart, L.ntiles, batch, alphas,
+                       tile_ctr, X0, xs, n8, bpm);
+    return check_launch("ns_finalize_kernel");
 }
 
 // The iterations and the last product of ns_run_parts in 64- or 128-wide tiles
@@ -1726,7 +1718,7 @@ static int ns_run_parts(const NSPart *parts, int n_parts, int64_t batch, int32_t
     int rc = MSR_OK;
     for (int i = 0; i < n_parts; ++i)
         if ((rc = ns_prologue_part(parts[i], X[0], tpart, L, s))) return rc;
-    if ((rc = ns_prologue_finish(batch, X[0], tpart, alphas, (int *)(ws + L.off_rexp), tile_ctr, L, s))) return rc;
+    if ((rc = ns_prologue_finish(batch, X[0], tpart, alphas, tile_ctr, L, s))) return rc;
 
     if (L.tile != 256) return ns_tile_products(parts, n_parts, batch, steps, a_coef, b_coef, c_coef, X, A, B, alphas, rho, rr, L, s);
     const int mp = (int)L.mp, np = (int)L.np;
