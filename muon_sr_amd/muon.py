@@ -32,7 +32,7 @@ import torch
 from torch.optim import Optimizer
 
 from . import _lib
-from .adamw import _adamw_add, _AdamWBatch
+from .adamw import _AdamWBatch
 from .adamw_8bit import _Adam8Batch, init_8bit_state, split_8bit_state, TritonAdamW8bit
 
 NS_COEFFS = (3.4445, -4.7750, 2.0315)
@@ -656,13 +656,13 @@ class TritonMuonSRWithAuxAdam(_StackedBufsMixin, Optimizer):
                 hyper = (lr, beta1, beta2, eps, weight_decay)
                 batch = _Adam8Batch(*hyper) if eight_bit else _AdamWBatch(_lib.ADAMW, *hyper)
                 try:
-                    self._step_adamw(group, group_offset, beta1, beta2, eight_bit, batch)
+                    self._step_adamw(group, group_offset, eight_bit, batch)
                 finally:
                     batch.flush()
 
         return loss
 
-    def _step_adamw(self, group, group_offset, beta1, beta2, eight_bit, batch):
+    def _step_adamw(self, group, group_offset, eight_bit, batch):
         for i, p in enumerate(group["params"]):
             assert p.dtype == torch.bfloat16, "only bfloat16 is supported."
             if p.grad is None:
@@ -680,7 +680,7 @@ class TritonMuonSRWithAuxAdam(_StackedBufsMixin, Optimizer):
                 state["ema"] = torch.zeros_like(p, dtype=torch.bfloat16, memory_format=torch.contiguous_format)
                 state["ema_squared"] = torch.zeros_like(p, dtype=torch.bfloat16, memory_format=torch.contiguous_format)
             state["step"] += 1
-            _adamw_add(batch, p, p.grad, state["ema"], state["ema_squared"], beta1, beta2, state["step"], group_offset + i)
+            batch.add_adamw(p, p.grad, state["ema"], state["ema_squared"], state["step"], group_offset + i)
 
     def load_state_dict(self, state_dict):
         """As torch's, except that the states of ``optim_bits=8`` AdamW groups keep
