@@ -1030,10 +1030,12 @@ __global__ __launch_bounds__(256) void ns_prologue_kernel(PrologueArgs a) {
     __shared__ __align__(16) uint16_t tile[64][72];
     __shared__ float red[256];
     // tile (tx, ty) of matrix b: work-groups in runs of MSR_PRO_XCD consecutive tiles per XCD
-    const int64_t gx = gridDim.x, gy = gridDim.y;
-    const int64_t lin = xcd_place((int64_t)blockIdx.x + gx * ((int64_t)blockIdx.y + gy * (int64_t)blockIdx.z),
-                                  gx * gy * (int64_t)gridDim.z, MSR_PRO_XCD);
-    const int64_t tx = lin % gx, ty = (lin / gx) % gy, b = lin / (gx * gy);
+    // (fewer than 2^32: a tile is 4096 elements in memory or padding to 256)
+    const uint32_t gx = gridDim.x, gy = gridDim.y;
+    const uint32_t lin = (uint32_t)xcd_place((int64_t)(blockIdx.x + gx * (blockIdx.y + gy * blockIdx.z)),
+                                             (int64_t)(gx * gy * gridDim.z), MSR_PRO_XCD);
+    const uint32_t row = lin / gx;
+    const int64_t tx = lin - row * gx, b = row / gy, ty = row % gy;
     const int64_t r0 = ty * 64, c0 = tx * 64;
     const int64_t numel = a.rows * a.cols;
     const int j = threadIdx.x & 7, i0 = threadIdx.x >> 3;
@@ -1121,7 +1123,10 @@ __global__ __launch_bounds__(256) void ns_prologue_kernel(PrologueArgs a) {
             s = s + lo * lo;
             s = s + hi * hi;
         }
-        *reinterpret_cast<uint4 *>(&tile[i][8 * j]) = make_uint4(w[0], w[1], w[2], w[3]);
+        // chunk j of row i at j ^ (i / 8): the transposed reads below take rows 8 apart, whose pitch
+        // alone would put them in two groups of banks (4-way conflicts; with 32-bit tile numbers, a call
+        // for 8 tall matrices of 1536 x 384: 111.0 -> 109.7 us)
+        *reinterpret_cast<uint4 *>(&tile[i][8 * (j ^ (i >> 3))]) = make_uint4(w[0], w[1], w[2], w[3]);
         if (a.S && r < a.Rp && c < a.Cp) {
             uint16_t *d = a.S + b * a.sS + r * a.ldS + c;
             if (VEC) {
@@ -1138,12 +1143,13 @@ __global__ __launch_bounds__(256) void ns_prologue_kernel(PrologueArgs a) {
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
         const int cc = i0 + 32 * h;            // T row (u column) within the tile
+        const int cs = cc ^ (8 * j);           // its place in rows 8 j .. 8 j + 7
         const int64_t c = c0 + cc, r = r0 + 8 * j;
         if (c < a.Cp && r < a.Rp) {
             uint32_t o[4];
 #pragma unroll
             for (int k = 0; k < 4; ++k)
-                o[k] = (uint32_t)tile[8 * j + 2 * k][cc] | ((uint32_t)tile[8 * j + 2 * k + 1][cc] << 16);
+                o[k] = (uint32_t)tile[8 * j + 2 * k][cs] | ((uint32_t)tile[8 * j + 2 * k + 1][cs] << 16);
             uint16_t *d = a.T + b * a.sT + c * a.ldT + r;
             if (VEC) {
                 *reinterpret_cast<uint4 *>(d) = make_uint4(o[0], o[1], o[2], o[3]);
