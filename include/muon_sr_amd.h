@@ -202,6 +202,12 @@ int msr_adamw8bit_multi(const msr_adam8_item *items, int32_t count, const float 
                         const void *qtable, int32_t block, float lr, float beta1, float beta2, float eps,
                         float weight_decay, float bc1, float bc2, int32_t noise_mode, msr_stream_t stream);
 
+/* Host only: *apart is 1 if no memory that a step of one of the two lists writes is touched by a
+ * step of the other, so that the lists may be launched one after the other whatever the order of their
+ * steps in the group; else 0.  block: the quantized list's. */
+int msr_adamw8bit_apart(const msr_adam8_item *quantized, int32_t n_quantized, int32_t block,
+                        const msr_adamw_item *bf16, int32_t n_bf16, int32_t *apart);
+
 /* ---------------------------------------------------------------------------
  * (b) Muon momentum prologue over one shape group.
  * Replaces the grad->stack copy and the _muon_prepare_kernel launch of

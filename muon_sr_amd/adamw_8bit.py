@@ -7,6 +7,8 @@ step runs fused gfx950 kernels over many tensors at a time (libmuon_sr_amd.so).
 """
 from __future__ import annotations
 
+import ctypes
+import itertools
 import math
 import struct
 import weakref
@@ -88,47 +90,84 @@ def quant_table(state):
 class _Adam8Batch:
     """The 8-bit steps of one parameter group, launched many tensors at a time: quantized ones by
     msr_adamw8bit_multi, bf16-moment ones by msr_adamw_multi (the reference launches one kernel
-    per tensor, muon_sr/triton_adamw_8bit.py:196-205).  Added in a ``try`` and flushed in its
-    ``finally``, as _AdamWBatch."""
+    per tensor, muon_sr/triton_adamw_8bit.py:196-205).  Steps run in the order they were added
+    wherever they share memory, also where one kind's share with the other's.  Added in a ``try`` and
+    flushed in its ``finally``, as _AdamWBatch."""
 
     _PACK = struct.Struct("=QQQQQQqIi").pack   # msr_adam8_item
 
     def __init__(self, lr, beta1, beta2, eps, weight_decay):
         self.hyper = (lr, beta1, beta2, eps, weight_decay)
-        self.b16 = _AdamWBatch(_lib.ADAMW_8BIT16, *self.hyper)
-        self.items, self.key = [], None
+        self.b16 = _AdamWBatch(_lib.ADAMW_8BIT16, *self.hyper)   # the pending bf16-moment steps
+        self.items, self.key = [], None                          # the pending quantized ones, and what they share
+        self.order = []                                          # whether each pending step, as added, is quantized
+        self.device = None
 
     def add(self, p, g, state, seed):
         """One tensor's step with a state from ``init_8bit_state``."""
         n = state["step"]
         _, beta1, beta2, _, _ = self.hyper
+        device = p.get_device()
+        if device != self.device:
+            self.flush()
+            self.device = device
         if state["optim_bits"] != 8:
             self.b16.add(p, g, state["state1"], state["state2"], 1 - beta1 ** n, 1 - beta2 ** n, seed)
+            self.order.append(False)
             return
         # what the tensors of a launch share
         key = (state["qmap1"].data_ptr(), state["qmap2"].data_ptr(), quant_table(state), state["block_size"], n,
-               p.get_device(), _lib.stream_of(p))
+               _lib.stream_of(p))
         if key != self.key:
             self._flush8()
             self.key = key
         self.items.append(self._PACK(p.data_ptr(), g.data_ptr(), state["state1"].data_ptr(), state["state2"].data_ptr(),
                                      state["absmax1"].data_ptr(), state["absmax2"].data_ptr(), p.numel(), seed, 0))
+        self.order.append(True)
 
-    def _flush8(self):
-        if not self.items:
-            return
-        items, self.items = self.items, []
-        q1, q2, qt, block, n, _, stream = self.key
+    def _launch8(self, items):
+        q1, q2, qt, block, n, stream = self.key
         lr, beta1, beta2, eps, weight_decay = self.hyper
         rc = _lib.lib().msr_adamw8bit_multi(b"".join(items), len(items), q1, q2, qt, block, lr, beta1, beta2, eps,
                                             weight_decay, 1 - beta1 ** n, 1 - beta2 ** n, _lib.noise_mode(), stream)
         _lib.check(rc, "msr_adamw8bit_multi")
+
+    def _apart(self):
+        """Whether no pending step of one kind touches memory that one of the other kind writes."""
+        apart = ctypes.c_int32(0)
+        _lib.check(_lib.lib().msr_adamw8bit_apart(b"".join(self.items), len(self.items), self.key[3],
+                                                  b"".join(self.b16.items), len(self.b16.items), ctypes.byref(apart)),
+                   "msr_adamw8bit_apart")
+        return apart.value != 0
+
+    def _flush8(self):
+        """Launches the pending quantized steps; the bf16-moment ones stay pending where they may."""
+        items, order = self.items, self.order
+        if not items:
+            return
+        if not self.b16.items or self._apart():
+            self.items, self.order = [], [False] * len(self.b16.items)
+            self._launch8(items)
+            return
+        self.items, self.order = [], []
+        items16, self.b16.items = self.b16.items, []
+        at8 = at16 = 0
+        for quantized, run in itertools.groupby(order):   # runs of one kind, as added
+            n = sum(1 for _ in run)
+            if quantized:
+                self._launch8(items[at8:at8 + n])
+                at8 += n
+            else:
+                self.b16.items = items16[at16:at16 + n]
+                self.b16.flush()
+                at16 += n
 
     def flush(self):
         try:
             self._flush8()
         finally:
             self.b16.flush()
+            self.order = []
 
 
 def adamw8bit_launch(p, g, state, lr, beta1, beta2, eps, weight_decay, seed):

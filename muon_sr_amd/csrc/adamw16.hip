@@ -372,15 +372,16 @@ int adamw16_launch(int form, const msr_adamw_item *items, int32_t count, float l
     return check_launch("adamw16_kernel");
 }
 
+void item_ranges(const msr_adamw_item &x, int32_t id, ItemRange *r) {
+    const size_t b = 2 * (size_t)x.n;
+    const void *q[4] = {x.p, x.m, x.v, x.g};
+    for (int k = 0; k < 4; ++k) r[k] = {(uintptr_t)q[k], (uintptr_t)q[k] + b, id, k < 3};
+}
+
 static bool items_conflict(const msr_adamw_item *items, int32_t count) {
     ItemRange r[4 * A16_MAXT];
-    int n = 0;
-    for (int32_t i = 0; i < count; ++i) {
-        const size_t b = 2 * (size_t)items[i].n;
-        const void *q[4] = {items[i].p, items[i].m, items[i].v, items[i].g};
-        for (int k = 0; k < 4; ++k) r[n++] = {(uintptr_t)q[k], (uintptr_t)q[k] + b, i, k < 3};
-    }
-    return ranges_conflict(r, n);
+    for (int32_t i = 0; i < count; ++i) item_ranges(items[i], i, r + 4 * i);
+    return ranges_conflict(r, 4 * count);
 }
 
 // Every item's own operands distinct (or the same buffer, updated in place).

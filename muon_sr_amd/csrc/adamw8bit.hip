@@ -7,6 +7,7 @@
 #include <cstring>
 #include <algorithm>
 #include <utility>
+#include <new>
 #include <vector>
 
 #include "common.hpp"
@@ -907,17 +908,18 @@ static int check_group8(const Adam8Group &g, const char *name) {
     return MSR_OK;
 }
 
+// The memory of an item: 6 ranges, marked `id`.
+static void item_ranges(const msr_adam8_item &x, int32_t block, int32_t id, ItemRange *r) {
+    const size_t e = (size_t)x.n, ab = 4 * ((e + block - 1) / block);
+    const void *q[6] = {x.p, x.state1, x.state2, x.absmax1, x.absmax2, x.g};
+    const size_t len[6] = {2 * e, e, e, ab, ab, 2 * e};
+    for (int k = 0; k < 6; ++k) r[k] = {(uintptr_t)q[k], (uintptr_t)q[k] + len[k], id, k < 5};
+}
+
 static bool items_conflict(const msr_adam8_item *items, int32_t count, int32_t block) {
     ItemRange r[6 * F8_MAXT];
-    int n = 0;
-    for (int32_t i = 0; i < count; ++i) {
-        const msr_adam8_item &x = items[i];
-        const size_t e = (size_t)x.n, ab = 4 * ((e + block - 1) / block);
-        const void *q[6] = {x.p, x.state1, x.state2, x.absmax1, x.absmax2, x.g};
-        const size_t len[6] = {2 * e, e, e, ab, ab, 2 * e};
-        for (int k = 0; k < 6; ++k) r[n++] = {(uintptr_t)q[k], (uintptr_t)q[k] + len[k], i, k < 5};
-    }
-    return ranges_conflict(r, n);
+    for (int32_t i = 0; i < count; ++i) item_ranges(items[i], block, i, r + 6 * i);
+    return ranges_conflict(r, 6 * count);
 }
 
 extern "C" {
@@ -988,6 +990,27 @@ int msr_adamw8bit_multi(const msr_adam8_item *items, int32_t count, const float 
             }
         }
         if (nfit > 0 && (rc = launch_fast8(grp, c, fit, nfit, s))) return rc;
+    }
+    return MSR_OK;
+}
+
+int msr_adamw8bit_apart(const msr_adam8_item *quantized, int32_t n_quantized, int32_t block, const msr_adamw_item *bf16,
+                        int32_t n_bf16, int32_t *apart) {
+    if (n_quantized < 0 || n_bf16 < 0 || (n_quantized > 0 && !quantized) || (n_bf16 > 0 && !bf16) || block < 1 || !apart) {
+        set_error("msr_adamw8bit_apart: bad arguments");
+        return MSR_ERR_ARG;
+    }
+    try {
+        std::vector<ItemRange> r(6 * (size_t)n_quantized + 4 * (size_t)n_bf16);
+        size_t n = 0;
+        for (int32_t i = 0; i < n_quantized; ++i)   // ids are the lists': sharing inside one is the step's own check
+            if (quantized[i].n > 0) { item_ranges(quantized[i], block, 0, &r[n]); n += 6; }
+        for (int32_t i = 0; i < n_bf16; ++i)
+            if (bf16[i].n > 0) { item_ranges(bf16[i], 1, &r[n]); n += 4; }
+        *apart = !ranges_conflict(r.data(), (int)n);
+    } catch (const std::bad_alloc &) {
+        set_error("msr_adamw8bit_apart: out of host memory");
+        return MSR_ERR_ARG;
     }
     return MSR_OK;
 }

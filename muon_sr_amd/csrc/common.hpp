@@ -480,7 +480,6 @@ inline bool partial_overlap(const void *a, size_t na, const void *b, size_t nb) 
     return x < y + nb && y < x + na;
 }
 
-
 // A memory range of one item of a launch, and whether some memory that one item writes is
 // touched by another (such items run in launches of their own, in order).
 struct ItemRange {
@@ -495,6 +494,8 @@ inline bool ranges_conflict(ItemRange *r, int n) {
             if (r[i].item != r[j].item && (r[i].write || r[j].write)) return true;
     return false;
 }
+// The memory of a bf16-moment AdamW item: 4 ranges, marked `id` (adamw16.hip).
+void item_ranges(const msr_adamw_item &x, int32_t id, ItemRange *r);
 
 // Grid size for a grid-stride loop over `work` items with `threads` per block.
 inline unsigned grid_for(int64_t work, int threads, int64_t cap = 256 * 32) {
