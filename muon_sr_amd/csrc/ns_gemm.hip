@@ -2115,12 +2115,13 @@ constexpr int64_t EACH_NUMEL = int64_t(1) << 27;
 
 // The calls of a list of matrices: indices, grouped by Newton-Schulz shape (a tall matrix has the
 // shape of its transpose) and cut evenly into runs of at most EACH_NUMEL elements; inside a run
-// the matrices of one layout and gradient type are next to each other.
+// the matrices of one layout, gradient type and scale (by its bits) are next to each other.
 static std::vector<std::vector<int32_t>> each_runs(const msr_muon_matrix *x, int32_t count) {
     std::vector<int32_t> order((size_t)count);
     for (int32_t i = 0; i < count; ++i) order[i] = i;
     auto key = [&](int32_t i) {
-        return std::make_tuple(std::min(x[i].rows, x[i].cols), std::max(x[i].rows, x[i].cols), x[i].rows > x[i].cols, x[i].grad_f32 != 0);
+        return std::make_tuple(std::min(x[i].rows, x[i].cols), std::max(x[i].rows, x[i].cols), x[i].rows > x[i].cols, x[i].grad_f32 != 0,
+                               __builtin_bit_cast(uint32_t, x[i].scale));
     };
     std::stable_sort(order.begin(), order.end(), [&](int32_t a, int32_t b) { return key(a) < key(b); });
     std::vector<std::vector<int32_t>> runs;
@@ -2165,22 +2166,28 @@ static int each_run(const msr_muon_matrix *x, const std::vector<int32_t> &run, f
         grads[i] = m.grad; bufs[i] = m.buf; params[i] = m.param;
         pseeds[i] = m.prepare_seed; aseeds[i] = m.apply_seed;
     }
-    NSPrepare pps[4];
-    NSApply aps[4];
-    NSPart parts[4];   // wide and tall, bf16 and fp32 gradients
-    int np = 0;
-    for (int64_t i = 0; i < n;) {
+    // parts: wide and tall, bf16 and fp32 gradients, and what scales the matrices have
+    auto same = [](const msr_muon_matrix &u, const msr_muon_matrix &v) {
+        return u.rows == v.rows && (u.grad_f32 != 0) == (v.grad_f32 != 0) &&
+               __builtin_bit_cast(uint32_t, u.scale) == __builtin_bit_cast(uint32_t, v.scale);
+    };
+    std::vector<int64_t> cut;
+    for (int64_t i = 0; i < n; ++i)
+        if (i == 0 || !same(x[run[i - 1]], x[run[i]])) cut.push_back(i);
+    const int np = (int)cut.size();
+    cut.push_back(n);
+    std::vector<NSPrepare> pps((size_t)np);
+    std::vector<NSApply> aps((size_t)np);
+    std::vector<NSPart> parts((size_t)np);
+    for (int k = 0; k < np; ++k) {
+        const int64_t i = cut[k];
         const msr_muon_matrix &m = x[run[i]];
-        int64_t e = i;
-        while (e < n && x[run[e]].rows == m.rows && (x[run[e]].grad_f32 != 0) == (m.grad_f32 != 0)) ++e;
-        pps[np] = NSPrepare{&grads[i], m.grad_f32 != 0, nullptr, 0, 0u, &bufs[i], &pseeds[i], beta, nesterov, nullptr, (int)mode};
-        aps[np] = NSApply{&params[i], &aseeds[i], lr, wd, m.scale, (int)mode, nullptr};
+        pps[k] = NSPrepare{&grads[i], m.grad_f32 != 0, nullptr, 0, 0u, &bufs[i], &pseeds[i], beta, nesterov, nullptr, (int)mode};
+        aps[k] = NSApply{&params[i], &aseeds[i], lr, wd, m.scale, (int)mode, nullptr};
         // the last product's store writes the parameters: `out` only marks the layout (never accessed)
-        parts[np] = NSPart{i, e - i, m.rows, m.cols, nullptr, static_cast<uint16_t *>(ws), &aps[np], &pps[np]};
-        ++np;
-        i = e;
+        parts[k] = NSPart{i, cut[k + 1] - i, m.rows, m.cols, nullptr, static_cast<uint16_t *>(ws), &aps[k], &pps[k]};
     }
-    return ns_run_parts(parts, np, n, steps, a, b, c, ws, L, s);
+    return ns_run_parts(parts.data(), np, n, steps, a, b, c, ws, L, s);
 }
 
 extern "C" {

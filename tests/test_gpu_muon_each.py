@@ -37,7 +37,7 @@ def _one_by_one(L, mats, mode):
         check(L, L.msr_muon_fused_step(ptr_array([m["g"].data_ptr()]), int(m["g"].dtype == torch.float32),
                                        m["b"].data_ptr(), 0, 1, r, c, 0.95, 1, m["seeds"][0], 5, *NS_COEFFS, None,
                                        ptr_array([m["p"].data_ptr()]), ptr_array([m["seeds"][1]], ctypes.c_uint32), 0.02,
-                                       0.01, _scale((r, c)), mode, None, None, ws.data_ptr(), nb.value, stream()))
+                                       0.01, m.get("scale", _scale((r, c))), mode, None, None, ws.data_ptr(), nb.value, stream()))
 
 
 def _each(L, mats, mode):
@@ -45,7 +45,7 @@ def _each(L, mats, mode):
     from muon_sr_amd.muon import NS_COEFFS
     arr = (_lib.MuonMatrix * len(mats))(*[
         _lib.MuonMatrix(m["g"].data_ptr(), m["b"].data_ptr(), m["p"].data_ptr(), *m["p"].shape, *m["seeds"],
-                        int(m["g"].dtype == torch.float32), _scale(m["p"].shape)) for m in mats])
+                        int(m["g"].dtype == torch.float32), m.get("scale", _scale(m["p"].shape))) for m in mats])
     at, n = ctypes.addressof(arr), len(mats)
     nb = ctypes.c_size_t(0)
     check(L, L.msr_muon_each_workspace_bytes(at, n, ctypes.byref(nb)))
@@ -98,3 +98,16 @@ def test_error_leaves_earlier_parameters_stepped(L):
         TritonMuonSR([*ps, bad, last]).step()
     changed = [not torch.equal(p, b) for p, b in zip((*ps, bad, last), before)]
     assert changed == [True, True, False, False]
+
+
+def test_scales_of_their_own(L):
+    """Matrices of one shape whose scales differ: each is stepped with its own."""
+    mk = lambda: _make([(64, 96)] * 5 + [(96, 64)] * 2, lambda i: i == 3, 11)  # noqa: E731
+    scales = [1.0, 0.5, 1.0, 0.25, 0.5, 2.0, 1.0]
+    x, y = mk(), mk()
+    for m, s in zip((*x, *y), scales * 2):
+        m["scale"] = s
+    _one_by_one(L, x, O.NOISE_PHILOX8)
+    _each(L, y, O.NOISE_PHILOX8)
+    for i, (u, v) in enumerate(zip(x, y)):
+        assert torch.equal(u["p"].view(torch.int16), v["p"].view(torch.int16)), i
