@@ -112,6 +112,7 @@ int msr_adamw_bf16_step(uint16_t *p, const uint16_t *g, uint16_t *ema, uint16_t 
  * msr_centralize_bf16(rows of item.cols elements, strength) gives, without writing it; tensors
  * 16-byte aligned, cols a multiple of 8 and at most MSR_ADAMW_CENTRAL_MAX_COLS (else
  * MSR_ERR_ARG: centralize first).  strength is unused in the other forms.  items: HOST array.
+ * A list with an item that is refused is refused whole, before anything is launched.
  * noise_mode: MSR_NOISE_TRITON or MSR_NOISE_PHILOX8. */
 typedef struct msr_adamw_item {
     uint16_t *p;
@@ -187,8 +188,8 @@ int msr_adamw8bit_step(uint16_t *p, const uint16_t *g, void *state1, void *state
  * launch, split internally): equal, bit for bit, to one msr_adamw8bit_step(quantized = 1) per
  * item in order, with the same codebooks, block, hyperparameters and bias corrections.  Tensors
  * that the fast kernel does not take (other codebooks, blocks outside 64-512, unaligned
- * operands) run one launch each.  items: HOST array.  noise_mode: MSR_NOISE_TRITON or
- * MSR_NOISE_PHILOX8. */
+ * operands) run one launch each.  items: HOST array.  A list with an item that is refused is
+ * refused whole, before anything is launched.  noise_mode: MSR_NOISE_TRITON or MSR_NOISE_PHILOX8. */
 typedef struct msr_adam8_item {
     uint16_t *p;
     const uint16_t *g;
@@ -202,9 +203,9 @@ int msr_adamw8bit_multi(const msr_adam8_item *items, int32_t count, const float 
                         const void *qtable, int32_t block, float lr, float beta1, float beta2, float eps,
                         float weight_decay, float bc1, float bc2, int32_t noise_mode, msr_stream_t stream);
 
-/* Host only: *apart is 1 if no memory that a step of one of the two lists writes is touched by a
- * step of the other, so that the lists may be launched one after the other whatever the order of their
- * steps in the group; else 0.  block: the quantized list's. */
+/* Host only: *apart is 1 if every item of the two lists would be accepted and no memory that a step of
+ * one list writes is touched by a step of the other, so that the lists may be launched one after the other
+ * whatever the order of their steps in the group; else 0.  block: the quantized list's. */
 int msr_adamw8bit_apart(const msr_adam8_item *quantized, int32_t n_quantized, int32_t block,
                         const msr_adamw_item *bf16, int32_t n_bf16, int32_t *apart);
 
@@ -350,6 +351,8 @@ int msr_muon_fused_steps(const msr_muon_group *groups, int32_t n_groups, float b
  * TritonMuonSR's per-parameter steps make it (_triton_muon_step, muon_sr/triton_muon_sr.py:88-120),
  * with matrices of one Newton-Schulz shape sharing product launches.  Equal, bit for bit, to
  * those calls in order; matrices that share memory which one of them writes run one by one.
+ * A list with a matrix that is refused, or too large for the workspace, is refused whole, before
+ * anything is launched.
  * matrices: HOST array, any shapes.  The workspace is what msr_muon_each_workspace_bytes gives
  * for the same list: the largest of the shared launches', bounded by them at 2^27 elements (or by
  * one larger matrix).

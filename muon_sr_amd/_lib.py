@@ -107,6 +107,9 @@ SIGNATURES = {
     "msr_linear_wgrad_sr_accum": (ctypes.c_int, [_P, _P, _I64, _P, _I64, _I64, _I64, _I64, _U32, _I32, _I32, _P, _P]),
 }
 
+# MSR_ERR_ARG, _ALIGN and _OVERLAP: a call that returns one of these has launched nothing
+REFUSED = (1001, 1002, 1005)
+
 _lib = None
 _lock = threading.Lock()
 

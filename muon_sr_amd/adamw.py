@@ -23,39 +23,59 @@ def _seed(step: int, param_idx: int) -> int:
     return (step * 2654435761 ^ param_idx * 1234567891) & 0xFFFFFFFF
 
 
+def launch_list(launch, items, states, adding=None):
+    """``launch(items)`` (a library call's status) of steps whose ``state["step"]`` is already the new
+    one.  Where the library refuses the list, or memory for it runs out (nothing is launched then), the
+    items go one by one, as one launch per parameter would: the first that is refused ends them, and
+    the steps of the later ones, and of the state ``adding``, are taken back."""
+    try:
+        rc = launch(items)
+    except torch.OutOfMemoryError:
+        rc = None
+    if rc is not None and rc not in _lib.REFUSED:
+        return rc
+    done = k = 0
+    try:
+        for k, item in enumerate(items):
+            rc = launch([item])
+            if rc:
+                break
+        else:
+            done = 1
+    finally:
+        if not done:
+            for state in (*states[k + 1:], adding):
+                if state is not None:
+                    state["step"] -= 1
+    return rc
+
+
+def adamw_multi(items, form, centralization, hyper, stream):
+    return _lib.lib().msr_adamw_multi(b"".join(items), len(items), form, centralization, *hyper, _lib.noise_mode(), stream)
+
+
+pack_adamw_item = struct.Struct("=QQQQqffIi").pack   # msr_adamw_item
+
+
 class _AdamWBatch:
     """The bf16-moment AdamW steps of one parameter group, launched many tensors at a time
     (msr_adamw_multi; muon_sr/triton_adamw.py:75-114 launches one kernel per tensor).  Steps run
-    in the order they were added wherever they share memory.  ``form``: _lib.ADAMW, or
-    _lib.ADAMW_8BIT16 for the bf16-moment tensors of the 8-bit optimizer.
+    in the order they were added wherever they share memory.  ``form``: _lib.ADAMW or
+    _lib.ADAMW_CENTRALIZED.
 
     A caller adds in a ``try`` and flushes in its ``finally``, so that an error at one parameter
-    leaves the earlier ones stepped, as one launch per parameter would."""
+    leaves the earlier ones stepped and the later ones as they were, as one launch per parameter would."""
 
-    _PACK = struct.Struct("=QQQQqffIi").pack   # msr_adamw_item
     MAX_KEPT_BYTES = 256 << 20   # gradient copies (made contiguous, or centred) held until their launch
 
     def __init__(self, form, lr, beta1, beta2, eps, weight_decay, centralization=0.0):
         self.form, self.centralization, self.hyper = form, centralization, (lr, beta1, beta2, eps, weight_decay)
-        self.items, self.kept, self.kept_bytes, self.stream, self.device = [], [], 0, None, None
+        self.items, self.states, self.kept, self.kept_bytes, self.stream, self.device = [], [], [], 0, None, None
         self.step = None
 
-    def add(self, p, g, m, v, bc1, bc2, seed, copied=False, cols=0):
-        """One tensor's step; ``copied``: nothing but the batch holds ``g``; ``cols``: elements of a
-        row, with form ADAMW_CENTRALIZED."""
-        device = p.get_device()
-        if device != self.device:   # the device's current stream does not change within a step
-            self.flush()
-            self.device, self.stream = device, _lib.stream_of(p)
-        self.items.append(self._PACK(p.data_ptr(), g.data_ptr(), m.data_ptr(), v.data_ptr(), p.numel(), bc1, bc2, seed, cols))
-        if copied:
-            self.kept.append(g)
-            self.kept_bytes += g.numel() * g.element_size()
-            if self.kept_bytes >= self.MAX_KEPT_BYTES:
-                self.flush()
-
-    def add_adamw(self, p, g, ema, ema_sq, step, param_idx, copied=False, cols=0):
-        """The AdamW step of one tensor (muon_sr/triton_adamw.py:75-114).
+    def add(self, p, g, state, param_idx, copied=False, cols=0):
+        """The AdamW step of one tensor (muon_sr/triton_adamw.py:75-114).  ``copied``: nothing but
+        the batch holds ``g``; ``cols``: elements of a row, with form ADAMW_CENTRALIZED.
 
         Bias corrections are Python doubles, passed to the kernel as fp32 (as a compiled Triton
         launch passes Python floats); the tensors of a group nearly always share ``step``, so they
@@ -67,17 +87,30 @@ class _AdamWBatch:
             raise RuntimeError("TritonAdamW requires contiguous parameters")
         if not g.is_contiguous():
             g, copied = g.contiguous(), True
+        step = state["step"]
         if step != self.step:
             _, beta1, beta2, _, _ = self.hyper
             self.bc1, self.bc2, self.seed, self.step = 1.0 - beta1 ** step, (1.0 - beta2 ** step) ** 0.5, _seed(step, 0), step
-        self.add(p, g, ema, ema_sq, self.bc1, self.bc2, self.seed ^ param_idx * 1234567891 & 0xFFFFFFFF, copied, cols)
+        device = p.get_device()
+        if device != self.device:   # the device's current stream does not change within a step
+            self.flush(state)
+            self.device, self.stream = device, _lib.stream_of(p)
+        self.items.append(pack_adamw_item(p.data_ptr(), g.data_ptr(), state["ema"].data_ptr(), state["ema_squared"].data_ptr(),
+                                          p.numel(), self.bc1, self.bc2, self.seed ^ param_idx * 1234567891 & 0xFFFFFFFF, cols))
+        self.states.append(state)
+        if copied:
+            self.kept.append(g)
+            self.kept_bytes += g.numel() * g.element_size()
+            if self.kept_bytes >= self.MAX_KEPT_BYTES:
+                self.flush()
 
-    def flush(self):
+    def flush(self, adding=None):
+        """``adding``: the state of a tensor whose step has begun but is not in the batch."""
         if not self.items:
             return
-        items, self.items = self.items, []
-        rc = _lib.lib().msr_adamw_multi(b"".join(items), len(items), self.form, self.centralization, *self.hyper,
-                                        _lib.noise_mode(), self.stream)
+        items, self.items, states, self.states = self.items, [], self.states, []
+        rc = launch_list(lambda some: adamw_multi(some, self.form, self.centralization, self.hyper, self.stream),
+                         items, states, adding)
         self.kept, self.kept_bytes = [], 0
         _lib.check(rc, "msr_adamw_multi")
 
@@ -182,14 +215,13 @@ class TritonAdamW(Optimizer):
                 _lib.require_gpu(p, "TritonAdamW", RuntimeError)
                 cols = _fused_central_cols(p, grad, state["ema"], state["ema_squared"])
                 if cols:
-                    batch.flush()   # parameters may share memory: the two batches keep their order
-                    central.add_adamw(p, grad, state["ema"], state["ema_squared"], state["step"], group_offset + i, cols=cols)
+                    batch.flush(state)   # parameters may share memory: the two batches keep their order
+                    central.add(p, grad, state, group_offset + i, cols=cols)
                     continue
-                central.flush()
+                central.flush(state)
                 grad = centralize(grad, centralization)
 
-            batch.add_adamw(p, grad, state["ema"], state["ema_squared"], state["step"], group_offset + i,
-                            copied=centralization != 0)
+            batch.add(p, grad, state, group_offset + i, copied=centralization != 0)
 
 
 class _AccumQueue:

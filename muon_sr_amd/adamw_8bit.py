@@ -8,7 +8,6 @@ step runs fused gfx950 kernels over many tensors at a time (libmuon_sr_amd.so).
 from __future__ import annotations
 
 import ctypes
-import itertools
 import math
 import struct
 import weakref
@@ -17,7 +16,7 @@ import torch
 from torch.optim import Optimizer
 
 from . import _lib
-from .adamw import _AdamWBatch
+from .adamw import adamw_multi, launch_list, pack_adamw_item
 
 
 def create_dynamic_map(signed: bool = True) -> torch.Tensor:
@@ -98,76 +97,63 @@ class _Adam8Batch:
 
     def __init__(self, lr, beta1, beta2, eps, weight_decay):
         self.hyper = (lr, beta1, beta2, eps, weight_decay)
-        self.b16 = _AdamWBatch(_lib.ADAMW_8BIT16, *self.hyper)   # the pending bf16-moment steps
-        self.items, self.key = [], None                          # the pending quantized ones, and what they share
-        self.order = []                                          # whether each pending step, as added, is quantized
-        self.device = None
+        self.items, self.states = [], []   # (quantized, packed item) and state of the pending steps
+        self.key = None                    # what the pending quantized ones share
+        self.device, self.stream = None, None
 
     def add(self, p, g, state, seed):
         """One tensor's step with a state from ``init_8bit_state``."""
         n = state["step"]
         _, beta1, beta2, _, _ = self.hyper
         device = p.get_device()
-        if device != self.device:
-            self.flush()
-            self.device = device
+        if device != self.device:   # the device's current stream does not change within a step
+            self.flush(state)
+            self.device, self.stream = device, _lib.stream_of(p)
         if state["optim_bits"] != 8:
-            self.b16.add(p, g, state["state1"], state["state2"], 1 - beta1 ** n, 1 - beta2 ** n, seed)
-            self.order.append(False)
+            item = pack_adamw_item(p.data_ptr(), g.data_ptr(), state["state1"].data_ptr(), state["state2"].data_ptr(),
+                                   p.numel(), 1 - beta1 ** n, 1 - beta2 ** n, seed, 0)
+        else:
+            key = (state["qmap1"].data_ptr(), state["qmap2"].data_ptr(), quant_table(state), state["block_size"], n)
+            if key != self.key:
+                if self.key is not None:
+                    self.flush(state)
+                self.key = key
+            item = self._PACK(p.data_ptr(), g.data_ptr(), state["state1"].data_ptr(), state["state2"].data_ptr(),
+                              state["absmax1"].data_ptr(), state["absmax2"].data_ptr(), p.numel(), seed, 0)
+        self.items.append((state["optim_bits"] == 8, item))
+        self.states.append(state)
+
+    def _launch(self, items):
+        """The quantized items in one call and the others in another, where their order does not
+        matter; else refused."""
+        L = _lib.lib()
+        quantized, bf16 = [x for q, x in items if q], [x for q, x in items if not q]
+        rc = 0
+        if quantized and bf16:
+            apart = ctypes.c_int32(0)
+            rc = L.msr_adamw8bit_apart(b"".join(quantized), len(quantized), self.key[3], b"".join(bf16), len(bf16),
+                                       ctypes.byref(apart))
+            if rc or not apart.value:
+                return rc or _lib.REFUSED[0]
+        if quantized:
+            q1, q2, qt, block, n = self.key
+            lr, beta1, beta2, eps, weight_decay = self.hyper
+            rc = L.msr_adamw8bit_multi(b"".join(quantized), len(quantized), q1, q2, qt, block, lr, beta1, beta2, eps,
+                                       weight_decay, 1 - beta1 ** n, 1 - beta2 ** n, _lib.noise_mode(), self.stream)
+        if bf16 and not rc:
+            rc = adamw_multi(bf16, _lib.ADAMW_8BIT16, 0.0, self.hyper, self.stream)
+            if quantized:   # accepted by msr_adamw8bit_apart: an error here is no refusal of the whole
+                _lib.check(rc, "msr_adamw_multi")
+        return rc
+
+    def flush(self, adding=None):
+        """``adding``: the state of a tensor whose step has begun but is not in the batch."""
+        if not self.items:
             return
-        # what the tensors of a launch share
-        key = (state["qmap1"].data_ptr(), state["qmap2"].data_ptr(), quant_table(state), state["block_size"], n,
-               _lib.stream_of(p))
-        if key != self.key:
-            self._flush8()
-            self.key = key
-        self.items.append(self._PACK(p.data_ptr(), g.data_ptr(), state["state1"].data_ptr(), state["state2"].data_ptr(),
-                                     state["absmax1"].data_ptr(), state["absmax2"].data_ptr(), p.numel(), seed, 0))
-        self.order.append(True)
-
-    def _launch8(self, items):
-        q1, q2, qt, block, n, stream = self.key
-        lr, beta1, beta2, eps, weight_decay = self.hyper
-        rc = _lib.lib().msr_adamw8bit_multi(b"".join(items), len(items), q1, q2, qt, block, lr, beta1, beta2, eps,
-                                            weight_decay, 1 - beta1 ** n, 1 - beta2 ** n, _lib.noise_mode(), stream)
-        _lib.check(rc, "msr_adamw8bit_multi")
-
-    def _apart(self):
-        """Whether no pending step of one kind touches memory that one of the other kind writes."""
-        apart = ctypes.c_int32(0)
-        _lib.check(_lib.lib().msr_adamw8bit_apart(b"".join(self.items), len(self.items), self.key[3],
-                                                  b"".join(self.b16.items), len(self.b16.items), ctypes.byref(apart)),
-                   "msr_adamw8bit_apart")
-        return apart.value != 0
-
-    def _flush8(self):
-        """Launches the pending quantized steps; the bf16-moment ones stay pending where they may."""
-        items, order = self.items, self.order
-        if not items:
-            return
-        if not self.b16.items or self._apart():
-            self.items, self.order = [], [False] * len(self.b16.items)
-            self._launch8(items)
-            return
-        self.items, self.order = [], []
-        items16, self.b16.items = self.b16.items, []
-        at8 = at16 = 0
-        for quantized, run in itertools.groupby(order):   # runs of one kind, as added
-            n = sum(1 for _ in run)
-            if quantized:
-                self._launch8(items[at8:at8 + n])
-                at8 += n
-            else:
-                self.b16.items = items16[at16:at16 + n]
-                self.b16.flush()
-                at16 += n
-
-    def flush(self):
-        try:
-            self._flush8()
-        finally:
-            self.b16.flush()
-            self.order = []
+        items, self.items, states, self.states = self.items, [], self.states, []
+        rc = launch_list(self._launch, items, states, adding)
+        self.key = None
+        _lib.check(rc, "the 8-bit AdamW step")
 
 
 def adamw8bit_launch(p, g, state, lr, beta1, beta2, eps, weight_decay, seed):

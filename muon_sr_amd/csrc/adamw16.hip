@@ -385,7 +385,7 @@ static bool items_conflict(const msr_adamw_item *items, int32_t count) {
 }
 
 // Every item's own operands distinct (or the same buffer, updated in place).
-static int check_item(const msr_adamw_item &x, const char *name, int32_t i) {
+int check_item(const msr_adamw_item &x, const char *name, int32_t i) {
     if (x.n < 0 || (x.n > 0 && (!x.p || !x.g || !x.m || !x.v))) {
         set_error("%s: bad arguments in item %d", name, (int)i);
         return MSR_ERR_ARG;

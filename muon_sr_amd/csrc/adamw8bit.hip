@@ -1000,6 +1000,11 @@ int msr_adamw8bit_apart(const msr_adam8_item *quantized, int32_t n_quantized, in
         set_error("msr_adamw8bit_apart: bad arguments");
         return MSR_ERR_ARG;
     }
+    *apart = 0;
+    for (int32_t i = 0; i < n_quantized; ++i)
+        if (check_item8(quantized[i], block, "msr_adamw8bit_apart", i)) return MSR_OK;
+    for (int32_t i = 0; i < n_bf16; ++i)
+        if (check_item(bf16[i], "msr_adamw8bit_apart", i)) return MSR_OK;
     try {
         std::vector<ItemRange> r(6 * (size_t)n_quantized + 4 * (size_t)n_bf16);
         size_t n = 0;

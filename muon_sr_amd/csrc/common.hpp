@@ -494,7 +494,9 @@ inline bool ranges_conflict(ItemRange *r, int n) {
             if (r[i].item != r[j].item && (r[i].write || r[j].write)) return true;
     return false;
 }
-// The memory of a bf16-moment AdamW item: 4 ranges, marked `id` (adamw16.hip).
+// What a bf16-moment AdamW step refuses (MSR_OK if nothing), and the memory of an item: 4 ranges,
+// marked `id` (adamw16.hip).
+int check_item(const msr_adamw_item &x, const char *name, int32_t i);
 void item_ranges(const msr_adamw_item &x, int32_t id, ItemRange *r);
 
 // Grid size for a grid-stride loop over `work` items with `threads` per block.

@@ -2149,22 +2149,27 @@ static int each_check(const msr_muon_matrix *x, int32_t count, const char *name)
     return MSR_OK;
 }
 
-static int each_run(const msr_muon_matrix *x, const std::vector<int32_t> &run, float beta, bool nesterov, int32_t steps,
-                    float a, float b, float c, float lr, float wd, int32_t mode, void *ws, size_t ws_bytes, hipStream_t s) {
+// One run of each_runs, ready to launch.
+struct EachRun {
+    NSLayout L;
+    std::vector<const void *> grads;
+    std::vector<uint16_t *> bufs, params;
+    std::vector<uint32_t> pseeds, aseeds;
+    std::vector<NSPrepare> pps;
+    std::vector<NSApply> aps;
+    std::vector<NSPart> parts;
+};
+
+static EachRun each_build(const msr_muon_matrix *x, const std::vector<int32_t> &run, float beta, bool nesterov, float lr,
+                          float wd, int32_t mode, void *ws) {
     const int64_t n = (int64_t)run.size();
     const msr_muon_matrix &x0 = x[run[0]];
-    const NSLayout L = ns_layout(n, std::min(x0.rows, x0.cols), std::max(x0.rows, x0.cols));
-    if (!ws || ws_bytes < L.total) {
-        set_error("msr_muon_each: workspace of %zu bytes is smaller than the %zu required", ws_bytes, L.total);
-        return MSR_ERR_WORKSPACE;
-    }
-    std::vector<const void *> grads((size_t)n);
-    std::vector<uint16_t *> bufs((size_t)n), params((size_t)n);
-    std::vector<uint32_t> pseeds((size_t)n), aseeds((size_t)n);
-    for (int64_t i = 0; i < n; ++i) {
-        const msr_muon_matrix &m = x[run[i]];
-        grads[i] = m.grad; bufs[i] = m.buf; params[i] = m.param;
-        pseeds[i] = m.prepare_seed; aseeds[i] = m.apply_seed;
+    EachRun r;
+    r.L = ns_layout(n, std::min(x0.rows, x0.cols), std::max(x0.rows, x0.cols));
+    for (const int32_t i : run) {
+        const msr_muon_matrix &m = x[i];
+        r.grads.push_back(m.grad); r.bufs.push_back(m.buf); r.params.push_back(m.param);
+        r.pseeds.push_back(m.prepare_seed); r.aseeds.push_back(m.apply_seed);
     }
     // parts: wide and tall, bf16 and fp32 gradients, and what scales the matrices have
     auto same = [](const msr_muon_matrix &u, const msr_muon_matrix &v) {
@@ -2174,20 +2179,20 @@ static int each_run(const msr_muon_matrix *x, const std::vector<int32_t> &run, f
     std::vector<int64_t> cut;
     for (int64_t i = 0; i < n; ++i)
         if (i == 0 || !same(x[run[i - 1]], x[run[i]])) cut.push_back(i);
-    const int np = (int)cut.size();
+    const size_t np = cut.size();
     cut.push_back(n);
-    std::vector<NSPrepare> pps((size_t)np);
-    std::vector<NSApply> aps((size_t)np);
-    std::vector<NSPart> parts((size_t)np);
-    for (int k = 0; k < np; ++k) {
+    r.pps.resize(np);
+    r.aps.resize(np);
+    r.parts.resize(np);
+    for (size_t k = 0; k < np; ++k) {
         const int64_t i = cut[k];
         const msr_muon_matrix &m = x[run[i]];
-        pps[k] = NSPrepare{&grads[i], m.grad_f32 != 0, nullptr, 0, 0u, &bufs[i], &pseeds[i], beta, nesterov, nullptr, (int)mode};
-        aps[k] = NSApply{&params[i], &aseeds[i], lr, wd, m.scale, (int)mode, nullptr};
+        r.pps[k] = NSPrepare{&r.grads[i], m.grad_f32 != 0, nullptr, 0, 0u, &r.bufs[i], &r.pseeds[i], beta, nesterov, nullptr, (int)mode};
+        r.aps[k] = NSApply{&r.params[i], &r.aseeds[i], lr, wd, m.scale, (int)mode, nullptr};
         // the last product's store writes the parameters: `out` only marks the layout (never accessed)
-        parts[k] = NSPart{i, cut[k + 1] - i, m.rows, m.cols, nullptr, static_cast<uint16_t *>(ws), &aps[k], &pps[k]};
+        r.parts[k] = NSPart{i, cut[k + 1] - i, m.rows, m.cols, nullptr, static_cast<uint16_t *>(ws), &r.aps[k], &r.pps[k]};
     }
-    return ns_run_parts(parts.data(), np, n, steps, a, b, c, ws, L, s);
+    return r;
 }
 
 extern "C" {
@@ -2219,6 +2224,7 @@ int msr_muon_each(const msr_muon_matrix *matrices, int32_t count, float beta, in
     }
     if (count == 0) return MSR_OK;
     hipStream_t s = (hipStream_t)stream;
+    std::vector<EachRun> ready;
     try {
         // a matrix's own operands and the workspace must not overlap; matrices that share
         // memory which one of them writes run one after the other, in order
@@ -2246,14 +2252,23 @@ int msr_muon_each(const msr_muon_matrix *matrices, int32_t count, float beta, in
         } else {
             runs = each_runs(matrices, count);
         }
-        for (const auto &run : runs)
-            if ((rc = each_run(matrices, run, beta, nesterov != 0, steps, a_coef, b_coef, c_coef, lr, weight_decay, noise_mode,
-                               workspace, workspace_bytes, s)))
-                return rc;
+        ready.reserve(runs.size());
+        for (const auto &run : runs) {
+            ready.push_back(each_build(matrices, run, beta, nesterov != 0, lr, weight_decay, noise_mode, workspace));
+            if (!workspace || workspace_bytes < ready.back().L.total) {
+                set_error("msr_muon_each: workspace of %zu bytes is smaller than the %zu required", workspace_bytes,
+                          ready.back().L.total);
+                return MSR_ERR_WORKSPACE;
+            }
+        }
     } catch (const std::bad_alloc &) {
         set_error("msr_muon_each: out of host memory");
         return MSR_ERR_ARG;
     }
+    for (const EachRun &r : ready)   // nothing is refused from here on
+        if ((rc = ns_run_parts(r.parts.data(), (int)r.parts.size(), (int64_t)r.grads.size(), steps, a_coef, b_coef, c_coef,
+                               workspace, r.L, s)))
+            return rc;
     return MSR_OK;
 }
 

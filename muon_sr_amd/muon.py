@@ -32,7 +32,7 @@ import torch
 from torch.optim import Optimizer
 
 from . import _lib
-from .adamw import _AdamWBatch
+from .adamw import _AdamWBatch, launch_list
 from .adamw_8bit import _Adam8Batch, init_8bit_state, split_8bit_state, TritonAdamW8bit
 
 NS_COEFFS = (3.4445, -4.7750, 2.0315)
@@ -301,27 +301,30 @@ class _MuonEach:
     (_triton_muon_step, muon_sr/triton_muon_sr.py:116-120).
 
     A caller adds in a ``try`` and flushes in its ``finally``, so that an error at one parameter
-    leaves the earlier ones stepped, as one step per parameter would."""
+    leaves the earlier ones stepped and the later ones as they were, as one step per parameter would."""
 
     _PACK = struct.Struct("=QQQqqIIif").pack   # msr_muon_matrix
     MAX_KEPT_BYTES = 256 << 20   # gradient copies (made contiguous or fp32) held until their launch
 
     def __init__(self, beta, nesterov, ns_steps, lr, weight_decay):
         self.beta, self.nesterov, self.ns_steps, self.lr, self.weight_decay = beta, nesterov, ns_steps, lr, weight_decay
-        self.items, self.kept, self.kept_bytes, self.device, self.stream = [], [], 0, None, None
+        self.items, self.states, self.kept, self.kept_bytes, self.device, self.stream = [], [], [], 0, None, None
 
-    def add(self, p, buf, step, param_idx):
+    def add(self, p, buf, step, param_idx, state=None):
+        """``state``: where the parameter's own step is counted, if it has one."""
         grad = _grad_operand(p.grad)
         seeds = [_deterministic_seed(step, param_idx, salt=salt) for salt in (0, 1)]
         if p.dim() != 2 or self.ns_steps < 1 or not p.numel():
+            self.flush(state)   # parameters may share memory: keep the order
             self._alone(p, grad, buf, *seeds)
             return
         device, stream = p.device, _lib.stream_of(p)
         if self.items and (device != self.device or stream != self.stream):
-            self.flush()
+            self.flush(state)
         self.device, self.stream = device, stream
         self.items.append(self._PACK(grad.data_ptr(), buf.data_ptr(), p.data_ptr(), *p.shape, *seeds,
                                      grad.dtype == torch.float32, _ns_scale(p.shape)))
+        self.states.append(state)
         if grad is not p.grad:
             self.kept.append(grad)
             self.kept_bytes += grad.numel() * grad.element_size()
@@ -330,7 +333,6 @@ class _MuonEach:
 
     def _alone(self, p, grad, buf, prepare_seed, apply_seed):
         """Parameters of more than 2 dims, and ns_steps = 0."""
-        self.flush()   # parameters may share memory: keep the order
         if p.dim() == 2 and self.ns_steps >= 1:   # an empty matrix, which the library refuses
             _fused_step([grad], buf, 0, [p.data], self.beta, self.nesterov, prepare_seed, self.ns_steps, self.lr,
                         self.weight_decay, 1.0, [apply_seed])
@@ -343,27 +345,23 @@ class _MuonEach:
         L = _lib.lib()
         arr, n = b"".join(items), len(items)
         nbytes = _lib.ctypes.c_size_t(0)
-        _lib.check(L.msr_muon_each_workspace_bytes(arr, n, _lib.ctypes.byref(nbytes)), "msr_muon_each_workspace_bytes")
-        try:
-            ws = torch.empty(nbytes.value, dtype=torch.uint8, device=self.device)
-        except torch.OutOfMemoryError:
-            if n == 1:
-                raise
-            for item in items:   # one by one, each with its own smaller workspace
-                self._launch([item])
-            return
-        rc = L.msr_muon_each(arr, n, self.beta, int(bool(self.nesterov)), self.ns_steps, *NS_COEFFS, self.lr,
-                             self.weight_decay, _lib.noise_mode(), ws.data_ptr(), nbytes.value, self.stream)
-        _lib.check(rc, "msr_muon_each")
+        rc = L.msr_muon_each_workspace_bytes(arr, n, _lib.ctypes.byref(nbytes))
+        if rc:
+            return rc
+        ws = torch.empty(nbytes.value, dtype=torch.uint8, device=self.device)   # one item's is smaller, if memory runs out
+        return L.msr_muon_each(arr, n, self.beta, int(bool(self.nesterov)), self.ns_steps, *NS_COEFFS, self.lr,
+                               self.weight_decay, _lib.noise_mode(), ws.data_ptr(), nbytes.value, self.stream)
 
-    def flush(self):
+    def flush(self, adding=None):
+        """``adding``: the state of a parameter whose step has begun but is not in the list."""
         if not self.items:
             return
-        items, self.items = self.items, []
+        items, self.items, states, self.states = self.items, [], self.states, []
         try:
-            self._launch(items)
+            rc = launch_list(self._launch, items, states, adding)
         finally:
             self.kept, self.kept_bytes = [], 0
+        _lib.check(rc, "msr_muon_each")
 
 
 def _muon_batch_step(shape_groups, stacked_bufs, buf_indices, beta, nesterov, ns_steps, lr, weight_decay, step):
@@ -482,7 +480,7 @@ def _muon_each_step(params, states, each, name):
             state["step"] = 0
             state["momentum_buffer"] = torch.zeros_like(p, dtype=torch.bfloat16, memory_format=torch.contiguous_format)
         state["step"] += 1
-        each.add(p, state["momentum_buffer"], state["step"], param_idx)
+        each.add(p, state["momentum_buffer"], state["step"], param_idx, state)
 
 
 class _StackedBufsMixin:
@@ -680,7 +678,7 @@ class TritonMuonSRWithAuxAdam(_StackedBufsMixin, Optimizer):
                 state["ema"] = torch.zeros_like(p, dtype=torch.bfloat16, memory_format=torch.contiguous_format)
                 state["ema_squared"] = torch.zeros_like(p, dtype=torch.bfloat16, memory_format=torch.contiguous_format)
             state["step"] += 1
-            batch.add_adamw(p, p.grad, state["ema"], state["ema_squared"], state["step"], group_offset + i)
+            batch.add(p, p.grad, state, group_offset + i)
 
     def load_state_dict(self, state_dict):
         """As torch's, except that the states of ``optim_bits=8`` AdamW groups keep
