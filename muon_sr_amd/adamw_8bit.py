@@ -163,6 +163,32 @@ def adamw8bit_launch(p, g, state, lr, beta1, beta2, eps, weight_decay, seed):
     batch.flush()
 
 
+def _device_maps(maps, device):
+    """The standard codebooks that an optimizer's states on ``device`` share (``maps``: its pairs)."""
+    if device not in maps:
+        maps[device] = tuple(m.to(device, copy=True) for m in _standard_maps())
+    return maps[device]
+
+
+def _shared_codebooks(maps):
+    """share(device, qmap1, qmap2) -> a pair on ``device`` with these bits, the same tensors for
+    every state that has them (the optimizer's own pair for the standard ones): steps of one launch share
+    their codebooks, and a copy per state would mean a launch per tensor."""
+    known = {}   # device -> [(bits of qmap1, bits of qmap2, pair)]
+
+    def share(device, *pair):
+        if device not in known:
+            known[device] = [(*(m.view(torch.int32) for m in _standard_maps()), _device_maps(maps, device))]
+        bits = [q.detach().cpu().contiguous().view(torch.int32) for q in pair]
+        for b1, b2, shared in known[device]:
+            if torch.equal(bits[0], b1) and torch.equal(bits[1], b2):
+                return shared
+        shared = tuple(q.to(device).clone(memory_format=torch.contiguous_format) for q in pair)
+        known[device].append((bits[0].clone(), bits[1].clone(), shared))
+        return shared
+    return share
+
+
 def init_8bit_state(p, block_size, optim_bits, min_8bit_size, maps):
     """State of one tensor (muon_sr/triton_adamw_8bit.py:152-165)."""
     bits = 16 if p.numel() < min_8bit_size else optim_bits
@@ -171,9 +197,7 @@ def init_8bit_state(p, block_size, optim_bits, min_8bit_size, maps):
     state.update(state1=torch.zeros_like(p, dtype=dtype, memory_format=torch.contiguous_format),
                  state2=torch.zeros_like(p, dtype=dtype, memory_format=torch.contiguous_format))
     if bits == 8:
-        if p.device not in maps:
-            maps[p.device] = (create_dynamic_map(True).to(p.device), create_dynamic_map(False).to(p.device))
-        state["qmap1"], state["qmap2"] = maps[p.device]
+        state["qmap1"], state["qmap2"] = _device_maps(maps, p.device)
         blocks = _cdiv(p.numel(), block_size)
         state["absmax1"] = torch.zeros(blocks, device=p.device, dtype=torch.float32)
         state["absmax2"] = torch.zeros_like(state["absmax1"])
@@ -184,7 +208,7 @@ def init_8bit_state(p, block_size, optim_bits, min_8bit_size, maps):
 _QUANT_KEYS = ("state1", "state2", "qmap1", "qmap2", "absmax1", "absmax2")
 
 
-def split_8bit_state(state_dict, param_groups, is_8bit_group):
+def split_8bit_state(state_dict, param_groups, is_8bit_group, maps):
     """Take the 8-bit states of a checkpoint out of torch's Optimizer.load_state_dict,
     which would cast every floating-point state tensor to the parameter's dtype
     (fp32 block scales and codebooks to bf16).
@@ -194,10 +218,12 @@ def split_8bit_state(state_dict, param_groups, is_8bit_group):
     and the group's block size and bits (the errors of
     muon_sr/triton_adamw_8bit.py:219-236).  Returns (the state dict without those
     tensors, restore), where ``restore(optimizer.state)`` puts copies back on each
-    parameter's device after torch has loaded the rest."""
+    parameter's device after torch has loaded the rest.  Equal codebooks come back as one pair per
+    device, as a new optimizer's states have them (``maps``: the optimizer's pairs)."""
     groups = state_dict["param_groups"]
     mapping = dict(zip([i for g in groups for i in g["params"]], [p for g in param_groups for p in g["params"]]))
     restored = {}
+    share = _shared_codebooks(maps)
     for group in groups:
         if not is_8bit_group(group):
             continue
@@ -220,8 +246,11 @@ def split_8bit_state(state_dict, param_groups, is_8bit_group):
                 value = state[key]
                 if value.dtype != dtype or tuple(value.shape) != tuple(shape):
                     raise ValueError(f"Invalid checkpoint state: {key}")
-                restored[ident][key] = value.to(device=p.device, dtype=dtype).clone(
-                    memory_format=torch.contiguous_format)
+                if key not in ("qmap1", "qmap2"):
+                    restored[ident][key] = value.to(device=p.device, dtype=dtype).clone(
+                        memory_format=torch.contiguous_format)
+            if bits == 8:
+                restored[ident]["qmap1"], restored[ident]["qmap2"] = share(p.device, state["qmap1"], state["qmap2"])
     stripped = dict(state_dict, state={i: ({k: v for k, v in st.items() if k not in _QUANT_KEYS}
                                            if i in restored else st)
                                        for i, st in state_dict["state"].items()})
@@ -336,6 +365,7 @@ class TritonAdamW8bit(Optimizer):
             raise ValueError("Checkpoint parameter groups do not match optimizer")
         for group in groups:
             self._validate_group(group)
-        stripped, restore = split_8bit_state(state_dict, self.param_groups, lambda group: True)
+        stripped, restore = split_8bit_state(state_dict, self.param_groups, lambda group: True,
+                                             self.__dict__.setdefault("_maps", {}))   # a copied optimizer has none
         super().load_state_dict(stripped)
         restore(self.state)

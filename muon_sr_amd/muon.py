@@ -688,7 +688,8 @@ class TritonMuonSRWithAuxAdam(_StackedBufsMixin, Optimizer):
             raise ValueError("loaded state dict has a different number of parameter groups")
         stripped, restore = split_8bit_state(
             state_dict, self.param_groups,
-            lambda group: not group.get("use_muon", False) and group.get("optim_bits", 16) == 8)
+            lambda group: not group.get("use_muon", False) and group.get("optim_bits", 16) == 8,
+            self.__dict__.setdefault("_maps", {}))   # a copied optimizer has none
         super().load_state_dict(stripped)
         restore(self.state)
 

@@ -157,3 +157,50 @@ def test_apart_checks_the_items():
         assert L.msr_adamw8bit_apart(q, 1, 256, b, 1, ctypes.byref(apart)) == 0
         assert apart.value == want, (p, g, n)
     assert L.msr_adamw8bit_apart(q, 1, 0, None, 0, ctypes.byref(apart)) == 1001
+
+
+@pytest.mark.parametrize("which", ["8bit", "hybrid"])
+def test_loaded_states_share_launches(rec, which):
+    """After load_state_dict the quantized tensors take one launch, as a new optimizer's do: states whose
+    codebooks have the same bits share one pair, beside parameters whose state begins later, and
+    other codebooks keep theirs."""
+    import copy
+    from muon_sr_amd import TritonAdamW8bit, TritonMuonSRWithAuxAdam
+    ps = [torch.nn.Parameter(torch.zeros(64, 96, dtype=torch.bfloat16)) for _ in range(6)]
+
+    def make():
+        if which == "8bit":
+            return TritonAdamW8bit(ps, lr=1e-3)
+        return TritonMuonSRWithAuxAdam([dict(params=ps, use_muon=False, optim_bits=8)])
+
+    def launches(opt):
+        rec.calls.clear()
+        batch = _Adam8Batch(1e-3, 0.9, 0.99, 1e-8, 0.0)
+        kept = []
+        for p in ps:
+            state = opt.state[p] or opt.state[p].update(init_8bit_state(p, 256, 8, 4096, opt._maps)) or opt.state[p]
+            state["step"] = 3
+            kept.append(torch.zeros_like(p))
+            batch.add(p, kept[-1], state, 7)
+        batch.flush()
+        return [len(items) for _, items in rec.calls]
+
+    opt = make()
+    assert launches(opt) == [6]
+    saved = copy.deepcopy(opt.state_dict())
+    for st in saved["state"].values():   # a pair per state, as an earlier load made them
+        st["qmap1"], st["qmap2"] = st["qmap1"].clone(), st["qmap2"].clone()
+    del saved["state"][2]                # a parameter that had no gradient yet
+    opt = make()
+    opt.load_state_dict(saved)
+    assert launches(opt) == [6]
+    opt = copy.deepcopy(make())
+    opt.load_state_dict(saved)
+    saved["state"][4]["qmap1"][3] += 1e-3
+    saved["state"][5]["qmap1"][3] += 1e-3
+    opt = make()
+    opt.load_state_dict(saved)
+    assert launches(opt) == [4, 2]
+    for i, st in saved["state"].items():
+        for key in ("qmap1", "qmap2"):
+            assert torch.equal(opt.state[ps[i]][key], st[key]) and opt.state[ps[i]][key].data_ptr() != st[key].data_ptr()
