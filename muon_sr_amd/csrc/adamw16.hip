@@ -77,11 +77,12 @@ __device__ __forceinline__ A16Consts a16_consts(const A16Args &a, const A16Item 
     return c;
 }
 
-// One group of 8 elements: p, m, v updated in place in their packed words.
+// One group of 8 elements: p, m, v updated in place in their packed words.  active: the lane's
+// values count for the choice of the branch.
 template <int MODE, int FORM>
 __device__ __forceinline__ void a16_group(const A16Consts &c, const Noise (&ns)[3], int64_t o0, int valid,
                                           uint32_t (&wp)[4], const uint32_t (&wg)[4], uint32_t (&wm)[4],
-                                          uint32_t (&wv)[4]) {
+                                          uint32_t (&wv)[4], bool active = true) {
     float p[8], g[8], m[8], v[8];
     unpack8(wp, p); unpack8(wg, g); unpack8(wm, m); unpack8(wv, v);
     // new moments; extremes of 2 bits(|m'|) and bits(v') (unsigned: NaN, infinities and negative v'
@@ -102,7 +103,7 @@ __device__ __forceinline__ void a16_group(const A16Consts &c, const Noise (&ns)[
     const bool ok = c.fast && vmax <= 0x4b800000u && tmax < (0x53800000u << 1) && (tmin >> 1) >= c.mmin;
     uint32_t r[8];
     uint32_t om[8], ov[8], op[8];
-    const bool exact = __builtin_amdgcn_ballot_w64(!ok) != 0;
+    const bool exact = __builtin_amdgcn_ballot_w64(active && !ok) != 0;
     if (!exact) {
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
@@ -229,21 +230,33 @@ template <int MODE, int G>
 __device__ __forceinline__ void a16_rows(const A16Args &a, const A16Item &it, int cols, int64_t row0, float *red) {
     const int tpr = a16_tpr(cols), groups = cols >> 3;
     const int lr = threadIdx.x & (tpr - 1);
-    const int64_t base = (row0 + threadIdx.x / tpr) * cols;
+    const int64_t base0 = row0 * cols, base = base0 + (int64_t)(threadIdx.x / tpr) * cols;
+    // Lanes without elements load and store nothing and have no say in the choice of the branch.  One
+    // group: they compute on whatever their registers hold.  Two: their loads are out of the buffer
+    // resource's range and give 0.  Against loads of the tensor's first group in their place, which its
+    // owner stores meanwhile (us before, now): 128256 x 4096 1260, 1258 (with the form of one group
+    // 1284); 400000 x 1000 1040, 1043; 400000 x 520 686, 695; 128256 x 2048 596, 620 on one box and
+    // 588, 588 on another.
     bool in[G];
-    int64_t at[G];   // lanes without elements compute on the tensor's first group and store nothing
+    int64_t at[G];
     uint32_t wp[G][4], wg[G][4], wm[G][4], wv[G][4];
+    auto load = [&](const uint16_t *t, int u, uint32_t (&w)[4]) __attribute__((always_inline)) {
+        if constexpr (G == 1) {
+            asm volatile("" : "=v"(w[0]), "=v"(w[1]), "=v"(w[2]), "=v"(w[3]));
+            if (in[u]) load_bf16x8<true>(t, at[u], 8, w);
+        } else {
+            const u32x4_t x = ldu_nt4(t + base0, in[u] ? (uint32_t)((at[u] - base0) * 2) : LDU_NONE);
+            w[0] = x.x; w[1] = x.y; w[2] = x.z; w[3] = x.w;
+        }
+    };
 #pragma unroll
     for (int u = 0; u < G; ++u) {
         in[u] = base < it.n && lr + u * tpr < groups;
-        at[u] = in[u] ? base + (int64_t)(lr + u * tpr) * 8 : 0;
-        load_bf16x8<true>(it.g, at[u], 8, wg[u]);
-    }
-#pragma unroll
-    for (int u = 0; u < G; ++u) {
-        load_bf16x8<true>(it.p, at[u], 8, wp[u]);
-        load_bf16x8<true>(it.m, at[u], 8, wm[u]);
-        load_bf16x8<true>(it.v, at[u], 8, wv[u]);
+        at[u] = base + (int64_t)(lr + u * tpr) * 8;
+        load(it.g, u, wg[u]);
+        load(it.p, u, wp[u]);
+        load(it.m, u, wm[u]);
+        load(it.v, u, wv[u]);
     }
     float s = 0.0f;
 #pragma unroll
@@ -279,7 +292,7 @@ __device__ __forceinline__ void a16_rows(const A16Args &a, const A16Item &it, in
     for (int u = 0; u < G; ++u) {
 #pragma unroll
         for (int k = 0; k < 4; ++k) wg[u][k] = rne_bf16x2(bf16_lo(wg[u][k]) - mean, bf16_hi(wg[u][k]) - mean);
-        a16_group<MODE, A16_ADAMW>(c, ns, at[u], 8, wp[u], wg[u], wm[u], wv[u]);
+        a16_group<MODE, A16_ADAMW>(c, ns, at[u], 8, wp[u], wg[u], wm[u], wv[u], G > 1 || in[u]);
         if (in[u]) {
             store_bf16x8<true>(it.m, at[u], 8, wm[u]);
             store_bf16x8<true>(it.v, at[u], 8, wv[u]);
@@ -288,8 +301,10 @@ __device__ __forceinline__ void a16_rows(const A16Args &a, const A16Item &it, in
     }
 }
 
+// Two groups: 4 waves per SIMD (128256 x 4096, on one box: 1272 us; left to the compiler, 5 waves and 1311).
 template <int MODE, int G>
-__global__ __launch_bounds__(CEN_THREADS) void adamw16_central_kernel(A16Args a) {
+__global__ __launch_bounds__(CEN_THREADS) __attribute__((amdgpu_waves_per_eu(G == 2 ? 4 : 1, G == 2 ? 4 : 8)))
+void adamw16_central_kernel(A16Args a) {
     __shared__ float red[CEN_THREADS];
     const int32_t total = a.tstart[a.count];
     for (int64_t tile = blockIdx.x; tile < total; tile += gridDim.x) {

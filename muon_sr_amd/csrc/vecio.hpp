@@ -29,7 +29,9 @@ __device__ __forceinline__ void st_nt2(void *p, u32x2_t v) { __builtin_nontempor
 // Non-temporal accesses at a wave-uniform base plus a per-lane byte offset, through a
 // buffer resource made from the base (scalar instructions): the 64-bit address
 // arithmetic of the global forms stays off the VALU.  `ubase` must be the same in
-// every lane; the offset is below 2^31.  aux 2 = nt.
+// every lane; the offset is below 2^31 - 16, or LDU_NONE for a load that reads 0 (out of the
+// resource's range: no access).  aux 2 = nt.
+constexpr uint32_t LDU_NONE = 0x80000000u;
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t uniform_rsrc(const void *ubase) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(ubase), (short)0, 0x7fffffff, 0x00020000);
 }
