@@ -354,8 +354,8 @@ int msr_muon_fused_steps(const msr_muon_group *groups, int32_t n_groups, float b
  * A list with a matrix that is refused, or too large for the workspace, is refused whole, before
  * anything is launched.
  * matrices: HOST array, any shapes.  The workspace is what msr_muon_each_workspace_bytes gives
- * for the same list: the largest of the shared launches', bounded by them at 2^27 elements (or by
- * one larger matrix).
+ * for the same list: the largest of the shared launches', bounded by them at 2^27 elements, each
+ * matrix padded to multiples of 256 (or by one larger matrix): about 1 GiB.
  * ------------------------------------------------------------------------- */
 typedef struct msr_muon_matrix {
     const void *grad;              /* bf16, or fp32 with grad_f32 */

@@ -2108,9 +2108,10 @@ int msr_muon_fused_steps(const msr_muon_group *groups, int32_t n_groups, float b
 // Matrices of their own (msr_muon_each)
 // ---------------------------------------------------------------------------
 
-// Elements of the matrices that share a call's product launches: enough for 2048 x 2048 ones to
-// fill the chip many times over (32), while a 4096 x 14336 one, which fills it by itself, is
-// nearly alone; it bounds the workspace at about 1 GiB.
+// Elements, padded to multiples of 256 as the workspace is, of the matrices that share a call's
+// product launches: enough for 2048 x 2048 ones to fill the chip many times over (32), while a
+// 4096 x 14336 one, which fills it by itself, is nearly alone; it bounds the workspace at about 1 GiB
+// (counted unpadded, 1000 matrices of 16 x 4096 took 4.2 GiB).
 constexpr int64_t EACH_NUMEL = int64_t(1) << 27;
 
 // The calls of a list of matrices: indices, grouped by Newton-Schulz shape (a tall matrix has the
@@ -2129,7 +2130,7 @@ static std::vector<std::vector<int32_t>> each_runs(const msr_muon_matrix *x, int
         size_t e = i;
         auto shape = [&](int32_t k) { return std::make_pair(std::min(x[k].rows, x[k].cols), std::max(x[k].rows, x[k].cols)); };
         while (e < order.size() && shape(order[e]) == shape(order[i])) ++e;
-        const int64_t numel = x[order[i]].rows * x[order[i]].cols, n = (int64_t)(e - i);
+        const int64_t numel = round_up(x[order[i]].rows, 256) * round_up(x[order[i]].cols, 256), n = (int64_t)(e - i);
         const int64_t most = std::max<int64_t>(1, EACH_NUMEL / numel), pieces = (n + most - 1) / most;
         for (int64_t k = 0; k < pieces; ++k)
             runs.emplace_back(order.begin() + i + n * k / pieces, order.begin() + i + n * (k + 1) / pieces);

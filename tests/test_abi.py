@@ -149,3 +149,15 @@ def test_fused_steps_validation_without_gpu(lib):
     assert call([g0, g3], ws_bytes=nb.value) == 1005
     assert b"overlaps a momentum" in lib.msr_last_error()
 
+
+def test_muon_list_workspace_is_bounded(lib):
+    """The workspace of a list follows its largest shared launch, at most 2^27 elements of matrices padded
+    to multiples of 256 or one larger matrix: four matrices of that many elements (two iterates, A
+    and B' of a square one) and sums, whatever the number and shape of the matrices."""
+    from muon_sr_amd import _lib
+    size, one = ctypes.c_size_t(0), ctypes.c_size_t(0)
+    for rows, cols, count in ((16, 4096, 1000), (4096, 16, 1000), (1, 300, 5000), (64, 64, 10000), (2048, 2048, 100), (4096, 14336, 3)):
+        items = (_lib.MuonMatrix * count)(*[_lib.MuonMatrix(16, 16, 16, rows, cols, 1, 2, 0, 1.0)] * count)
+        assert lib.msr_muon_each_workspace_bytes(ctypes.addressof(items), count, ctypes.byref(size)) == 0
+        assert lib.msr_ns_workspace_bytes(1, rows, cols, ctypes.byref(one)) == 0
+        assert one.value <= size.value <= max(one.value * 2, 4 * 2 * (1 << 27) * 1.02), (rows, cols, size.value)
