@@ -47,7 +47,7 @@ struct A16Item {
     uint32_t seed, flags;
     float step;          // lr / bc                  | lr sqrt(BC2) / BC1
     float den, rden;     // sqrt(bias corr.) 2^32, RN of its reciprocal | sqrt(BC2) eps, unused
-    uint32_t mmin;       // bits of the smallest nonzero |m'| of the fast branch, minus 1 (see mom_ok)
+    uint32_t mmin;       // bits of the smallest nonzero |m'| of the fast branch, minus 1 (`ok` in a16_group)
 };
 
 struct A16Args {

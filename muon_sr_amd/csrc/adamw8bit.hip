@@ -692,6 +692,8 @@ __global__ __launch_bounds__(THREADS) void quant_table_check_kernel(const QuantT
 //   kind 3: rne_bf16x2 (hardware conversion) vs rne_bf16 (any u; both halves)
 //   kind 4: div_upd(n, d) vs n/d              (d in [2^-60, 2^32), 16 n per d: +-0 and
 //           15 hashed n with |n| in [2^-90, 2^60], spread over the quotient's range)
+//   kind 5: div_rn(m, d, 1/d) vs m/d          (d in [2^16, 2^32], 16 m per d: 0 and 15 hashed m in
+//           [2^-43, 2^44]: the scaled denominators of adamw16.hip, whose 1/d is the host's)
 __device__ __forceinline__ uint32_t mix32(uint32_t x) {
     x ^= x >> 16; x *= 0x7feb352du; x ^= x >> 15; x *= 0x846ca68bu; x ^= x >> 16;
     return x;
@@ -710,6 +712,14 @@ __global__ __launch_bounds__(THREADS) void fastmath_check_kernel(int kind, uint3
             bad += __float_as_uint(__builtin_fmaf(sqrt_rn_x2p32(x), 0x1p-32f, e)) != __float_as_uint(r + e);
         } else if (kind == 1) {
             bad += __float_as_uint(rcp_rn(x)) != __float_as_uint(1.0f / x);
+        } else if (kind == 5) {
+            const float y = 1.0f / x;
+            for (uint32_t k = 0; k < 16; ++k) {
+                const uint32_t h = mix32(u * 16u + k);
+                const float f = 1.0f + (float)(mix32(h) >> 8) * 0x1p-24f;   // t in [-43, 43]; 2^44 itself for u = k = 15 mod 16
+                const float m = k == 0 ? 0.0f : k == 15 && (u & 15u) == 15u ? 0x1p44f : ldexpf(f, (int)(h % 87u) - 43);
+                bad += __float_as_uint(div_rn(m, x, y)) != __float_as_uint(m / x);
+            }
         } else if (kind == 3) {
             const float x2 = __uint_as_float(~u);
             bad += rne_bf16x2(x, x2) != pack2(rne_bf16(x), rne_bf16(x2));
@@ -1179,9 +1189,11 @@ int msr_fastmath_check(int32_t kind, uint32_t bits_lo, uint32_t bits_hi, uint32_
                        msr_stream_t stream) {
     const uint32_t SQRT_HI = 0x5e800000u, RCP_LO = 0x21800000u, RCP_HI = 0x3fffffffu;   // 2^62, 2^-60, 2 - ulp
     const uint32_t UPD_HI = 0x4f7fffffu;                                                 // 2^32 - ulp
+    const uint32_t DEN_LO = 0x47800000u, DEN_HI = 0x4f800000u;                           // 2^16, 2^32
     const bool range_ok = kind == 0 ? bits_hi <= SQRT_HI
                         : kind == 3 ? true
                         : kind == 2 ? bits_lo >= RCP_LO && bits_hi <= RCP_HI
+                        : kind == 5 ? bits_lo >= DEN_LO && bits_hi <= DEN_HI
                                     : (kind == 1 || kind == 4) && bits_lo >= RCP_LO && bits_hi <= UPD_HI;
     if (!counts || n_counts <= 0 || bits_hi < bits_lo || !range_ok) {
         set_error("msr_fastmath_check: bad arguments (kind %d, range %08x..%08x)", (int)kind, bits_lo, bits_hi);

@@ -382,6 +382,10 @@ __device__ __forceinline__ float rcp_rn(float d) {
 // |m| in [2^-100, d].  For smaller |m| the quotient keeps m's sign and is +0
 // for m = +-0, which is all the codes need there: with d >= 2^-60 such an
 // |x| = |m/d| is below 2^-23, where every x of one sign codes alike.
+// Scaling d and m by powers of two scales every step exactly while d, y, q0 and r stay normal, and
+// nothing in the argument needs |m| <= d: it also holds for d in [2^16, 2^32] and m = +0 or in
+// [2^-43, 2^44] (q0 in [2^-75, 2^28], r a multiple of 2^-90), which adamw16.hip uses.
+// msr_fastmath_check tests both (kinds 2 and 5).
 __device__ __forceinline__ float div_rn(float m, float d, float y) {
     const float q0 = m * y;
     const float r = __builtin_fmaf(-q0, d, m);

@@ -137,3 +137,16 @@ def test_centralized_equals_centralize_then_step(L, mode, strength):
             assert torch.equal(d[k].view(torch.int16), w[k].view(torch.int16)), (it.n // it.cols, it.cols, "pgmv"[k])
     bad = (_lib.AdamWItem * 1)(_lib.AdamWItem(*[x.data_ptr() for x in dev[0]], 8, 0.1, 0.03, 1, 4104))
     assert L.msr_adamw_multi(ctypes.addressof(bad), 1, 2, strength, *hyper[:5], mode, stream()) == 1001
+
+
+@pytest.mark.parametrize("octave", range(16, 33))
+def test_scaled_quotient_is_correctly_rounded(L, octave):
+    """sqrt(v') / sqrt(bias correction) as the fast branch forms it, both scaled by 2^32: every
+    denominator of [2^16, 2^32], 16 numerators each over 0 and [2^-43, 2^44], against IEEE division."""
+    lo = (127 + octave) << 23
+    hi = lo + ((1 << 23) - 1 if octave < 32 else 0)
+    counts = torch.zeros(1024, dtype=torch.int32, device="cuda:0")
+    check(L, L.msr_fastmath_check(5, lo, hi, counts.data_ptr(), 1024, stream()), "fastmath check")
+    assert int(counts.sum().item()) == 0
+    assert L.msr_fastmath_check(5, 0x47800000 - 1, 0x47800000, counts.data_ptr(), 1024, stream()) == 1001
+    assert L.msr_fastmath_check(5, 0x4F800000, 0x4F800001, counts.data_ptr(), 1024, stream()) == 1001
