@@ -425,6 +425,20 @@ int msr_quant_table_check(const void *qtable, const float *qmap_signed, const fl
 int msr_fastmath_check(int32_t kind, uint32_t bits_lo, uint32_t bits_hi, uint32_t *counts, int32_t n_counts,
                        msr_stream_t stream);
 
+/* One product of the small-tile kernels in a given tile (64 or 128 wide) and ring (2 or 4 LDS stages),
+ * which the library otherwise picks by size; row-major contiguous operands, m and n multiples of the tile, k of
+ * 64, every extent at most 16384.
+ *   product 0  d = alpha p p^T                          p [batch][m][k]; resid out
+ *   product 1  d = alpha p p + beta p + diag I, the diagonal corrected for rvec (p symmetric, m = n = k;
+ *              d_ii += rvec_i (beta + 2 alpha p_ii)); resid out
+ *   product 2  d = alpha (p q + bf16(rvec) q)           p [batch][m][m], q [batch][m][n], rvec [batch][m]
+ *   product 3  d <- SR(d + bf16(p^T q)), noise of seed  p [k][m], q [k][n]; batch 1
+ * resid [batch][m]: fp32 rounding residuals of d's diagonal.  Test support: no counterpart in
+ * the reference. */
+int msr_tile_gemm(int32_t product, int32_t tile, int32_t stages, const uint16_t *p, const uint16_t *q, uint16_t *d,
+                  int64_t batch, int64_t m, int64_t n, int64_t k, float alpha, float beta, float diag,
+                  const float *rvec, float *resid, uint32_t seed, int32_t noise_mode, msr_stream_t stream);
+
 /* Batched bf16 GEMM  D[b] = alpha * P[b] Q[b]^T + beta * C[b] + diag * I  (fp32 accumulate, RNE
  * bf16 out; the diag term is added where m == n).
  * P: [M][K] (row stride ldp), Q: [N][K] (ldq), C/D: [M][N] (ldc/ldd); C may be NULL when beta == 0.

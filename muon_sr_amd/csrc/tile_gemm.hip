@@ -522,16 +522,17 @@ static int launch_tiles(int prod, int out, int mode, TileArgs &a, int64_t batch,
 // Estimated time (us) of a product in `tiles` tiles of T (ring of S stages) over `slabs` K slabs:
 // rounds of the work-groups that run at once (LDS and registers allow 512 of 64/4, 768 of 64/2, 256
 // of 128/4 and 512 of 128/2), each the slabs plus a tile's start and end.  Fitted to kernel times
-// of A, B' and X' at 20 Newton-Schulz shapes (1-64 matrices of 256-2048 x 256-5632); the estimates
-// pick the fastest of the four, or one within 5 % of it, on nearly all.  Some of the times, us
-// (64/4, 64/2, 128/4, 128/2):
-//   40 tiles of 64 (12 of 128),  4 slabs   4.1   4.4   6.9   6.6
-//   168 (48),                   24 slabs   6.8   8.8  13.4  13.7
-//   528 (136),                  88 slabs  59.3  44.8  38.2  57.3
-//   576 (144),                  12 slabs  12.0   9.9  10.5  10.5
-//   1024 (256),                 32 slabs  30.9  30.6  20.6  24.3
-//   1152 (288),                  6 slabs  12.0  11.0  14.0   9.8
-//   8192 (2048),                16 slabs   121   105    90    72
+// of A, B' and X' at 20 Newton-Schulz shapes (1-64 matrices of 256-2048 x 256-5632).  Some of the
+// times, us (64/4, 64/2, 128/4, 128/2), and what the estimates pick:
+//   40 tiles of 64 (12 of 128),  4 slabs   4.1   4.4   6.9   6.6   64/4, the fastest
+//   168 (48),                   24 slabs   6.8   8.8  13.4  13.7   64/4, the fastest
+//   528 (136),                  88 slabs  59.3  44.8  38.2  57.3   64/2, 17 % over 128/4
+//   576 (144),                  12 slabs  12.0   9.9  10.5  10.5   64/2, the fastest
+//   1024 (256),                 32 slabs  30.9  30.6  20.6  24.3   128/4, the fastest
+//   1152 (288),                  6 slabs  12.0  11.0  14.0   9.8   64/2, 12 % over 128/2
+//   8192 (2048),                16 slabs   121   105    90    72   128/2, the fastest
+// The two misses are 64/2, whose term is one line in `slabs` and a plain share of a round: 0.6 us
+// more for it mends the second and makes 40 other shapes 1.1 % slower (geometric mean).
 // 256-wide tiles (ns_gemm.hip): one work-group per CU.
 static double tile_cost(int T, int S, int64_t tiles, int64_t slabs) {
     const double f = (double)tiles / TILE_CUS, k = (double)slabs;
@@ -623,3 +624,40 @@ bool wgrad_takes_tiles(int64_t M, int64_t N, int64_t K) {
 }
 
 }  // namespace msr
+
+using namespace msr;
+
+extern "C" int msr_tile_gemm(int32_t product, int32_t tile, int32_t stages, const uint16_t *p, const uint16_t *q,
+                             uint16_t *d, int64_t batch, int64_t m, int64_t n, int64_t k, float alpha, float beta,
+                             float diag, const float *rvec, float *resid, uint32_t seed, int32_t noise_mode,
+                             msr_stream_t stream) {
+    const bool sym = product == TILE_A || product == TILE_B;
+    const int64_t lim = 1 << 14;   // operands below 2 GiB
+    if (product < TILE_A || product > TILE_W || !p || !d || (!sym && !q) || batch < 1 || batch > 1024 || m < 1 || m > lim ||
+        n < 1 || n > lim || k < 1 || k > lim || (sym && m != n) || ((product == TILE_B || product == TILE_X) && (k != m || !rvec)) ||
+        (sym && !resid) || (product == TILE_W && batch != 1) || (noise_mode != NOISE_TRITON && noise_mode != NOISE_PHILOX8)) {
+        set_error("msr_tile_gemm: bad arguments");
+        return MSR_ERR_ARG;
+    }
+    if (!aligned(p, 16) || !aligned(q, 16) || !aligned(d, 16)) { set_error("msr_tile_gemm: operands must be 16-byte aligned"); return MSR_ERR_ALIGN; }
+    const size_t np = 2 * (size_t)batch * m * k, nq = sym ? 0 : 2 * (size_t)batch * k * n, nd = 2 * (size_t)batch * m * n;
+    auto touch = [&](const void *x, size_t nx) { return x && (uintptr_t)x < (uintptr_t)d + nd && (uintptr_t)d < (uintptr_t)x + nx; };
+    if (touch(p, np) || touch(q, nq)) { set_error("msr_tile_gemm: d overlaps an operand"); return MSR_ERR_OVERLAP; }
+    TileArgs a = {};
+    const bool w = product == TILE_W;
+    a.P = p; a.ldp = w ? m : k; a.sP = m * k;
+    a.Q = sym ? p : q; a.ldq = sym ? k : n; a.sQ = sym ? m * k : k * n;
+    a.C = product == TILE_B ? p : nullptr; a.ldc = k; a.sC = m * k;
+    a.D = d; a.ldd = n; a.sD = m * n;
+    a.M = (int)m; a.N = (int)n; a.K = (int)k;
+    a.alpha = alpha; a.beta = beta; a.diag = diag;
+    a.rvec = rvec; a.resid = resid; a.sv = m;
+    a.ns.key = seed_key(seed, 0);
+    const hipStream_t s = (hipStream_t)stream;
+    if (tile == 64 && stages == 4) return launch_tiles<64, 4>(product, TILE_WS, noise_mode, a, batch, nullptr, s);
+    if (tile == 64 && stages == 2) return launch_tiles<64, 2>(product, TILE_WS, noise_mode, a, batch, nullptr, s);
+    if (tile == 128 && stages == 4) return launch_tiles<128, 4>(product, TILE_WS, noise_mode, a, batch, nullptr, s);
+    if (tile == 128 && stages == 2) return launch_tiles<128, 2>(product, TILE_WS, noise_mode, a, batch, nullptr, s);
+    set_error("msr_tile_gemm: no kernel of tile %d with %d stages", (int)tile, (int)stages);
+    return MSR_ERR_ARG;
+}
