@@ -34,8 +34,9 @@ struct NoTab {};
 // the weight gradient's SR accumulation.  OUT (X'): workspace matrix, caller's output as is
 // or transposed (bounded stores), or the Muon apply on the parameters in either layout.
 // MODE: noise mode of the apply or accumulation.  T: tile; S: LDS stages.
+// Two work-groups per CU, but for the 128 KiB ring, of which the LDS holds one.
 template <int T, int S, int PROD, int OUT, int MODE, typename TAB>
-__global__ __launch_bounds__(TG_THREADS, 2) void tile_gemm_kernel(TileArgs a, TAB tab) {
+__global__ __launch_bounds__(TG_THREADS, T * S == 512 ? 1 : 2) void tile_gemm_kernel(TileArgs a, TAB tab) {
     constexpr int W = T / 2, F = W / 32;            // a wave's sub-tile and its 32-wide blocks per side
     constexpr int SLAB = T * TBK * 2;               // bytes of one operand's slab
     constexpr int NL = SLAB / 4096;                 // direct-to-LDS loads per wave, operand and slab
