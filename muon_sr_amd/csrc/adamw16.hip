@@ -13,7 +13,8 @@
 //    extreme moments, a denominator that could leave the range).
 // Both give the same bits where both apply.  Measured on 128256 x 4096 (525 M elements, 7.35 GB):
 // 1735 us with IEEE square root and divisions throughout, 1260 us now (5.84 TB/s; a copy kernel
-// reaches 6.27).  The 73 tensors of an 8-layer d = 384 model: 502 us as 73 launches, 134 us as two.
+// reaches 6.27).  The 73 tensors of an 8-layer d = 384 model: 536 us as 73 launches, 100 us as two
+// (host time; the kernels take 52).
 #include <cmath>
 #include <algorithm>
 #include <vector>
